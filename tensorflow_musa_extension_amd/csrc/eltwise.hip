@@ -18,6 +18,7 @@
 // shapes such as [8191, 4095]).  Broadcast operands are tiny and stay in
 // L1/L2, so HBM traffic is the compulsory stream of the full-size tensors.
 #include <atomic>
+#include <type_traits>
 
 #include "device_util.h"
 #include "tfma_internal.h"
@@ -358,7 +359,189 @@ __global__ __launch_bounds__(kThreads) void ew_flat_kernel(
   }
 }
 
-// General broadcast: per element coordinate decomposition (64-bit).
+// General broadcast over the rows of the innermost (merged) dimension.
+// Neighbouring dimensions that every operand walks alike are merged first
+// (merge_dims), so an attention mask [N,1,1,S] over [N,H,S,S] is three
+// dimensions and a channel gate [N,1,1,C] over [N,H,W,C] too.  Along the
+// innermost dimension an operand then either runs with the output (a vector
+// per access) or has one value per row (splat).
+struct RowsOperand {
+  const void* p;
+  uint32_t stride[TFMA_MAX_DIMS - 1];  // elements per step of outer dimension d
+};
+struct RowsShape {
+  uint32_t w;       // innermost extent
+  uint32_t chunks;  // total chunks: rows * ceil(w / V)
+  int outer;        // outer dimensions; outer[outer - 1] varies fastest
+  int whole;        // every chunk may be stored whole (see the kernel)
+  FastDiv per_row;  // chunks of a row
+  FastDiv dim[TFMA_MAX_DIMS - 1];
+  // Two outer dimensions: one thread's step of `gridDim.x * kThreads` chunks
+  // as (dim 0, dim 1, chunk of the row).
+  uint32_t step0, step1, step_pos;
+};
+
+// Elements at p, which need only S's own alignment (rows of an odd extent
+// start anywhere): one 16-byte access, which global memory allows at any
+// address.
+template <int kAlign> struct AnyWord;
+template <> struct AnyWord<1> { typedef nt_u32x4 __attribute__((aligned(1))) T; };
+template <> struct AnyWord<2> { typedef nt_u32x4 __attribute__((aligned(2))) T; };
+template <> struct AnyWord<4> { typedef nt_u32x4 __attribute__((aligned(4))) T; };
+template <> struct AnyWord<8> { typedef nt_u32x4 __attribute__((aligned(8))) T; };
+template <typename S, int V>
+__device__ inline void vload_any(const S* p, S (&out)[V]) {
+  if constexpr (V == 1) {
+    out[0] = *p;
+  } else {
+    static_assert(V * sizeof(S) == 16, "one 16-byte access");
+    const nt_u32x4 w = *reinterpret_cast<const typename AnyWord<sizeof(S)>::T*>(p);
+    __builtin_memcpy(out, &w, 16);
+  }
+}
+template <typename S, int V>
+__device__ inline void vstore_any(S* p, const S (&in)[V]) {
+  if constexpr (V == 1) {
+    *p = in[0];
+  } else {
+    nt_u32x4 w;
+    __builtin_memcpy(&w, in, 16);
+    *reinterpret_cast<typename AnyWord<sizeof(S)>::T*>(p) = w;
+  }
+}
+
+// Where one thread's next chunk is, for at most two outer dimensions (one:
+// dim[0] is 1): the chunk's position as digits that advance by a constant
+// step with carries, and each operand's offset of the row with them.  All
+// additions and selects: a multiply-high division per chunk and dimension
+// kept the vector units busy for half of the kernel's time.
+struct RowsWalk {
+  uint32_t pos, c1, row_out;  // chunk of the row, index in dim 1, row * w
+  uint32_t ro[3];             // offset of each operand's row
+
+  __device__ RowsWalk(const RowsShape& sh, const RowsOperand* (&op)[3], uint32_t k) {
+    uint32_t row, c0;
+    sh.per_row.divmod(k, row, pos);
+    sh.dim[1].divmod(row, c0, c1);
+    row_out = row * sh.w;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) ro[i] = c0 * op[i]->stride[0] + c1 * op[i]->stride[1];
+  }
+  __device__ void step(const RowsShape& sh, const RowsOperand* (&op)[3]) {
+    const uint32_t per_row = sh.per_row.d, dim1 = sh.dim[1].d;
+    pos += sh.step_pos;
+    const bool carry = pos >= per_row;
+    pos -= carry ? per_row : 0;
+    c1 += sh.step1 + (carry ? 1u : 0u);  // at most 2 * dim1 - 1
+    const bool carry1 = c1 >= dim1;
+    c1 -= carry1 ? dim1 : 0;
+    row_out += (sh.step0 * dim1 + sh.step1) * sh.w + (carry ? sh.w : 0);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const uint32_t s0 = op[i]->stride[0], s1 = op[i]->stride[1];
+      ro[i] += sh.step0 * s0 + sh.step1 * s1 + (carry ? s1 : 0) + (carry1 ? s0 - dim1 * s1 : 0);
+    }
+  }
+};
+
+// A chunk is V elements of a row; a row's last chunk ends at the row's end,
+// so where w is no multiple of V it overlaps the one before and its loads
+// need no branch.  Both compute the same values for the elements they share,
+// and both store them (`whole`) unless the output lies over an operand: then
+// the last chunk might read what the other has just written, and stores only
+// its own elements.  Rows shorter than V run with V = 1.
+//
+// Bound by HBM: [16,16,384,384] bf16 + [16,1,1,384] 29.5 us (5.1 TB/s),
+// [64,28,28,512] f16 gate 21.3 us (4.8 TB/s).  An element-wise walk with a
+// 64-bit division per dimension and two bytes per access took 348 and 260 us.
+// U chunks of every operand are loaded before the first is used.  Odd rows
+// start between vectors: their accesses are not aligned, which costs a
+// quarter ([64,35,35,333] f16 gate 3.6 TB/s) and no element loop.
+template <class Tr, EwOp OP, int V, bool kVecA, bool kVecB, bool kVecC, bool kWalk>
+__global__ __launch_bounds__(kThreads) void ew_rows_kernel(RowsOperand a, RowsOperand b,
+                                                           RowsOperand c, RowsShape sh,
+                                                           typename Tr::S* out) {
+  using S = typename Tr::S;
+  constexpr int kArity = arity<OP>();
+  constexpr int U = 4;
+  const S* const pa = static_cast<const S*>(a.p);
+  const S* const pb = static_cast<const S*>(b.p);
+  const S* const pc = static_cast<const S*>(c.p);
+  const RowsOperand* op[3] = {&a, &b, &c};
+  const uint32_t stride = gridDim.x * kThreads;
+  const uint32_t first = blockIdx.x * kThreads + threadIdx.x;
+  [[maybe_unused]] RowsWalk at(sh, op, first);
+  for (uint32_t k0 = first; k0 < sh.chunks; k0 += U * stride) {
+    uint32_t oo[U], oa[U], ob[U], oc[U], keep[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      // Chunks past the end load from the operands' starts and store
+      // nothing.
+      const uint32_t k = k0 + u * stride;
+      const bool in = k < sh.chunks && k >= k0;
+      uint32_t pos, ro[3];
+      if constexpr (kWalk) {
+        pos = at.pos;
+        oo[u] = at.row_out;
+        for (int i = 0; i < 3; ++i) ro[i] = at.ro[i];
+        at.step(sh, op);
+      } else {
+        uint32_t row;
+        sh.per_row.divmod(k, row, pos);
+        oo[u] = row * sh.w;
+        for (int i = 0; i < 3; ++i) ro[i] = 0;
+        for (int d = sh.outer - 1; d >= 0; --d) {
+          uint32_t q = 0, r = row;
+          if (d > 0) sh.dim[d].divmod(row, q, r);
+          row = q;
+          for (int i = 0; i < kArity; ++i) ro[i] += r * op[i]->stride[d];
+        }
+      }
+      const uint32_t e0 = pos * V;
+      const uint32_t e = e0 + V <= sh.w ? e0 : sh.w - V;
+      keep[u] = in ? V - (e0 - e) : 0;  // the chunk's last keep elements are its own
+      oo[u] += e;
+      oa[u] = in ? ro[0] + (kVecA ? e : 0) : 0;
+      ob[u] = in ? ro[1] + (kVecB ? e : 0) : 0;
+      oc[u] = in ? ro[2] + (kVecC ? e : 0) : 0;
+    }
+    S av[U][V], bv[U][V], cv[U][V];
+    auto fetch_any = [](const S* p, uint32_t o, S (&v)[V], auto vec) {
+      if constexpr (decltype(vec)::value) {
+        vload_any<S, V>(p + o, v);
+      } else {
+        const S s = p[o];
+#pragma unroll
+        for (int j = 0; j < V; ++j) v[j] = s;
+      }
+    };
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      fetch_any(pa, oa[u], av[u], std::integral_constant<bool, kVecA>{});
+      if constexpr (kArity >= 2)
+        fetch_any(pb, ob[u], bv[u], std::integral_constant<bool, kVecB>{});
+      if constexpr (kArity >= 3)
+        fetch_any(pc, oc[u], cv[u], std::integral_constant<bool, kVecC>{});
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      S ov[V];
+#pragma unroll
+      for (int j = 0; j < V; ++j)
+        ov[j] = ew_apply<Tr, OP>(av[u][j], kArity >= 2 ? bv[u][j] : S(0),
+                                 kArity >= 3 ? cv[u][j] : S(0));
+      if (keep[u] == V || (keep[u] > 0 && sh.whole)) {
+        vstore_any<S, V>(out + oo[u], ov);
+      } else if (keep[u] > 0) {
+#pragma unroll
+        for (int j = 1; j < V; ++j)
+          if (j >= V - static_cast<int>(keep[u])) out[oo[u] + j] = ov[j];
+      }
+    }
+  }
+}
+
+// More than 2^31 elements: per element coordinate decomposition (64-bit).
 template <class Tr, EwOp OP>
 __global__ __launch_bounds__(kThreads) void ew_strided_kernel(
     const typename Tr::S* __restrict__ a, const typename Tr::S* __restrict__ b,
@@ -618,15 +801,154 @@ hipError_t launch_ew(int64_t n, const BcastOperand& a, const BcastOperand& b,
   return hipGetLastError();
 }
 
+// Drops dimensions of extent 1 and merges an outer dimension into its inner
+// neighbour where every operand (and the contiguous output) walks the two as
+// one: no step (0) in both, or the outer step equal to the inner extent times
+// the inner step.
+void merge_dims(const StridedShape& sh, StridedShape* out) {
+  StridedShape m{};
+  auto get = [](StridedShape& x, int i) -> int64_t* {
+    return i == 0 ? x.stride_a : (i == 1 ? x.stride_b : x.stride_c);
+  };
+  StridedShape in = sh;
+  // Innermost first, reversed at the end.
+  for (int d = sh.ndims - 1; d >= 0; --d) {
+    if (sh.dims[d] == 1) continue;
+    bool joins = m.ndims > 0;
+    for (int i = 0; i < 3 && joins; ++i)
+      joins = get(in, i)[d] == get(m, i)[m.ndims - 1] * m.dims[m.ndims - 1];
+    if (joins) {
+      m.dims[m.ndims - 1] *= sh.dims[d];
+    } else {
+      m.dims[m.ndims] = sh.dims[d];
+      for (int i = 0; i < 3; ++i) get(m, i)[m.ndims] = get(in, i)[d];
+      ++m.ndims;
+    }
+  }
+  *out = StridedShape{};
+  out->ndims = m.ndims;
+  for (int d = 0; d < m.ndims; ++d) {
+    const int r = m.ndims - 1 - d;
+    out->dims[d] = m.dims[r];
+    out->stride_a[d] = m.stride_a[r];
+    out->stride_b[d] = m.stride_b[r];
+    out->stride_c[d] = m.stride_c[r];
+  }
+}
+
+// [p, p + elems * esize) and [q, q + n * esize) share bytes.
+bool overlaps(const void* p, int64_t elems, const void* q, int64_t n, int esize) {
+  const uintptr_t a = reinterpret_cast<uintptr_t>(p), b = reinterpret_cast<uintptr_t>(q);
+  return a < b + static_cast<uintptr_t>(n) * esize && b < a + static_cast<uintptr_t>(elems) * esize;
+}
+
+template <class Tr, EwOp OP, int V, bool kVecA, bool kVecB, bool kVecC>
+void launch_rows(const RowsOperand& a, const RowsOperand& b, const RowsOperand& c,
+                 RowsShape sh, typename Tr::S* out, hipStream_t stream) {
+  // 2-byte types: 3 workgroups per CU, whose extra chunks in flight cover the
+  // unpacking and rounding ([16,16,384,384] bf16 mask 31.7 us with 2, 29.5
+  // with 3, 30.9 with 4; [64,28,28,512] f16 gate 22.6 / 21.3 / 22.1); others
+  // 2 ([64,12,384,384] f32 mask 159 / 167 / 185).
+  int64_t blocks = grid_for(sh.chunks, 4);
+  const int64_t cap = static_cast<int64_t>(DeviceCUs()) * 3;
+  if (sizeof(typename Tr::S) == 2 && blocks_per_cu() == 2) {
+    blocks = (static_cast<int64_t>(sh.chunks) + kThreads * 4 - 1) / (kThreads * 4);
+    if (blocks > cap) blocks = cap;
+  }
+  // Up to two outer dimensions advance as digits (RowsWalk): [64,28,28,512]
+  // f16 gate 23.6 -> 21.3 us, [16,12,197,197] f16 mask 9.2 -> 7.8 us.
+  if (sh.outer <= 2) {
+    const uint32_t step = static_cast<uint32_t>(blocks) * kThreads;
+    const uint32_t rows = step / sh.per_row.d;
+    sh.step_pos = step % sh.per_row.d;
+    sh.step1 = rows % sh.dim[1].d;
+    sh.step0 = rows / sh.dim[1].d;
+    TFMA_LAUNCH(op_kernel_name(OP), (ew_rows_kernel<Tr, OP, V, kVecA, kVecB, kVecC, true>),
+                dim3(blocks), dim3(kThreads), 0, stream, a, b, c, sh, out);
+  } else {
+    TFMA_LAUNCH(op_kernel_name(OP), (ew_rows_kernel<Tr, OP, V, kVecA, kVecB, kVecC, false>),
+                dim3(blocks), dim3(kThreads), 0, stream, a, b, c, sh, out);
+  }
+}
+
 template <class Tr, EwOp OP>
 hipError_t launch_ew_strided(int64_t n, const void* a, const void* b,
-                             const void* c, const StridedShape& sh, void* out,
+                             const void* c, const StridedShape& full, void* out,
                              hipStream_t stream) {
   using S = typename Tr::S;
-  TFMA_LAUNCH("tfma_ew_strided", (ew_strided_kernel<Tr, OP>), dim3(grid_for(n, 4)),
-                     dim3(kThreads), 0, stream, static_cast<const S*>(a),
-                     static_cast<const S*>(b), static_cast<const S*>(c), sh,
-                     static_cast<S*>(out), n);
+  if (n > 0x7fffffff) {
+    TFMA_LAUNCH("tfma_ew_strided", (ew_strided_kernel<Tr, OP>), dim3(grid_for(n, 4)),
+                dim3(kThreads), 0, stream, static_cast<const S*>(a),
+                static_cast<const S*>(b), static_cast<const S*>(c), full,
+                static_cast<S*>(out), n);
+    return hipGetLastError();
+  }
+  StridedShape m;
+  merge_dims(full, &m);
+  if (m.ndims == 0) {  // one element
+    m.ndims = 1;
+    m.dims[0] = 1;
+  }
+  const int in = m.ndims - 1;
+  RowsOperand oa{a, {}}, ob{b, {}}, oc{c, {}};
+  RowsShape sh{};
+  sh.w = static_cast<uint32_t>(m.dims[in]);
+  // Two outer dimensions at least (leading ones of extent 1).
+  const int lead = in < 2 ? 2 - in : 0;
+  sh.outer = in + lead;
+  int64_t ea = 1, eb = 1, ec = 1;  // elements of each operand
+  for (int d = 0; d < sh.outer; ++d) {
+    if (d < lead) {
+      sh.dim[d] = FastDiv(1);
+      continue;
+    }
+    sh.dim[d] = FastDiv(static_cast<uint32_t>(m.dims[d - lead]));
+    oa.stride[d] = static_cast<uint32_t>(m.stride_a[d - lead]);
+    ob.stride[d] = static_cast<uint32_t>(m.stride_b[d - lead]);
+    oc.stride[d] = static_cast<uint32_t>(m.stride_c[d - lead]);
+  }
+  for (int d = 0; d <= in; ++d) {
+    ea *= m.stride_a[d] != 0 ? m.dims[d] : 1;
+    eb *= m.stride_b[d] != 0 ? m.dims[d] : 1;
+    ec *= m.stride_c[d] != 0 ? m.dims[d] : 1;
+  }
+  constexpr int kEs = sizeof(S);
+  sh.whole = !overlaps(a, ea, out, n, kEs) && (arity<OP>() < 2 || !overlaps(b, eb, out, n, kEs)) &&
+             (arity<OP>() < 3 || !overlaps(c, ec, out, n, kEs));
+  // An operand contiguous in its own order steps by 1 along the innermost
+  // output dimension, or not at all.
+  const bool one = sh.w == 1;
+  const bool va = one || m.stride_a[in] != 0, vb = one || m.stride_b[in] != 0,
+             vc = one || m.stride_c[in] != 0;
+  const int64_t rows = n / sh.w;
+  const int V = static_cast<int64_t>(sh.w) >= Tr::kVec ? Tr::kVec : 1;
+  const int64_t per_row = (sh.w + V - 1) / V;
+  sh.per_row = FastDiv(static_cast<uint32_t>(per_row));
+  sh.chunks = static_cast<uint32_t>(rows * per_row);
+  S* const o = static_cast<S*>(out);
+  auto go = [&](auto v, auto fa, auto fb, auto fc) {
+    launch_rows<Tr, OP, decltype(v)::value, decltype(fa)::value, decltype(fb)::value,
+                decltype(fc)::value>(oa, ob, oc, sh, o, stream);
+  };
+  using Yes = std::integral_constant<bool, true>;
+  using No = std::integral_constant<bool, false>;
+  auto pick = [&](auto v) {
+    // Some operand runs with the output, or w would have merged away.
+    if constexpr (arity<OP>() < 2) {
+      go(v, Yes{}, Yes{}, Yes{});
+    } else if constexpr (arity<OP>() < 3) {
+      if (va) vb ? go(v, Yes{}, Yes{}, Yes{}) : go(v, Yes{}, No{}, Yes{});
+      else go(v, No{}, Yes{}, Yes{});
+    } else if (vc) {
+      if (va) vb ? go(v, Yes{}, Yes{}, Yes{}) : go(v, Yes{}, No{}, Yes{});
+      else vb ? go(v, No{}, Yes{}, Yes{}) : go(v, No{}, No{}, Yes{});
+    } else {
+      if (va) vb ? go(v, Yes{}, Yes{}, No{}) : go(v, Yes{}, No{}, No{});
+      else go(v, No{}, Yes{}, No{});
+    }
+  };
+  if (V == 1) pick(std::integral_constant<int, 1>{});
+  else pick(std::integral_constant<int, Tr::kVec>{});
   return hipGetLastError();
 }
 

@@ -317,3 +317,37 @@ def test_float64_binary_and_mul_add(dev, xs, ys, zs):
             ("MusaShiftedAffineMap", ops.MusaShiftedAffineMap(xd, yd, zd), y * x + z)):
         assert got.dtype == torch.float64
         assert_bitwise(got.cpu().numpy(), ref, name)
+
+
+# Broadcasts that no (inner, period) walk describes, by row: a row of less than
+# a vector, of one, of one and a remainder of one or of all but one element,
+# of many; one, two and three merged outer dimensions; either operand splat
+# along the row; chunks past a grid's stride.
+ROWS = [
+    ((4, 5, 3), (4, 1, 3)),
+    ((4, 5, 8), (4, 1, 8)),
+    ((6, 7, 9), (6, 1, 9)),
+    ((6, 7, 15), (6, 1, 15)),
+    ((3, 1, 17), (3, 5, 1)),
+    ((33, 1), (1, 29)),
+    ((3, 4, 5, 6, 31), (3, 1, 5, 1, 31)),
+    ((2, 1, 3, 1, 33), (1, 4, 1, 5, 33)),
+    ((64, 12, 97, 97), (64, 1, 1, 97)),
+    ((5, 9, 1031), (5, 1, 1031)),
+]
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("xs,ys", ROWS)
+def test_broadcast_rows(dev, dtype, xs, ys):
+    rng = np.random.default_rng(12)
+    x, y = gen(rng, xs, dtype), gen(rng, ys, dtype)
+    z = gen(rng, ys[-1:], dtype)
+    xd, yd, zd = (to_dev(t, dtype, dev) for t in (x, y, z))
+    want = oracle.eltwise("add_relu", [x, y], dtype)
+    assert_bitwise(to_np(ops.MusaAddV2Relu(xd, yd), dtype), want, "x + y")
+    assert_bitwise(to_np(ops.MusaAddV2Relu(yd, xd), dtype), want, "y + x")
+    assert_bitwise(to_np(ops.MusaShiftedAffineMap(xd, yd, zd), dtype),
+                   oracle.eltwise("mul_add", [x, y, z], dtype), "x * y + z")
+    if want.shape == x.shape:  # the output in place of an operand
+        assert_bitwise(to_np(ops.MusaAddV2Relu(xd, yd, out=xd), dtype), want, "in place")
