@@ -847,6 +847,10 @@ struct FusedArgs {
   unsigned long long* ekey;
   unsigned epoch;
   unsigned* epoch_dev;
+  // Folded launches: rows [tail_row, tail_row + tail) are no whole super-row;
+  // the waves that finish a channel sum and write them.
+  int tail;
+  int64_t tail_row;
   FinArgs fin;
 };
 
@@ -1175,7 +1179,9 @@ __device__ __forceinline__ void finish_channels(const FusedArgs& a, int cs0, int
 // 0 .. B-1 finish one channel each.  B = 16, or smaller where the groups
 // need more than kEpochPerLane words per lane.  Same give-up behaviour as
 // finish_channels.
-template <class Tr, bool kGrad>
+// kFold: the channel's elements in the tail rows are added to its sums here,
+// and written once its coefficients are known.
+template <class Tr, bool kGrad, bool kFold = false>
 __device__ __forceinline__ void finish_channel_blocks(const FusedArgs& a, int cs0, int cs1,
                                                       int wave, int lane, uint32_t wtag,
                                                       uint64_t etag, unsigned epoch) {
@@ -1239,8 +1245,25 @@ __device__ __forceinline__ void finish_channel_blocks(const FusedArgs& a, int cs
       t2 += __shfl_xor(t2, off, 64);
     }
     float4 cfc = make_float4(0.f, 0.f, 0.f, 0.f);
+    using S = typename Tr::S;
+    const S* const xt = static_cast<const S*>(a.x) + a.tail_row * a.c + ch;
+    const S* const dt = static_cast<const S*>(a.dy) + a.tail_row * a.c + ch;
+    if constexpr (kFold) {
+      const float kc = kGrad ? fin_in.mi : fin_in.k;
+      for (int r = 0; r < a.tail && lane < B && chv; ++r) {
+        const float xc = Tr::ld(xt[r * a.c]) - kc;
+        const float f = kGrad ? Tr::ld(dt[r * a.c]) : xc;
+        t1 += f;
+        t2 += f * xc;
+      }
+    }
     if (lane < B && chv) cfc = finish_channel<Tr, kGrad>(a.fin, ch, t1, t2, fin_in);
     store_coefs(a, ch, chv, cfc, lane, B, etag);
+    if constexpr (kFold) {
+      S* const ot = static_cast<S*>(a.out) + a.tail_row * a.c + ch;
+      for (int r = 0; r < a.tail && lane < B && chv; ++r)
+        ot[r * a.c] = apply_one<Tr, kGrad>(xt[r * a.c], kGrad ? dt[r * a.c] : S(0), cfc);
+    }
   }
 }
 
@@ -2019,6 +2042,365 @@ __global__ __launch_bounds__(kFusedThreads) void bn_sliced_grad_kernel(FusedArgs
   }
 }
 
+// Exit of a launch recorded into a graph: counted in two levels; the
+// workgroup completing the count zeroes the counters and advances the
+// replays' epoch word (as in bn_fused_nhwc_kernel, which documents the
+// orderings).  Every thread of the workgroup calls it.
+__device__ inline void recorded_exit(const FusedArgs& a, unsigned epoch) {
+  if (!a.reset_at_exit) return;
+  const int lane = threadIdx.x & 63;
+  __syncthreads();
+  if (threadIdx.x >= 64) return;
+  unsigned done = 0;
+  if (lane == 0) {
+    const unsigned r = blockIdx.x & 7;
+    unsigned last = a.sub_last[0];
+#pragma unroll
+    for (int i = 1; i < 8; ++i) last = r == static_cast<unsigned>(i) ? a.sub_last[i] : last;
+    const unsigned old =
+        __hip_atomic_fetch_add(a.sub + 64 * r, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (old == last) {
+      const unsigned long long gg =
+          __hip_atomic_fetch_add(a.barrier, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      done = gg == a.base + barrier_classes() - 1;
+    }
+  }
+  if (__builtin_amdgcn_readfirstlane(done)) {
+    if (lane < 8)
+      __hip_atomic_store(a.sub + 64 * lane, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (lane == 0) {
+      __hip_atomic_store(a.barrier, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (a.epoch_dev)
+        __hip_atomic_store(a.epoch_dev, (epoch - 0x80000001u + 1u) % 0x7fffffffu,
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// 4c. Folded kernel: NHWC with a channel count that is no multiple of the
+//     vector width.  F = VEC / gcd(C, VEC) rows are one super-row of C * F
+//     elements, a whole number of 16-byte vectors, in which every vector
+//     position has fixed channels (element e: channel e mod C); rows past the
+//     last whole super-row (fewer than F) are the finishing waves' (tail).
+//     A workgroup owns a range of super-rows and a tile of tw vector
+//     positions, thread (ty, tx) position tx of every ry-th row, ry =
+//     512 / tw: with any tw instead of a power of two at most a few lanes
+//     are idle.  One tile holds a super-row of up to 512 vectors and channels;
+//     its workgroups sum the F appearances of a channel before they publish
+//     it, and stream whole rows (in tiles of 64 vectors, whose ends share
+//     cache lines with the next tile's, [256,56,56,163] f16 took 163 / 252 us
+//     instead of 134 / 218).  Wider super-rows run in tiles of at most 512
+//     columns, and each appearance is a partial of its own: slot (g * F + f) * C + c, so the
+//     finals read them as G * F groups.  K (the shift; the grad's mean) and
+//     the coefficients are per channel and go through LDS.
+//     Bound as bn_fused_nhwc_kernel is: HBM for large tensors, the two
+//     cross-XCD hand-offs for small ones.  The split kernels it replaces
+//     read twice in 2-byte accesses, in three launches; forward / grad, back
+//     to back: f16 [64,35,35,99] 34.2 / 48.7 -> 15.7 / 17.6 us, [256,56,56,
+//     163] 352 / 672 -> 133 / 217 us, f32 [128,28,28,1021] 384 / 597 -> 195
+//     / 351 us, f16 [32,14,14,99] 11.0 / 13.2 -> 11.4 / 11.6 us.
+// ---------------------------------------------------------------------------
+constexpr int kFoldChannels = 512; // most channels (one tile) or columns of a tile
+constexpr int kFoldParts = 32;     // most threads that share one channel's sums
+
+// Register rows per thread (the largest spill-free counts), and of the
+// kernels for at most that many rows and the LDS rows (kFoldedSmall: less
+// code, run once).
+template <class Tr> struct FoldedRows { static constexpr int kFwd = 24, kGrad = 11; };
+template <> struct FoldedRows<TF32> { static constexpr int kFwd = 28, kGrad = 13; };
+template <> struct FoldedRows<TBF16> { static constexpr int kFwd = 24, kGrad = 9; };
+constexpr int kFoldedSmall = 6;
+
+struct FoldedArgs {
+  FusedArgs f;         // c: real channels; groups: partial words per channel
+  int fold;            // F
+  int cv;              // vectors of a super-row
+  int tw;              // vector positions of a tile
+  int tiles;
+  int ry;              // super-rows of one pass
+  int64_t rows;        // whole super-rows
+  int64_t rows_per_g;
+  FastDiv div_tw, div_ry, div_c;
+};
+
+template <class Tr, bool kGrad, int KR, int KL>
+__global__ __launch_bounds__(kFusedThreads) void bn_folded_nhwc_kernel(FoldedArgs fa) {
+  using S = typename Tr::S;
+  constexpr int VEC = Tr::kVec;
+  constexpr int kIn = kGrad ? 2 : 1;
+  constexpr int U = kGrad ? 4 : 8;
+  // Local channel l at l + l / VEC, component by component (one pad word per
+  // vector: consecutive lanes' reads fall on distinct banks).
+  constexpr int kComp = kFoldChannels + kFoldChannels / VEC;
+  constexpr int kRed = kFusedThreads * VEC > 4 * kComp ? kFusedThreads * VEC : 4 * kComp;
+  extern __shared__ uint4 lds_rows[];  // [KL][kIn][kFusedThreads]
+  __shared__ __align__(16) float red[kRed];
+  const FusedArgs& a = fa.f;
+  const int tid = threadIdx.x;
+  const int wave = tid >> 6, lane = tid & 63;
+  const uint32_t C = static_cast<uint32_t>(a.c);
+  const bool single = fa.tiles == 1;
+  const int tile = static_cast<int>(blockIdx.x % static_cast<unsigned>(fa.tiles));
+  const int64_t g = blockIdx.x / static_cast<unsigned>(fa.tiles);
+  const int64_t r0 = g * fa.rows_per_g;
+  int64_t r1 = r0 + fa.rows_per_g;
+  if (r1 > fa.rows) r1 = fa.rows;
+  uint32_t ty, tx;
+  fa.div_tw.divmod(static_cast<uint32_t>(tid), ty, tx);
+  const int col = tile * fa.tw + static_cast<int>(tx);
+  // nk_t: rows of this thread's ty whatever its column (the wave's lane 0
+  // has the wave's smallest ty, so the most rows).
+  const uint32_t rows_g = static_cast<uint32_t>(r1 - r0);
+  const int nk_t = static_cast<int>(ty) < fa.ry && ty < rows_g
+                       ? static_cast<int>(fa.div_ry.div(rows_g - ty + fa.ry - 1))
+                       : 0;
+  const bool active = static_cast<int>(ty) < fa.ry && col < fa.cv;
+  const int nk = active ? nk_t : 0;
+  const int nk_w = __builtin_amdgcn_readfirstlane(nk_t);
+  const int kl_w = nk_w - KR < 0 ? 0 : (nk_w - KR < KL ? nk_w - KR : KL);
+  const uint32_t row_b = static_cast<uint32_t>(fa.cv) * 16u;
+  const int64_t first = r0 * row_b;  // byte offset of the group's rows
+  const auto rx = rows_rsrc(static_cast<const char*>(a.x) + first, (r1 - r0) * row_b);
+  const auto rd =
+      rows_rsrc(static_cast<const char*>(kGrad ? a.dy : a.x) + first, (r1 - r0) * row_b);
+  char* const obase = static_cast<char*>(a.out) + first;
+  const uint32_t lane_off = active ? ty * row_b + static_cast<uint32_t>(col) * 16u : kOutOfRange;
+  const uint32_t rstride_b = static_cast<uint32_t>(fa.ry) * row_b;
+  auto roff = [&](int q) { return lane_off + static_cast<uint32_t>(q) * rstride_b; };
+  auto lds = [&](int q2, int which) -> uint4& {
+    return lds_rows[(q2 * kIn + which) * kFusedThreads + tid];
+  };
+  // The tile's local channels: the channels themselves, or (several tiles)
+  // its columns.  Thread t < nl owns local channel t, channel ch_t.
+  const uint32_t col_e = static_cast<uint32_t>(tile * fa.tw) * VEC;  // first column's element
+  const uint32_t left = static_cast<uint32_t>(fa.cv) * VEC - col_e;
+  const uint32_t nl =
+      single ? C : (left < static_cast<uint32_t>(fa.tw) * VEC ? left : fa.tw * VEC);
+  const bool owner = static_cast<uint32_t>(tid) < nl;
+  const uint32_t ve = col_e + static_cast<uint32_t>(tid);
+  const uint32_t ch_t = owner ? ve - fa.div_c.div(ve) * C : 0;
+  // Local channel of this thread's element j.
+  const uint32_t e0 = active ? tx * VEC : 0;
+  const uint32_t l0 = single ? e0 - fa.div_c.div(e0) * C : e0;
+  auto local = [&](int j) {
+    uint32_t l = l0 + static_cast<uint32_t>(j);
+    if (single) {
+      while (l >= C) l -= C;  // C may be less than a vector
+    }
+    return l;
+  };
+
+  // ---- phase 1 ----------------------------------------------------------
+  float k_own = 0.f;
+  if constexpr (kGrad) {
+    if (owner) k_own = a.fin.mean_in[ch_t];
+  }
+  S ks[5];
+  if constexpr (!kGrad) {
+    int64_t js[5];
+    shift_rows(a.fin.n, js);
+#pragma unroll
+    for (int i = 0; i < 5; ++i) ks[i] = static_cast<const S*>(a.x)[js[i] * C + ch_t];
+  }
+  uint4 xr[KR];
+  uint4 dr[kGrad ? KR : 1];
+  uint4 xl[KL];
+  uint4 dl[kGrad ? KL : 1];
+#pragma unroll
+  for (int q = 0; q < KR; ++q) {
+    xr[q] = bld16_last(rx, roff(q));
+    if constexpr (kGrad) dr[q] = bld16_last(rd, roff(q));
+  }
+#pragma unroll
+  for (int q = 0; q < KL; ++q) {
+    xl[q] = bld16_last(rx, roff(KR + q));
+    if constexpr (kGrad) dl[q] = bld16_last(rd, roff(KR + q));
+  }
+  const unsigned epoch =
+      a.epoch_dev ? 0x80000001u + __hip_atomic_load(a.epoch_dev, __ATOMIC_RELAXED,
+                                                    __HIP_MEMORY_SCOPE_AGENT) % 0x7fffffffu
+                  : a.epoch;
+  const uint64_t etag = static_cast<uint64_t>(epoch) << 32;
+  const uint32_t wtag = epoch ^ a.wait_xor;
+  if constexpr (!kGrad) {
+    float v[5];
+#pragma unroll
+    for (int i = 0; i < 5; ++i) v[i] = Tr::ld(ks[i]);
+    k_own = shift_of(v);
+  }
+  if (owner) red[tid + tid / VEC] = k_own;
+  __syncthreads();
+  float k[VEC], s1[VEC], s2[VEC];
+#pragma unroll
+  for (int j = 0; j < VEC; ++j) {
+    const uint32_t l = local(j);
+    k[j] = red[l + l / VEC];
+    s1[j] = 0.f;
+    s2[j] = 0.f;
+  }
+#pragma unroll
+  for (int q = 0; q < KR; ++q) {
+    if (q < nk) accum_words<Tr, kGrad>(xr[q], dr[kGrad ? q : 0], k, s1, s2);
+    if constexpr (kGrad ? Resident<Tr>::kOpaqueGrad : Resident<Tr>::kOpaqueFwd) {
+      asm volatile("" : "+v"(xr[q].x), "+v"(xr[q].y), "+v"(xr[q].z), "+v"(xr[q].w));
+      if constexpr (kGrad)
+        asm volatile("" : "+v"(dr[q].x), "+v"(dr[q].y), "+v"(dr[q].z), "+v"(dr[q].w));
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < KL; ++q) {
+    if (q < kl_w) {
+      lds(q, 0) = xl[q];
+      if constexpr (kGrad) lds(q, kGrad ? 1 : 0) = dl[kGrad ? q : 0];
+    }
+  }
+#pragma unroll 2
+  for (int q = 0; q < kl_w; ++q) {
+    if (KR + q < nk) {
+      const uint4 xw = lds(q, 0);
+      const uint4 dw = kGrad ? lds(q, kGrad ? 1 : 0) : xw;
+      accum_words<Tr, kGrad>(xw, dw, k, s1, s2);
+    }
+  }
+  // Streamed rows (rows past nk are out of range and not summed).
+  for (int q = KR + KL; q < nk; q += U) {
+    uint4 xw[U], dw[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      xw[u] = bld16(rx, roff(q + u));
+      if constexpr (kGrad) dw[u] = bld16(rd, roff(q + u));
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (q + u < nk) accum_words<Tr, kGrad>(xw[u], dw[u], k, s1, s2);
+  }
+  // The workgroup's sums per local channel: the threads' sums as a matrix
+  // of nl columns - one tile: entry i of the ry passes' columns is channel
+  // i mod C, ry * F rows; several: a row per pass - whose rows are dealt to
+  // `parts` threads a column, then those added in order.
+  const uint32_t nrows = single ? static_cast<uint32_t>(fa.ry * fa.fold) : fa.ry;
+  const uint32_t pitch = single ? C : static_cast<uint32_t>(fa.tw) * VEC;
+  uint32_t parts = kFusedThreads / nl;
+  parts = parts < 1 ? 1 : (parts > kFoldParts ? kFoldParts : parts);
+  uint32_t part = 0, pl = static_cast<uint32_t>(tid);
+  while (pl >= nl && part < parts) {
+    pl -= nl;
+    ++part;
+  }
+  float sum[2];
+#pragma unroll
+  for (int w = 0; w < 2; ++w) {
+    __syncthreads();
+    if (static_cast<int>(ty) < fa.ry) {
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) red[tid * VEC + j] = w == 0 ? s1[j] : s2[j];
+    }
+    __syncthreads();
+    float t = 0.f;
+    if (part < parts)
+      for (uint32_t r = part; r < nrows; r += parts) t += red[r * pitch + pl];
+    sum[w] = t;
+  }
+  if (parts > 1) {
+    __syncthreads();
+    if (part < parts) {
+      red[2 * tid] = sum[0];
+      red[2 * tid + 1] = sum[1];
+    }
+    __syncthreads();
+    if (owner) {
+      for (uint32_t p = 1; p < parts; ++p) {
+        sum[0] += red[2 * (p * nl + tid)];
+        sum[1] += red[2 * (p * nl + tid) + 1];
+      }
+    }
+  }
+  if (owner) {
+    if constexpr (!kGrad) {
+      if (g == 0 && ve < C) store_shared(a.ekey + ve, etag | __builtin_bit_cast(uint32_t, k_own));
+    }
+    const int64_t slot = single ? g * C + tid : g * fa.fold * C + ve;
+    store_pair(slots_rsrc(a.eslots, a.groups, a.c), slot, static_cast<uint32_t>(etag >> 32),
+               sum[0], sum[1]);
+  }
+
+  // ---- phase 2 ----------------------------------------------------------
+  finish_channel_blocks<Tr, kGrad, true>(a, 0, a.c, wave, lane, wtag, etag, epoch);
+  zero_side_outputs<kGrad>(a.fin);
+
+  // ---- phase 3 ----------------------------------------------------------
+#pragma unroll
+  for (int r = 0; r < KR; ++r) {
+    asm volatile("" : "+v"(xr[r].x), "+v"(xr[r].y), "+v"(xr[r].z), "+v"(xr[r].w));
+    if constexpr (kGrad)
+      asm volatile("" : "+v"(dr[r].x), "+v"(dr[r].y), "+v"(dr[r].z), "+v"(dr[r].w));
+  }
+  // The local channels' coefficients, one channel per thread, polled until
+  // tagged (as tile_coefs); coefficients that never arrive are used as NaN.
+  {
+    const int64_t copy0 = (g % a.coef_copies) * a.coef_copy;
+    const auto rc = rows_rsrc(a.ecoef, a.coef_copies * a.coef_copy * 8);
+    const int64_t pr =
+        owner ? (copy0 + 4 * static_cast<int64_t>(ch_t)) / 2 : int64_t(kOutOfRange / 16);
+    u32x4 v0 = load_pair(rc, pr), v1 = load_pair(rc, pr + 1);
+    unsigned spins = 0;
+    while (owner && !(pair_tagged(v0, wtag) && pair_tagged(v1, wtag))) {
+      if (++spins > a.spin_limit) {
+        v0 = v1 = u32x4{0x7fc00000u, wtag, 0x7fc00000u, wtag};
+        __hip_atomic_store(a.gave_up, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        break;
+      }
+      __builtin_amdgcn_s_sleep(1);
+      asm volatile("" ::: "memory");  // the reloads are not the loads above
+      v0 = load_pair(rc, pr);
+      v1 = load_pair(rc, pr + 1);
+    }
+    __syncthreads();
+    if (owner) {
+      float* const c = red + tid + tid / VEC;
+      c[0] = bits_f32(v0[0]);
+      c[kComp] = bits_f32(v0[2]);
+      c[2 * kComp] = bits_f32(v1[0]);
+      c[3 * kComp] = bits_f32(v1[2]);
+    }
+    __syncthreads();
+  }
+  float4 cf[VEC];
+#pragma unroll
+  for (int j = 0; j < VEC; ++j) {
+    const uint32_t l = local(j);
+    const float* const c = red + l + l / VEC;
+    cf[j] = make_float4(c[0], c[kComp], c[2 * kComp], c[3 * kComp]);
+  }
+  constexpr int U3 = kGrad ? 4 : 8;
+  for (int q = nk - 1; q >= KR + KL; q -= U3) {
+    uint4 xw[U3], dw[U3];
+#pragma unroll
+    for (int u = 0; u < U3; ++u) {
+      const uint32_t o = q - u >= KR + KL ? roff(q - u) : kOutOfRange;
+      xw[u] = bld16_last(rx, o);
+      if constexpr (kGrad) dw[u] = bld16_last(rd, o);
+    }
+#pragma unroll
+    for (int u = 0; u < U3; ++u)
+      if (q - u >= KR + KL)
+        st16(obase + roff(q - u), apply_words<Tr, kGrad>(xw[u], dw[kGrad ? u : 0], cf));
+  }
+#pragma unroll 2
+  for (int q2 = 0; q2 < kl_w; ++q2) {
+    if (KR + q2 < nk) {
+      const uint4 xw = lds(q2, 0);
+      const uint4 dw = kGrad ? lds(q2, kGrad ? 1 : 0) : xw;
+      st16(obase + roff(KR + q2), apply_words<Tr, kGrad>(xw, dw, cf));
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < KR; ++r)
+    if (r < nk) st16(obase + roff(r), apply_words<Tr, kGrad>(xr[r], dr[kGrad ? r : 0], cf));
+  recorded_exit(a, epoch);
+}
+
 // ---------------------------------------------------------------------------
 // 5. NCHW, one channel per workgroup: workgroup ch sums, finishes and applies
 //    channel ch alone, so no value crosses workgroups - no waits, no
@@ -2445,6 +2827,12 @@ struct FusedPlan {
   int blocks;
   int dyn_rows;   // per-thread streamed rows handed out dynamically
   int dyn_chunk;  // rows per thread in one chunk
+  // Folded (fold > 1): super-rows of `fold` rows, tiles of tw vectors; groups
+  // is then the number of partials per channel, row_groups that of row
+  // ranges.
+  int fold = 1;
+  int tw = 0;
+  int64_t row_groups = 0;
 };
 
 // Channels of the largest fused plan (at most 2 workgroups per CU, tiles of
@@ -2496,6 +2884,93 @@ bool make_fused_plan(const BnGeometry& g, int vec, int blocks_per_cu, FusedPlan*
   fp->slices = 1;
   fp->dyn_rows = 0;
   fp->dyn_chunk = 1;
+  return true;
+}
+
+template <class Tr, bool kGrad>
+constexpr int folded_kr() { return kGrad ? FoldedRows<Tr>::kGrad : FoldedRows<Tr>::kFwd; }
+template <class Tr, bool kGrad>
+constexpr int folded_kl() { return kGrad ? 8 : 16; }
+
+template <class Tr, bool kGrad, int KR = folded_kr<Tr, kGrad>()>
+const void* folded_kernel() {
+  return reinterpret_cast<const void*>(
+      &bn_folded_nhwc_kernel<Tr, kGrad, KR, folded_kl<Tr, kGrad>()>);
+}
+template <class Tr, bool kGrad>
+size_t folded_smem() {
+  return static_cast<size_t>(folded_kl<Tr, kGrad>()) * (kGrad ? 2 : 1) * kFusedThreads * 16;
+}
+
+// Whether one workgroup of every folded kernel fits a CU (-1: no), once per
+// device.
+template <class Tr, bool kGrad>
+int folded_blocks_per_cu() {
+  static std::atomic<int> cached[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
+  const int known = cached[dev].load(std::memory_order_acquire);
+  if (known != 0) return known;
+  int count = 1;
+  const void* kerns[2] = {folded_kernel<Tr, kGrad>(), folded_kernel<Tr, kGrad, kFoldedSmall>()};
+  for (const void* k : kerns) {
+    int nb = 0;
+    hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       static_cast<int>(folded_smem<Tr, kGrad>()));
+    if (e == hipSuccess)
+      e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k, kFusedThreads,
+                                                       folded_smem<Tr, kGrad>());
+    if (e != hipSuccess || nb < 1) count = -1;
+  }
+  cached[dev].store(count, std::memory_order_release);
+  return count;
+}
+
+// The folded plan of an NHWC op whose channel count is no multiple of vec
+// (aligned pointers).  Fewer than 4 super-rows stay with the split kernels.
+bool make_folded_plan(const BnGeometry& g, int vec, int blocks_per_cu, FusedPlan* fp) {
+  if (!g.nhwc || blocks_per_cu < 1 || g.c % vec == 0 || g.c > (int64_t(1) << 20)) return false;
+  int gcd = vec;
+  while (g.c % gcd != 0) gcd >>= 1;
+  const int F = vec / gcd;
+  const int64_t rows = g.rows / F;
+  if (rows < 4) return false;
+  const int64_t cv = g.c * F / vec;
+  const int64_t tile_max = kFoldChannels / vec;
+  int64_t tiles = 1;
+  if (g.c > kFoldChannels || cv > kFusedThreads) tiles = (cv + tile_max - 1) / tile_max;
+  const int64_t tw = (cv + tiles - 1) / tiles;
+  tiles = (cv + tw - 1) / tw;
+  const int64_t ry = kFusedThreads / tw;
+  const int per_channel = tiles == 1 ? 1 : F;  // partials of a channel per row group
+  int64_t groups = static_cast<int64_t>(DeviceCUs()) / tiles;
+  if (groups > kMaxEpochGroups / per_channel) groups = kMaxEpochGroups / per_channel;
+  // At least 2 rows per thread, 4 for wide super-rows: fewer partials per
+  // channel, of few rows each (forward + grad, f16 [16,14,14,333] 25.3 us
+  // with 1, 25.3 with 2, 22.9 with 4; [32,14,14,99] 22.8 / 22.9 / 23.7;
+  // [256,14,14,33] 26.0 / 25.4 / 25.9).
+  const int64_t least = ry * (cv > 128 ? 4 : 2);
+  const int64_t max_groups = (rows + least - 1) / least;
+  if (groups > max_groups) groups = max_groups;
+  if (groups < 1) return false;
+  const int64_t rpg = (rows + groups - 1) / groups;
+  if ((rpg + 64 * ry) * cv * 16 >= (int64_t{1} << 31)) return false;
+  groups = (rows + rpg - 1) / rpg;
+  if (groups * per_channel * g.c > 512 * static_cast<int64_t>(DeviceCUs()) ||
+      g.c > max_fused_channels())
+    return false;
+  *fp = FusedPlan{};
+  fp->tx_shift = 0;
+  fp->ct = fp->ct_conc = static_cast<int>(tiles);
+  fp->cv = cv;
+  fp->groups = groups * per_channel;
+  fp->rows_per_g = rpg;
+  fp->blocks = static_cast<int>(groups * tiles);
+  fp->dyn_rows = 0;
+  fp->dyn_chunk = 1;
+  fp->fold = F;
+  fp->tw = static_cast<int>(tw);
+  fp->row_groups = groups;
   return true;
 }
 
@@ -2813,7 +3288,8 @@ hipError_t launch_fused(const FusedPlan& fp, const BnGeometry& g, const void* x,
   fa.epoch_dev = recorded ? reinterpret_cast<unsigned*>(reinterpret_cast<char*>(region) +
                                                         kEpochOffset)
                           : nullptr;
-  const int ry = kFusedThreads >> fp.tx_shift;
+  const bool folded = fp.fold > 1;
+  const int ry = folded ? kFusedThreads / fp.tw : kFusedThreads >> fp.tx_shift;
   const int64_t nk_max = (fp.rows_per_g + ry - 1) / ry;  // rows of a thread
   const bool sliced = kGrad && fp.slices > 1;
   const bool small = !kGrad && nk_max <= kSmallFwdRows;
@@ -2832,7 +3308,15 @@ hipError_t launch_fused(const FusedPlan& fp, const BnGeometry& g, const void* x,
     size_t shards = slots / per_shard;
     if (shards > 16) shards = 16;
     fa.shards = shards > 0 ? static_cast<int>(shards) : 1;
-    fa.dyn_rows = shards > 0 ? fd.dyn_rows : 0;
+    fa.dyn_rows = shards > 0 && !folded ? fd.dyn_rows : 0;
+  }
+  fa.tail = 0;
+  fa.tail_row = 0;
+  if (folded) {
+    fa.tail = static_cast<int>(g.rows % fp.fold);
+    fa.tail_row = g.rows - fa.tail;
+    fa.coef_copies = static_cast<int>(std::min<int64_t>(
+        kCoefCopies, std::max<int64_t>(1, fp.row_groups / kPollersPerCopy)));
   }
   fa.fin = fin;
   fa.fin.groups = fp.groups;
@@ -2862,8 +3346,28 @@ hipError_t launch_fused(const FusedPlan& fp, const BnGeometry& g, const void* x,
   if constexpr (!kGrad) {
     if (small) kern = fused_kernel<Tr, kGrad, Resident<Tr>::kRegFwdSmall>();
   }
-  const size_t smem = fused_smem<Tr, kGrad>();
+  size_t smem = fused_smem<Tr, kGrad>();
   void* kargs[] = {&fa};
+  FoldedArgs fo;
+  if (folded) {
+    const bool few = nk_max <= kFoldedSmall + folded_kl<Tr, kGrad>();
+    kern = few ? folded_kernel<Tr, kGrad, kFoldedSmall>() : folded_kernel<Tr, kGrad>();
+    smem = folded_smem<Tr, kGrad>();
+    t_last_plan.register_rows = few ? kFoldedSmall : folded_kr<Tr, kGrad>();
+    t_last_plan.lds_rows = folded_kl<Tr, kGrad>();
+    fo.f = fa;
+    fo.fold = fp.fold;
+    fo.cv = static_cast<int>(fp.cv);
+    fo.tw = fp.tw;
+    fo.tiles = fp.ct;
+    fo.ry = ry;
+    fo.rows = g.rows / fp.fold;
+    fo.rows_per_g = fp.rows_per_g;
+    fo.div_tw = FastDiv(static_cast<uint32_t>(fp.tw));
+    fo.div_ry = FastDiv(static_cast<uint32_t>(ry));
+    fo.div_c = FastDiv(static_cast<uint32_t>(g.c));
+    kargs[0] = &fo;
+  }
   if (recorded) {  // no events, no tracing, no chain bookkeeping inside a graph
     hipError_t le = hipLaunchKernel(kern, dim3(fp.blocks), dim3(kFusedThreads), kargs, smem,
                                     stream);
@@ -3041,6 +3545,9 @@ hipError_t forward_t(const BnGeometry& g, const BnFwdArgs& a, void* ws,
     return launch_fused<Tr, false>(fp, g, a.x, nullptr, a.y, fa,
                                                   stream);
   }
+  if (a.is_training && aligned && fused_enabled() &&
+      make_folded_plan(g, Tr::kVec, folded_blocks_per_cu<Tr, false>(), &fp))
+    return launch_fused<Tr, false>(fp, g, a.x, nullptr, a.y, fa, stream);
   note_split_plan(p);
   if (!a.is_training)
     return p.vec == 1
@@ -3089,6 +3596,9 @@ hipError_t grad_t(const BnGeometry& g, const BnGradArgs& a, void* ws,
     return launch_fused<Tr, true>(fp, g, a.x, a.dy, a.dx, fa,
                                                   stream);
   }
+  if (aligned && fused_enabled() &&
+      make_folded_plan(g, Tr::kVec, folded_blocks_per_cu<Tr, true>(), &fp))
+    return launch_fused<Tr, true>(fp, g, a.x, a.dy, a.dx, fa, stream);
   note_split_plan(p);
   hipError_t e =
       p.vec == 1 ? launch_reduce<Tr, 1, true>(p, g, a.x, a.dy, a.saved_mean, partial, stream)

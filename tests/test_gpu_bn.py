@@ -750,3 +750,60 @@ def test_fused_give_up_is_an_error(tmp_path):
                        text=True, timeout=240)
     assert r.returncode == 0, r.stdout + r.stderr
     assert "give-up ok" in r.stdout
+
+
+# Channel counts that are no multiple of a vector (folded super-rows): less
+# than a vector; one vector per super-row and more; a super-row of exactly one
+# pass and of more than one tile; every remainder of rows modulo the fold; the
+# fewest rows and fewer (split path); all rows on chip and streamed ones.
+FOLDED_CASES = [
+    ((1, 4, 8, 1), "float16"),
+    ((3, 5, 7, 3), "float32"),
+    ((2, 3, 11, 5), "bfloat16"),
+    ((4, 9, 9, 63), "float16"),
+    ((2, 17, 19, 130), "float32"),
+    ((2, 8, 9, 300), "float16"),
+    ((1, 37, 5, 511), "bfloat16"),
+    ((2, 9, 7, 513), "float16"),
+    ((1, 16, 3, 1021), "float32"),
+    ((1, 5, 6, 33), "float16"),       # 3 super-rows: split path
+    ((64, 56, 56, 33), "float16"),
+    ((32, 56, 56, 255), "bfloat16"),
+    ((32, 56, 56, 99), "float32"),
+]
+
+
+def _folded_rows(shape, dtype):
+    vec = 4 if dtype == "float32" else 8
+    return shape[0] * shape[1] * shape[2] // (vec // np.gcd(shape[3], vec))
+
+
+@pytest.mark.parametrize("is_training", [True, False])
+@pytest.mark.parametrize("shape,dtype", FOLDED_CASES)
+def test_folded_matches_oracle(dev, shape, dtype, is_training):
+    rng = np.random.default_rng(zlib.crc32(repr((shape, dtype, "folded")).encode()))
+    eps = 1e-3
+    c = shape[-1]
+    x, scale, offset, dy = _inputs(rng, shape, dtype, "NHWC", loc=0.5)
+    dy = gen(rng, shape, dtype, loc=0.25)
+    mean = (0.1 * rng.standard_normal(c)).astype(np.float32)
+    var = rng.uniform(0.5, 2.0, c).astype(np.float32)
+    fwd, grad = _run_fwd_grad(dev, x, scale, offset, dy, dtype, "NHWC", eps, mean=mean, var=var,
+                              factor=0.75 if is_training else 1.0, is_training=is_training)
+    assert ops.fused_batch_norm_last_plan()["fused"] == (1 if _folded_rows(shape, dtype) >= 4 else 0)
+    ry, rbm, rbv, rsm, rsv = oracle.bn_fwd(x, scale, offset, mean, var, epsilon=eps,
+                                          exponential_avg_factor=0.75 if is_training else 1.0,
+                                          is_training=is_training, dtype=dtype)
+    assert_close(to_np(fwd.y, dtype), ry, dtype, ACT_TOL[dtype], "y")
+    for name, got, ref in (("batch_mean", fwd.batch_mean, rbm),
+                           ("batch_variance", fwd.batch_variance, rbv),
+                           ("reserve_space_1", fwd.reserve_space_1, rsm),
+                           ("reserve_space_2", fwd.reserve_space_2, rsv)):
+        assert_close(got.cpu().numpy(), ref, "float32", STAT_TOL, name)
+    rdx, rsb, rob = oracle.bn_grad(dy, x, scale, fwd.reserve_space_1.cpu().numpy(),
+                                   fwd.reserve_space_2.cpu().numpy(), epsilon=eps, dtype=dtype,
+                                   is_training=is_training)
+    assert_close(to_np(grad.x_backprop, dtype), rdx, dtype, ACT_TOL[dtype], "x_backprop")
+    assert_close(grad.scale_backprop.cpu().numpy(), rsb, "float32", STAT_TOL, "scale_backprop")
+    assert_close(grad.offset_backprop.cpu().numpy(), rob, "float32", STAT_TOL, "offset_backprop")
+    assert torch.all(grad.reserve_space_4 == 0) and torch.all(grad.reserve_space_5 == 0)

@@ -95,6 +95,41 @@ def test_recorded_training_step_replays(dev, tune, shape, slice_tw, slices):
     assert not ops.fused_batch_norm_barrier_timed_out()
 
 
+@pytest.mark.parametrize("shape,fmt", [((8, 13, 13, 99), "NHWC"), ((2, 9, 7, 515), "NHWC")])
+def test_recorded_batch_norm_replays(dev, shape, fmt):
+    """The other batch-norm kernels whose workgroups wait for one another,
+    recorded: three replays between eager launches, bit for bit."""
+    gen_ = torch.Generator(device=dev)
+    gen_.manual_seed(33)
+    c = shape[-1] if fmt == "NHWC" else shape[1]
+    x, dy = (torch.randn(shape, generator=gen_, device=dev).half() for _ in range(2))
+    scale = torch.rand(c, generator=gen_, device=dev) + 0.5
+    offset = torch.randn(c, generator=gen_, device=dev)
+    e = torch.empty(0, device=dev)
+    kw = dict(epsilon=EPS, data_format=fmt)
+
+    def step():
+        f = ops.FusedBatchNormV3(x, scale, offset, e, e, **kw)
+        assert ops.fused_batch_norm_last_plan()["fused"] != 0
+        return tuple(f) + tuple(ops.FusedBatchNormGradV3(
+            dy, x, scale, f.reserve_space_1, f.reserve_space_2, f.reserve_space_3, **kw))
+
+    want = [t.clone() for t in step()]
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        outs = step()
+    for _ in range(3):
+        for t in outs:
+            t.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(outs, want))
+        assert all(torch.equal(a, b) for a, b in zip(step(), want))
+        torch.cuda.synchronize()
+    assert not ops.fused_batch_norm_barrier_timed_out()
+
+
 @pytest.mark.parametrize("gdtype", [torch.float32, torch.bfloat16])
 def test_grouped_adam_recorded_replays(dev, gdtype):
     """MusaGroupedResourceApplyAdam recorded into a graph (its tensor table
