@@ -768,7 +768,7 @@ constexpr int kPollersPerCopy = 32;
 // phase 3, and with it the bf16 and f32 forwards schedule worse - so it is
 // chosen per type and direction, by the spill-free KR it allows.
 // kRegFwdSmall: the forward's register rows when a thread has at most
-// kSmallFwdRows rows (the 14x14 and 7x7 stage shapes): there fewer register
+// kSmallFwdRows rows (the 14x14 stage shape): there fewer register
 // rows measured faster even where that leaves rows to stream (each register
 // row adds unrolled code to a kernel run about once, and the resident loads
 // arrive as one burst that streams worse than the pipelined loop).
@@ -802,6 +802,34 @@ template <> struct Resident<TBF16> {
   static constexpr int kRegFwdSmall = 8;
   static constexpr int kPaFwd = 0, kPbFwd = 0, kPaGrad = 0, kPbGrad = 0;
 };
+
+template <class Tr, bool kGrad>
+constexpr int fused_kr() { return kGrad ? Resident<Tr>::kRegGrad : Resident<Tr>::kRegFwd; }
+template <class Tr, bool kGrad>
+constexpr int fused_kl() { return kGrad ? Resident<Tr>::kLdsGrad : Resident<Tr>::kLdsFwd; }
+
+// Ops with few rows per thread run kernels with few resident rows: their
+// code, unrolled per resident row, runs once, and the loads of rows a thread
+// does not have are still issued.  Forward / grad back to back, (KR, KL) of
+// the large kernels against the chosen one:
+//   f16 [32,14,14,256] (2 rows)   12.0 / 13.5 -> 10.6 / 9.9 us with (3, 1)
+//   f16 [32,7,7,2048] (4)         11.6 / 13.3 -> 10.1 / 9.9 us with (3, 1)
+//   f16 [32,14,14,1024] (7)       12.4 / 15.2 -> 11.4 / 12.7 us with (6, 2)
+//   f32 [32,56,56,64] (13)        15.1 / 19.0 -> 14.0 / 18.2 us
+//   f16 [64,28,28,384] (19)       23.8 -> 21.7 us (forward, (13, 1))
+//   f16 [64,56,56,128] (25)       27.6 -> 24.6 us (forward, (13, 1))
+// The rows such a forward streams come back from the caches; at 49 rows
+// (f16 [256,14,14,1024]) (13, 1) takes 45.0 us and the (8, 18) kernel 43.9,
+// and the grads past 14 rows gain nothing ([256,7,7,2048] bf16 32.6 us with
+// all resident rows, 33.2 with (12, 2)).
+struct FewRows {
+  int kr, kl;
+  int64_t most;  // rows per thread up to which it runs
+};
+constexpr FewRows kFew0 = {3, 1, 4};
+constexpr FewRows kFew1Fwd = {6, 2, 8}, kFew1Grad = {6, 2, 14};
+constexpr FewRows kFew2Fwd = {13, 1, 32};
+constexpr int64_t kSmallFwdRows = 64;  // then (kRegFwdSmall, kLdsFwd), forward only
 
 struct FusedArgs {
   const void* x;
@@ -1388,7 +1416,7 @@ __global__ __launch_bounds__(kFusedThreads) void bn_fused_nhwc_kernel(FusedArgs 
   // The wave's last LDS row (see the LDS loops below); the large forwards
   // keep all KL slots (bounded, their phase 1 was scheduled worse: the
   // 56x56 forward 178 -> 194 us).
-  constexpr bool kWaveLds = kGrad || KR == Resident<Tr>::kRegFwdSmall;
+  constexpr bool kWaveLds = kGrad || KR < fused_kr<Tr, kGrad>();
   const int nk_w = __builtin_amdgcn_readfirstlane(static_cast<int>(nk));
   const int kl_w =
       !kWaveLds ? KL : (nk_w - KR < 0 ? 0 : (nk_w - KR < KL ? nk_w - KR : KL));
@@ -2078,8 +2106,8 @@ __device__ inline void recorded_exit(const FusedArgs& a, unsigned epoch) {
 }
 
 // ---------------------------------------------------------------------------
-// 4c. Folded kernel: NHWC with a channel count that is no multiple of the
-//     vector width.  F = VEC / gcd(C, VEC) rows are one super-row of C * F
+// 4c. Folded kernel: NHWC with any channel count (one that is no multiple of
+//     the vector width, and others: prefer_folded).  F = VEC / gcd(C, VEC) rows are one super-row of C * F
 //     elements, a whole number of 16-byte vectors, in which every vector
 //     position has fixed channels (element e: channel e mod C); rows past the
 //     last whole super-row (fewer than F) are the finishing waves' (tail).
@@ -2104,13 +2132,11 @@ __device__ inline void recorded_exit(const FusedArgs& a, unsigned epoch) {
 constexpr int kFoldChannels = 512; // most channels (one tile) or columns of a tile
 constexpr int kFoldParts = 32;     // most threads that share one channel's sums
 
-// Register rows per thread (the largest spill-free counts), and of the
-// kernels for at most that many rows and the LDS rows (kFoldedSmall: less
-// code, run once).
+// Register rows per thread (the largest spill-free counts); ops with few rows
+// per thread run the FewRows counts.
 template <class Tr> struct FoldedRows { static constexpr int kFwd = 24, kGrad = 11; };
 template <> struct FoldedRows<TF32> { static constexpr int kFwd = 28, kGrad = 13; };
 template <> struct FoldedRows<TBF16> { static constexpr int kFwd = 24, kGrad = 9; };
-constexpr int kFoldedSmall = 6;
 
 struct FoldedArgs {
   FusedArgs f;         // c: real channels; groups: partial words per channel
@@ -2722,17 +2748,31 @@ bool fused_enabled() {
 // Upper bound on fused workgroups (one or two per CU); sizes the partials.
 int64_t fused_group_bound() { return 2 * static_cast<int64_t>(DeviceCUs()); }
 
-template <class Tr, bool kGrad>
-constexpr int fused_kr() { return kGrad ? Resident<Tr>::kRegGrad : Resident<Tr>::kRegFwd; }
-template <class Tr, bool kGrad>
-constexpr int fused_kl() { return kGrad ? Resident<Tr>::kLdsGrad : Resident<Tr>::kLdsFwd; }
-
-constexpr int64_t kSmallFwdRows = 64;
-
-template <class Tr, bool kGrad, int KR = fused_kr<Tr, kGrad>(), bool kSliced = false>
+template <class Tr, bool kGrad, int KR = fused_kr<Tr, kGrad>(), bool kSliced = false,
+          int KL = fused_kl<Tr, kGrad>()>
 const void* fused_kernel() {
-  return reinterpret_cast<const void*>(
-      &bn_fused_nhwc_kernel<Tr, kGrad, KR, fused_kl<Tr, kGrad>(), kSliced>);
+  return reinterpret_cast<const void*>(&bn_fused_nhwc_kernel<Tr, kGrad, KR, KL, kSliced>);
+}
+
+// The unsliced kernel for ops of nk rows per thread, and its resident rows.
+struct FusedPick {
+  const void* kernel;
+  int kr, kl;
+};
+template <class Tr, bool kGrad>
+FusedPick pick_fused(int64_t nk) {
+  constexpr FewRows f1 = kGrad ? kFew1Grad : kFew1Fwd;
+  if (nk <= kFew0.most)
+    return {fused_kernel<Tr, kGrad, kFew0.kr, false, kFew0.kl>(), kFew0.kr, kFew0.kl};
+  if (nk <= f1.most) return {fused_kernel<Tr, kGrad, f1.kr, false, f1.kl>(), f1.kr, f1.kl};
+  if constexpr (!kGrad) {
+    constexpr FewRows f2 = kFew2Fwd;
+    if (nk <= f2.most) return {fused_kernel<Tr, kGrad, f2.kr, false, f2.kl>(), f2.kr, f2.kl};
+    if (nk <= kSmallFwdRows)
+      return {fused_kernel<Tr, kGrad, Resident<Tr>::kRegFwdSmall>(), Resident<Tr>::kRegFwdSmall,
+              fused_kl<Tr, kGrad>()};
+  }
+  return {fused_kernel<Tr, kGrad>(), fused_kr<Tr, kGrad>(), fused_kl<Tr, kGrad>()};
 }
 
 template <class Tr, bool kGrad>
@@ -2782,12 +2822,12 @@ int fused_blocks_per_cu() {
     hipError_t e = hipFuncSetAttribute(fused_kernel<Tr, kGrad>(),
                                        hipFuncAttributeMaxDynamicSharedMemorySize,
                                        static_cast<int>(fused_smem<Tr, kGrad>()));
-    if constexpr (!kGrad) {  // the small-shape forward: same LDS, fewer VGPRs
+    // The kernels for fewer rows: the same LDS, no more VGPRs.
+    for (int64_t nk : {int64_t(1), kFew1Fwd.most, kFew1Grad.most, kFew2Fwd.most, kSmallFwdRows})
       if (e == hipSuccess)
-        e = hipFuncSetAttribute(fused_kernel<Tr, kGrad, Resident<Tr>::kRegFwdSmall>(),
+        e = hipFuncSetAttribute(pick_fused<Tr, kGrad>(nk).kernel,
                                 hipFuncAttributeMaxDynamicSharedMemorySize,
                                 static_cast<int>(fused_smem<Tr, kGrad>()));
-    }
     if constexpr (kGrad) {  // the sliced grads: same LDS, and they must fit as often
       int overlap_ns = 0;
       if (e == hipSuccess)
@@ -2827,9 +2867,8 @@ struct FusedPlan {
   int blocks;
   int dyn_rows;   // per-thread streamed rows handed out dynamically
   int dyn_chunk;  // rows per thread in one chunk
-  // Folded (fold > 1): super-rows of `fold` rows, tiles of tw vectors; groups
-  // is then the number of partials per channel, row_groups that of row
-  // ranges.
+  // Folded (tw > 0): super-rows of `fold` rows, tiles of tw vectors; groups is
+  // then the number of partials per channel, row_groups that of row ranges.
   int fold = 1;
   int tw = 0;
   int64_t row_groups = 0;
@@ -2892,10 +2931,19 @@ constexpr int folded_kr() { return kGrad ? FoldedRows<Tr>::kGrad : FoldedRows<Tr
 template <class Tr, bool kGrad>
 constexpr int folded_kl() { return kGrad ? 8 : 16; }
 
-template <class Tr, bool kGrad, int KR = folded_kr<Tr, kGrad>()>
+template <class Tr, bool kGrad, int KR = folded_kr<Tr, kGrad>(), int KL = folded_kl<Tr, kGrad>()>
 const void* folded_kernel() {
-  return reinterpret_cast<const void*>(
-      &bn_folded_nhwc_kernel<Tr, kGrad, KR, folded_kl<Tr, kGrad>()>);
+  return reinterpret_cast<const void*>(&bn_folded_nhwc_kernel<Tr, kGrad, KR, KL>);
+}
+template <class Tr, bool kGrad>
+FusedPick pick_folded(int64_t nk) {
+  constexpr FewRows f1 = kGrad ? kFew1Grad : kFew1Fwd;
+  if (nk <= f1.most) return {folded_kernel<Tr, kGrad, f1.kr, f1.kl>(), f1.kr, f1.kl};
+  if constexpr (!kGrad) {
+    constexpr FewRows f2 = kFew2Fwd;
+    if (nk <= f2.most) return {folded_kernel<Tr, kGrad, f2.kr, f2.kl>(), f2.kr, f2.kl};
+  }
+  return {folded_kernel<Tr, kGrad>(), folded_kr<Tr, kGrad>(), folded_kl<Tr, kGrad>()};
 }
 template <class Tr, bool kGrad>
 size_t folded_smem() {
@@ -2912,8 +2960,8 @@ int folded_blocks_per_cu() {
   const int known = cached[dev].load(std::memory_order_acquire);
   if (known != 0) return known;
   int count = 1;
-  const void* kerns[2] = {folded_kernel<Tr, kGrad>(), folded_kernel<Tr, kGrad, kFoldedSmall>()};
-  for (const void* k : kerns) {
+  for (int64_t nk : {int64_t(1), kFew2Fwd.most, kFew2Fwd.most + 1}) {
+    const void* const k = pick_folded<Tr, kGrad>(nk).kernel;
     int nb = 0;
     hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
                                        static_cast<int>(folded_smem<Tr, kGrad>()));
@@ -2926,10 +2974,30 @@ int folded_blocks_per_cu() {
   return count;
 }
 
-// The folded plan of an NHWC op whose channel count is no multiple of vec
-// (aligned pointers).  Fewer than 4 super-rows stay with the split kernels.
+// Whole-vector channel counts (F = 1) that the folded kernel runs faster
+// than bn_fused_nhwc_kernel, whose tiles are a power of two of at most 32
+// vectors:
+//  - rows of one tile that leave at least 5 of 16 lanes idle (forward + grad
+//    back to back: f16 [64,56,56,136] 82.2 -> 72.4 us, [64,56,56,72] 49.5 ->
+//    43.0, f32 [32,14,14,72] 22.1 -> 19.6; 13 of 16 lanes in use, f16
+//    [64,56,56,104], 59.0 -> 62.1);
+//  - rows in several tiles whose ends fall inside cache lines, from 16 MiB,
+//    where the folded kernel streams whole rows (f16 [64,28,28,400] 68.6 ->
+//    58.3, f32 [64,56,56,264] 312 -> 262; f16 [32,14,14,400] 26.5 -> 29.6:
+//    its partials are too many for few rows; whole lines, f16 [64,28,28,384],
+//    54.7 -> 55.4).
+// A forced slice width ("bn_slice_tw") keeps the fused kernel.
+bool prefer_folded(const BnGeometry& g, int vec) {
+  if (!g.nhwc || g.c % vec != 0 || TuneValue(kTuneBnSliceTw) >= 0) return false;
+  const int64_t cv = g.c / vec;
+  if (cv <= 32) return cv > 8 && cv * 16 <= (int64_t(11) << pow2_ceil_log2(cv));
+  return g.c <= kFoldChannels && cv * 16 % 128 != 0 && g.rows * cv * 16 >= (int64_t(16) << 20);
+}
+
+// The folded plan of an NHWC op (aligned pointers).  Fewer than 4 super-rows
+// stay with the split kernels.
 bool make_folded_plan(const BnGeometry& g, int vec, int blocks_per_cu, FusedPlan* fp) {
-  if (!g.nhwc || blocks_per_cu < 1 || g.c % vec == 0 || g.c > (int64_t(1) << 20)) return false;
+  if (!g.nhwc || blocks_per_cu < 1 || g.c > (int64_t(1) << 20)) return false;
   int gcd = vec;
   while (g.c % gcd != 0) gcd >>= 1;
   const int F = vec / gcd;
@@ -3288,20 +3356,20 @@ hipError_t launch_fused(const FusedPlan& fp, const BnGeometry& g, const void* x,
   fa.epoch_dev = recorded ? reinterpret_cast<unsigned*>(reinterpret_cast<char*>(region) +
                                                         kEpochOffset)
                           : nullptr;
-  const bool folded = fp.fold > 1;
+  const bool folded = fp.tw > 0;
   const int ry = folded ? kFusedThreads / fp.tw : kFusedThreads >> fp.tx_shift;
   const int64_t nk_max = (fp.rows_per_g + ry - 1) / ry;  // rows of a thread
   const bool sliced = kGrad && fp.slices > 1;
-  const bool small = !kGrad && nk_max <= kSmallFwdRows;
-  int kr = small ? Resident<Tr>::kRegFwdSmall : fused_kr<Tr, kGrad>();
+  FusedPick pick = pick_fused<Tr, kGrad>(nk_max);
   if constexpr (kGrad) {
-    if (sliced) kr = Resident<Tr>::kRegGradSliced;
+    if (sliced)
+      pick = {sliced_kernel<Tr>(), Resident<Tr>::kRegGradSliced, fused_kl<Tr, kGrad>()};
   }
   {
     FusedPlan fd = fp;
     constexpr int kPre = kGrad ? Resident<Tr>::kPaGrad + Resident<Tr>::kPbGrad
                                : Resident<Tr>::kPaFwd + Resident<Tr>::kPbFwd;
-    set_dynamic_share(&fd, kr + fused_kl<Tr, kGrad>(), kPre, kGrad ? 4 : 8);
+    set_dynamic_share(&fd, pick.kr + pick.kl, kPre, kGrad ? 4 : 8);
     fa.dyn_chunk = fd.dyn_chunk;
     const size_t slots = kQueueBytes / sizeof(unsigned);
     const size_t per_shard = static_cast<size_t>(fp.ct) * (kFusedThreads / 64);
@@ -3327,34 +3395,22 @@ hipError_t launch_fused(const FusedPlan& fp, const BnGeometry& g, const void* x,
   t_last_plan.channel_tiles = fp.ct;
   t_last_plan.dynamic_rows = fa.dyn_rows;
   t_last_plan.dynamic_chunk = fa.dyn_chunk;
-  t_last_plan.register_rows = kr;
-  t_last_plan.lds_rows = fused_kl<Tr, kGrad>();
   t_last_plan.slices = fp.slices;
   const char* name = kGrad ? "tfma_bn_grad_fused" : "tfma_bn_fwd_fused";
   SetLastKernel(name);
-  const void* kern = fused_kernel<Tr, kGrad>();
   if constexpr (kGrad) {
-    if (sliced) {
-      kern = sliced_kernel<Tr>();
-      // No dynamic tail: the kernel that hides the slices' hand-offs.
-      if (fp.ct_conc == 1 && fa.dyn_rows == 0 && sliced_overlap_enabled()) {
-        kern = sliced_overlap_kernel<Tr>();
-        t_last_plan.register_rows = Resident<Tr>::kRegGradOverlap;
-      }
+    // No dynamic tail: the kernel that hides the slices' hand-offs.
+    if (sliced && fp.ct_conc == 1 && fa.dyn_rows == 0 && sliced_overlap_enabled()) {
+      pick.kernel = sliced_overlap_kernel<Tr>();
+      pick.kr = Resident<Tr>::kRegGradOverlap;
     }
-  }
-  if constexpr (!kGrad) {
-    if (small) kern = fused_kernel<Tr, kGrad, Resident<Tr>::kRegFwdSmall>();
   }
   size_t smem = fused_smem<Tr, kGrad>();
   void* kargs[] = {&fa};
   FoldedArgs fo;
   if (folded) {
-    const bool few = nk_max <= kFoldedSmall + folded_kl<Tr, kGrad>();
-    kern = few ? folded_kernel<Tr, kGrad, kFoldedSmall>() : folded_kernel<Tr, kGrad>();
+    pick = pick_folded<Tr, kGrad>(nk_max);
     smem = folded_smem<Tr, kGrad>();
-    t_last_plan.register_rows = few ? kFoldedSmall : folded_kr<Tr, kGrad>();
-    t_last_plan.lds_rows = folded_kl<Tr, kGrad>();
     fo.f = fa;
     fo.fold = fp.fold;
     fo.cv = static_cast<int>(fp.cv);
@@ -3368,6 +3424,9 @@ hipError_t launch_fused(const FusedPlan& fp, const BnGeometry& g, const void* x,
     fo.div_c = FastDiv(static_cast<uint32_t>(g.c));
     kargs[0] = &fo;
   }
+  t_last_plan.register_rows = pick.kr;
+  t_last_plan.lds_rows = pick.kl;
+  const void* const kern = pick.kernel;
   if (recorded) {  // no events, no tracing, no chain bookkeeping inside a graph
     hipError_t le = hipLaunchKernel(kern, dim3(fp.blocks), dim3(kFusedThreads), kargs, smem,
                                     stream);
@@ -3540,6 +3599,9 @@ hipError_t forward_t(const BnGeometry& g, const BnFwdArgs& a, void* ws,
   FusedPlan fp;
   if (a.is_training && nchw_owned_ok(g, p.vec, sizeof(typename Tr::S)))
     return launch_nchw_owned<Tr, false>(g, a.x, nullptr, a.y, fa, stream);
+  if (a.is_training && p.vec > 1 && fused_enabled() && prefer_folded(g, p.vec) &&
+      make_folded_plan(g, p.vec, folded_blocks_per_cu<Tr, false>(), &fp))
+    return launch_fused<Tr, false>(fp, g, a.x, nullptr, a.y, fa, stream);
   if (a.is_training && p.vec > 1 && fused_enabled() &&
       choose_fused_plan<Tr, false>(g, p.vec, &fp)) {
     return launch_fused<Tr, false>(fp, g, a.x, nullptr, a.y, fa,
@@ -3591,6 +3653,9 @@ hipError_t grad_t(const BnGeometry& g, const BnGradArgs& a, void* ws,
   FusedPlan fp;
   if (nchw_owned_ok(g, p.vec, sizeof(typename Tr::S)))
     return launch_nchw_owned<Tr, true>(g, a.x, a.dy, a.dx, fa, stream);
+  if (p.vec > 1 && fused_enabled() && prefer_folded(g, p.vec) &&
+      make_folded_plan(g, p.vec, folded_blocks_per_cu<Tr, true>(), &fp))
+    return launch_fused<Tr, true>(fp, g, a.x, a.dy, a.dx, fa, stream);
   if (p.vec > 1 && fused_enabled() &&
       choose_fused_plan<Tr, true>(g, p.vec, &fp)) {
     return launch_fused<Tr, true>(fp, g, a.x, a.dy, a.dx, fa,

@@ -770,6 +770,8 @@ FOLDED_CASES = [
     ((64, 56, 56, 33), "float16"),
     ((32, 56, 56, 255), "bfloat16"),
     ((32, 56, 56, 99), "float32"),
+    ((4, 9, 9, 72), "float16"),       # whole vectors, lanes idle in a power-of-two tile
+    ((64, 28, 28, 264), "bfloat16"),  # whole vectors, row ends inside cache lines
 ]
 
 
@@ -807,3 +809,27 @@ def test_folded_matches_oracle(dev, shape, dtype, is_training):
     assert_close(grad.scale_backprop.cpu().numpy(), rsb, "float32", STAT_TOL, "scale_backprop")
     assert_close(grad.offset_backprop.cpu().numpy(), rob, "float32", STAT_TOL, "offset_backprop")
     assert torch.all(grad.reserve_space_4 == 0) and torch.all(grad.reserve_space_5 == 0)
+
+
+@pytest.mark.parametrize("rows", [65536, 65537, 131072, 131073, 229376, 229377, 524288, 524289])
+def test_few_rows_kernels_match_oracle(dev, rows):
+    """Rows per thread (256 row groups of 64 row lanes) on both sides of every
+    change of kernel: 4, 8, 14 (grad) and 32 (forward)."""
+    rng = np.random.default_rng(rows)
+    shape, dtype = (1, 1, rows, 64), "float16"
+    x, scale, offset, dy = _inputs(rng, shape, dtype, "NHWC", loc=0.5)
+    fwd, grad = _run_fwd_grad(dev, x, scale, offset, dy, dtype, "NHWC", 1e-3)
+    ry, _, rbv, rsm, rsv = oracle.bn_fwd(x, scale, offset, epsilon=1e-3, dtype=dtype)
+    assert_close(to_np(fwd.y, dtype), ry, dtype, ACT_TOL[dtype], "y")
+    assert_close(fwd.batch_variance.cpu().numpy(), rbv, "float32", STAT_TOL, "batch_variance")
+    assert_close(fwd.reserve_space_1.cpu().numpy(), rsm, "float32", STAT_TOL, "reserve_space_1")
+    assert_close(fwd.reserve_space_2.cpu().numpy(), rsv, "float32", STAT_TOL, "reserve_space_2")
+    rdx, rsb, rob = oracle.bn_grad(dy, x, scale, fwd.reserve_space_1.cpu().numpy(),
+                                   fwd.reserve_space_2.cpu().numpy(), epsilon=1e-3, dtype=dtype)
+    assert_close(to_np(grad.x_backprop, dtype), rdx, dtype, ACT_TOL[dtype], "x_backprop")
+    # Sums of 65536 rows and more cancel: relative to sqrt(rows), the spread of
+    # such a sum of N(0, 1) terms.
+    for name, got, ref in (("scale_backprop", grad.scale_backprop, rsb),
+                           ("offset_backprop", grad.offset_backprop, rob)):
+        err = np.abs(got.cpu().numpy().astype(np.float64) - ref).max()
+        assert err <= STAT_TOL * max(np.abs(ref).max(), np.sqrt(rows)), name
