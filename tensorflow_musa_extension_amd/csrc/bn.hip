@@ -34,6 +34,7 @@
 // workgroup uses the same K.
 #include <hip/hip_ext.h>
 
+
 #include <atomic>
 #include <mutex>
 
@@ -261,6 +262,23 @@ __device__ inline float chan_shift(const typename Tr::S* x, int64_t ch, int64_t 
   return shift_of(v);
 }
 
+// The same K for NCHW tensors of fewer than 2^31 elements, with 32-bit
+// arithmetic: div_plane divides by the plane (a 64-bit division per sample
+// took 1-3 us of a workgroup's start).
+template <class Tr>
+__device__ inline float chan_shift_nchw(const typename Tr::S* x, uint32_t ch, uint32_t n,
+                                        uint32_t c, const FastDiv& div_plane) {
+  const uint32_t js[5] = {0u, n / 4, n / 2, n - (n + 3) / 4, n - 1};
+  float v[5];
+#pragma unroll
+  for (int i = 0; i < 5; ++i) {
+    uint32_t img, r;
+    div_plane.divmod(js[i], img, r);
+    v[i] = Tr::ld(x[(img * c + ch) * div_plane.d + r]);
+  }
+  return shift_of(v);
+}
+
 // ---------------------------------------------------------------------------
 // 1. Reduce.
 // ---------------------------------------------------------------------------
@@ -472,11 +490,11 @@ __device__ inline FinIn fin_inputs(const FinArgs& a, int ch) {
 
 // Final statistics and apply coefficients of channel ch from the double
 // sums s1, s2 over all of the channel's elements and its inputs p (FinIn or
-// FinLoad); writes the op's per-channel outputs and returns the coefficients
+// FinLoad); writes (where `write`) the op's per-channel outputs and returns the coefficients
 // {mean, a, b, c2} for apply_one().
 template <class Tr, bool kGrad, class In>
 __device__ inline float4 finish_channel(const FinArgs& a, int ch, double s1, double s2,
-                                        const In& p) {
+                                        const In& p, bool write = true) {
   const double n = static_cast<double>(a.n);
   if constexpr (!kGrad) {
     const double mean = static_cast<double>(p.kshift()) + s1 / n;
@@ -487,23 +505,27 @@ __device__ inline float4 finish_channel(const FinArgs& a, int ch, double s1, dou
     const float nf = static_cast<float>(a.n);
     const float nm1 = static_cast<float>(a.n > 1 ? a.n - 1 : 1);
     const float adj = nf / nm1;
-    a.saved_mean[ch] = mean_f;
-    a.saved_var[ch] = var_f;
-    if (a.f == 1.0f) {
-      a.batch_mean[ch] = mean_f;
-      a.batch_var[ch] = var_f * adj;
-    } else {
-      const float omf = 1.0f - a.f;
-      a.batch_mean[ch] = p.mean_in() * omf + mean_f * a.f;
-      a.batch_var[ch] = p.var_in() * omf + (var_f * adj) * a.f;
+    if (write) {
+      a.saved_mean[ch] = mean_f;
+      a.saved_var[ch] = var_f;
+      if (a.f == 1.0f) {
+        a.batch_mean[ch] = mean_f;
+        a.batch_var[ch] = var_f * adj;
+      } else {
+        const float omf = 1.0f - a.f;
+        a.batch_mean[ch] = p.mean_in() * omf + mean_f * a.f;
+        a.batch_var[ch] = p.var_in() * omf + (var_f * adj) * a.f;
+      }
     }
     const float inv = 1.0f / __builtin_sqrtf(var_f + a.eps);
     return make_float4(mean_f, inv * p.scale(), p.offset(), 0.f);
   } else {
     const float mu = p.mean_in();
     const float k = 1.0f / __builtin_sqrtf(p.var_in() + a.eps);
-    a.offset_bp[ch] = static_cast<float>(s1);
-    a.scale_bp[ch] = static_cast<float>(s2 * static_cast<double>(k));
+    if (write) {
+      a.offset_bp[ch] = static_cast<float>(s1);
+      a.scale_bp[ch] = static_cast<float>(s2 * static_cast<double>(k));
+    }
     if (a.is_training) {
       const float mean_dy = static_cast<float>(s1 / n);
       const float mean_dyxc = static_cast<float>(s2 / n);
@@ -875,11 +897,11 @@ struct FusedArgs {
   unsigned long long* ekey;
   unsigned epoch;
   unsigned* epoch_dev;
+  FinArgs fin;
   // Folded launches: rows [tail_row, tail_row + tail) are no whole super-row;
   // the waves that finish a channel sum and write them.
-  int tail;
   int64_t tail_row;
-  FinArgs fin;
+  int tail;
 };
 
 // Per-wave phase timestamps of the fused NHWC kernel, compiled in only with
@@ -1273,10 +1295,10 @@ __device__ __forceinline__ void finish_channel_blocks(const FusedArgs& a, int cs
       t2 += __shfl_xor(t2, off, 64);
     }
     float4 cfc = make_float4(0.f, 0.f, 0.f, 0.f);
-    using S = typename Tr::S;
-    const S* const xt = static_cast<const S*>(a.x) + a.tail_row * a.c + ch;
-    const S* const dt = static_cast<const S*>(a.dy) + a.tail_row * a.c + ch;
     if constexpr (kFold) {
+      using S = typename Tr::S;
+      const S* const xt = static_cast<const S*>(a.x) + a.tail_row * a.c + ch;
+      const S* const dt = static_cast<const S*>(a.dy) + a.tail_row * a.c + ch;
       const float kc = kGrad ? fin_in.mi : fin_in.k;
       for (int r = 0; r < a.tail && lane < B && chv; ++r) {
         const float xc = Tr::ld(xt[r * a.c]) - kc;
@@ -1288,6 +1310,9 @@ __device__ __forceinline__ void finish_channel_blocks(const FusedArgs& a, int cs
     if (lane < B && chv) cfc = finish_channel<Tr, kGrad>(a.fin, ch, t1, t2, fin_in);
     store_coefs(a, ch, chv, cfc, lane, B, etag);
     if constexpr (kFold) {
+      using S = typename Tr::S;
+      const S* const xt = static_cast<const S*>(a.x) + a.tail_row * a.c + ch;
+      const S* const dt = static_cast<const S*>(a.dy) + a.tail_row * a.c + ch;
       S* const ot = static_cast<S*>(a.out) + a.tail_row * a.c + ch;
       for (int r = 0; r < a.tail && lane < B && chv; ++r)
         ot[r * a.c] = apply_one<Tr, kGrad>(xt[r * a.c], kGrad ? dt[r * a.c] : S(0), cfc);
@@ -2128,6 +2153,13 @@ __device__ inline void recorded_exit(const FusedArgs& a, unsigned epoch) {
 //     to back: f16 [64,35,35,99] 34.2 / 48.7 -> 15.7 / 17.6 us, [256,56,56,
 //     163] 352 / 672 -> 133 / 217 us, f32 [128,28,28,1021] 384 / 597 -> 195
 //     / 351 us, f16 [32,14,14,99] 11.0 / 13.2 -> 11.4 / 11.6 us.
+//     kUnit: NCHW planes that are no multiple of a vector.  VEC / gcd(plane,
+//     VEC) channels - a unit - are a whole number of vectors, contiguous in
+//     every image: a unit is a tile, its rows the images (element e: channel
+//     e / plane).  With one row group the workgroup finishes its channels
+//     itself and waits for none.  Forward / grad: f16 [256,2048,7,7] 57.7 /
+//     69.7 -> 28.5 / 39.4 us, bf16 [64,1024,14,14] 41.4 / 40.7 -> 21.8 / 26.0,
+//     f16 [32,512,7,7] 11.9 / 11.1 -> 7.4 / 8.1.
 // ---------------------------------------------------------------------------
 constexpr int kFoldChannels = 512; // most channels (one tile) or columns of a tile
 constexpr int kFoldParts = 32;     // most threads that share one channel's sums
@@ -2148,9 +2180,14 @@ struct FoldedArgs {
   int64_t rows;        // whole super-rows
   int64_t rows_per_g;
   FastDiv div_tw, div_ry, div_c;
+  // NCHW units (kUnit): rows are images, tiles units of `fold` channels, div_c
+  // divides by the plane.
+  int64_t plane;
+  int64_t row_bytes;   // one image
+  int own;             // one row group: the workgroup finishes its channels
 };
 
-template <class Tr, bool kGrad, int KR, int KL>
+template <class Tr, bool kGrad, int KR, int KL, bool kUnit = false>
 __global__ __launch_bounds__(kFusedThreads) void bn_folded_nhwc_kernel(FoldedArgs fa) {
   using S = typename Tr::S;
   constexpr int VEC = Tr::kVec;
@@ -2181,17 +2218,21 @@ __global__ __launch_bounds__(kFusedThreads) void bn_folded_nhwc_kernel(FoldedArg
   const int nk_t = static_cast<int>(ty) < fa.ry && ty < rows_g
                        ? static_cast<int>(fa.div_ry.div(rows_g - ty + fa.ry - 1))
                        : 0;
-  const bool active = static_cast<int>(ty) < fa.ry && col < fa.cv;
+  const bool active = static_cast<int>(ty) < fa.ry && (kUnit || col < fa.cv);
   const int nk = active ? nk_t : 0;
   const int nk_w = __builtin_amdgcn_readfirstlane(nk_t);
   const int kl_w = nk_w - KR < 0 ? 0 : (nk_w - KR < KL ? nk_w - KR : KL);
-  const uint32_t row_b = static_cast<uint32_t>(fa.cv) * 16u;
-  const int64_t first = r0 * row_b;  // byte offset of the group's rows
-  const auto rx = rows_rsrc(static_cast<const char*>(a.x) + first, (r1 - r0) * row_b);
-  const auto rd =
-      rows_rsrc(static_cast<const char*>(kGrad ? a.dy : a.x) + first, (r1 - r0) * row_b);
+  const uint32_t row_b =
+      kUnit ? static_cast<uint32_t>(fa.row_bytes) : static_cast<uint32_t>(fa.cv) * 16u;
+  // Byte offset of the group's rows (a unit's: of its segment of them) and
+  // their span.
+  const int64_t first = r0 * row_b + (kUnit ? static_cast<int64_t>(tile) * fa.tw * 16 : 0);
+  const int64_t span = kUnit ? (r1 - r0 - 1) * row_b + fa.tw * 16 : (r1 - r0) * row_b;
+  const auto rx = rows_rsrc(static_cast<const char*>(a.x) + first, span);
+  const auto rd = rows_rsrc(static_cast<const char*>(kGrad ? a.dy : a.x) + first, span);
   char* const obase = static_cast<char*>(a.out) + first;
-  const uint32_t lane_off = active ? ty * row_b + static_cast<uint32_t>(col) * 16u : kOutOfRange;
+  const uint32_t lane_off =
+      active ? ty * row_b + static_cast<uint32_t>(kUnit ? tx : col) * 16u : kOutOfRange;
   const uint32_t rstride_b = static_cast<uint32_t>(fa.ry) * row_b;
   auto roff = [&](int q) { return lane_off + static_cast<uint32_t>(q) * rstride_b; };
   auto lds = [&](int q2, int which) -> uint4& {
@@ -2202,14 +2243,17 @@ __global__ __launch_bounds__(kFusedThreads) void bn_folded_nhwc_kernel(FoldedArg
   const uint32_t col_e = static_cast<uint32_t>(tile * fa.tw) * VEC;  // first column's element
   const uint32_t left = static_cast<uint32_t>(fa.cv) * VEC - col_e;
   const uint32_t nl =
-      single ? C : (left < static_cast<uint32_t>(fa.tw) * VEC ? left : fa.tw * VEC);
+      kUnit ? fa.fold
+            : (single ? C : (left < static_cast<uint32_t>(fa.tw) * VEC ? left : fa.tw * VEC));
   const bool owner = static_cast<uint32_t>(tid) < nl;
   const uint32_t ve = col_e + static_cast<uint32_t>(tid);
-  const uint32_t ch_t = owner ? ve - fa.div_c.div(ve) * C : 0;
+  const uint32_t ch_t =
+      !owner ? 0 : (kUnit ? static_cast<uint32_t>(tile) * nl + tid : ve - fa.div_c.div(ve) * C);
   // Local channel of this thread's element j.
   const uint32_t e0 = active ? tx * VEC : 0;
   const uint32_t l0 = single ? e0 - fa.div_c.div(e0) * C : e0;
   auto local = [&](int j) {
+    if constexpr (kUnit) return fa.div_c.div(e0 + static_cast<uint32_t>(j));
     uint32_t l = l0 + static_cast<uint32_t>(j);
     if (single) {
       while (l >= C) l -= C;  // C may be less than a vector
@@ -2223,12 +2267,15 @@ __global__ __launch_bounds__(kFusedThreads) void bn_folded_nhwc_kernel(FoldedArg
     if (owner) k_own = a.fin.mean_in[ch_t];
   }
   S ks[5];
-  if constexpr (!kGrad) {
+  if constexpr (!kGrad && !kUnit) {
     int64_t js[5];
     shift_rows(a.fin.n, js);
 #pragma unroll
     for (int i = 0; i < 5; ++i) ks[i] = static_cast<const S*>(a.x)[js[i] * C + ch_t];
   }
+  if constexpr (!kGrad && kUnit)
+    k_own = chan_shift_nchw<Tr>(static_cast<const S*>(a.x), ch_t,
+                                static_cast<uint32_t>(a.fin.n), C, fa.div_c);
   uint4 xr[KR];
   uint4 dr[kGrad ? KR : 1];
   uint4 xl[KL];
@@ -2249,7 +2296,7 @@ __global__ __launch_bounds__(kFusedThreads) void bn_folded_nhwc_kernel(FoldedArg
                   : a.epoch;
   const uint64_t etag = static_cast<uint64_t>(epoch) << 32;
   const uint32_t wtag = epoch ^ a.wait_xor;
-  if constexpr (!kGrad) {
+  if constexpr (!kGrad && !kUnit) {
     float v[5];
 #pragma unroll
     for (int i = 0; i < 5; ++i) v[i] = Tr::ld(ks[i]);
@@ -2305,15 +2352,21 @@ __global__ __launch_bounds__(kFusedThreads) void bn_folded_nhwc_kernel(FoldedArg
   // of nl columns - one tile: entry i of the ry passes' columns is channel
   // i mod C, ry * F rows; several: a row per pass - whose rows are dealt to
   // `parts` threads a column, then those added in order.
-  const uint32_t nrows = single ? static_cast<uint32_t>(fa.ry * fa.fold) : fa.ry;
-  const uint32_t pitch = single ? C : static_cast<uint32_t>(fa.tw) * VEC;
-  uint32_t parts = kFusedThreads / nl;
-  parts = parts < 1 ? 1 : (parts > kFoldParts ? kFoldParts : parts);
-  uint32_t part = 0, pl = static_cast<uint32_t>(tid);
-  while (pl >= nl && part < parts) {
-    pl -= nl;
-    ++part;
+  const uint32_t nrows = single && !kUnit ? static_cast<uint32_t>(fa.ry * fa.fold) : fa.ry;
+  const uint32_t pitch = single && !kUnit ? C : static_cast<uint32_t>(fa.tw) * VEC;
+  uint32_t parts, part, pl;
+  if constexpr (kUnit) {  // a power of two of neighbouring lanes per channel
+    parts = 64;
+    while (parts * nl > kFusedThreads) parts >>= 1;
+    part = static_cast<uint32_t>(tid) & (parts - 1);
+    pl = static_cast<uint32_t>(tid) / parts;
+  } else {
+    parts = kFusedThreads / nl;
+    parts = parts < 1 ? 1 : (parts > kFoldParts ? kFoldParts : parts);
+    part = nl > kFusedThreads / 2 ? 0 : static_cast<uint32_t>(tid) / nl;
+    pl = static_cast<uint32_t>(tid) - part * nl;
   }
+  const bool adds = part < parts && pl < nl;
   float sum[2];
 #pragma unroll
   for (int w = 0; w < 2; ++w) {
@@ -2324,35 +2377,67 @@ __global__ __launch_bounds__(kFusedThreads) void bn_folded_nhwc_kernel(FoldedArg
     }
     __syncthreads();
     float t = 0.f;
-    if (part < parts)
-      for (uint32_t r = part; r < nrows; r += parts) t += red[r * pitch + pl];
+    if (adds) {
+      if constexpr (kUnit) {
+        const uint32_t pl0 = pl * static_cast<uint32_t>(fa.plane);
+        for (uint32_t e = part; e < fa.plane; e += parts) {
+#pragma unroll 4
+          for (uint32_t r = 0; r < nrows; ++r) t += red[r * pitch + pl0 + e];
+        }
+      } else {
+#pragma unroll 4
+        for (uint32_t r = part; r < nrows; r += parts) t += red[r * pitch + pl];
+      }
+    }
     sum[w] = t;
+  }
+  if constexpr (kUnit) {
+    for (uint32_t off = parts >> 1; off > 0; off >>= 1) {
+      sum[0] += __shfl_xor(sum[0], off, 64);
+      sum[1] += __shfl_xor(sum[1], off, 64);
+    }
   }
   if (parts > 1) {
     __syncthreads();
-    if (part < parts) {
-      red[2 * tid] = sum[0];
-      red[2 * tid + 1] = sum[1];
+    if (kUnit ? adds && part == 0 : adds) {
+      const uint32_t at = kUnit ? pl : static_cast<uint32_t>(tid);
+      red[2 * at] = sum[0];
+      red[2 * at + 1] = sum[1];
     }
     __syncthreads();
     if (owner) {
-      for (uint32_t p = 1; p < parts; ++p) {
-        sum[0] += red[2 * (p * nl + tid)];
-        sum[1] += red[2 * (p * nl + tid) + 1];
+      sum[0] = red[2 * tid];
+      sum[1] = red[2 * tid + 1];
+      if constexpr (!kUnit) {
+#pragma unroll 4
+        for (uint32_t p = 1; p < parts; ++p) {
+          sum[0] += red[2 * (p * nl + tid)];
+          sum[1] += red[2 * (p * nl + tid) + 1];
+        }
       }
     }
   }
-  if (owner) {
-    if constexpr (!kGrad) {
-      if (g == 0 && ve < C) store_shared(a.ekey + ve, etag | __builtin_bit_cast(uint32_t, k_own));
-    }
-    const int64_t slot = single ? g * C + tid : g * fa.fold * C + ve;
-    store_pair(slots_rsrc(a.eslots, a.groups, a.c), slot, static_cast<uint32_t>(etag >> 32),
-               sum[0], sum[1]);
-  }
-
   // ---- phase 2 ----------------------------------------------------------
-  finish_channel_blocks<Tr, kGrad, true>(a, 0, a.c, wave, lane, wtag, etag, epoch);
+  float4 own_cf = make_float4(0.f, 0.f, 0.f, 0.f);
+  const bool finish_own = kUnit && fa.own != 0;
+  if (finish_own) {
+    if (owner)
+      own_cf = finish_channel<Tr, kGrad>(
+          a.fin, static_cast<int>(ch_t), sum[0], sum[1],
+          fin_inputs<Tr, kGrad>(a.fin, static_cast<int>(ch_t), k_own));
+  } else {
+    if (owner) {
+      if constexpr (!kGrad) {
+        if (g == 0 && (kUnit || ve < C))
+          store_shared(a.ekey + ch_t, etag | __builtin_bit_cast(uint32_t, k_own));
+      }
+      const int64_t slot =
+          kUnit ? g * C + ch_t : (single ? g * C + tid : g * fa.fold * C + ve);
+      store_pair(slots_rsrc(a.eslots, a.groups, a.c), slot, static_cast<uint32_t>(etag >> 32),
+                 sum[0], sum[1]);
+    }
+    finish_channel_blocks<Tr, kGrad, !kUnit>(a, 0, a.c, wave, lane, wtag, etag, epoch);
+  }
   zero_side_outputs<kGrad>(a.fin);
 
   // ---- phase 3 ----------------------------------------------------------
@@ -2364,7 +2449,17 @@ __global__ __launch_bounds__(kFusedThreads) void bn_folded_nhwc_kernel(FoldedArg
   }
   // The local channels' coefficients, one channel per thread, polled until
   // tagged (as tile_coefs); coefficients that never arrive are used as NaN.
-  {
+  if (finish_own) {
+    __syncthreads();
+    if (owner) {
+      float* const c = red + tid + tid / VEC;
+      c[0] = own_cf.x;
+      c[kComp] = own_cf.y;
+      c[2 * kComp] = own_cf.z;
+      c[3 * kComp] = own_cf.w;
+    }
+    __syncthreads();
+  } else {
     const int64_t copy0 = (g % a.coef_copies) * a.coef_copy;
     const auto rc = rows_rsrc(a.ecoef, a.coef_copies * a.coef_copy * 8);
     const int64_t pr =
@@ -2449,14 +2544,19 @@ struct NchwArgs {
   int c;          // channels
   int64_t plane;  // elements per (image, channel) plane
   int64_t pv;     // 16-byte vectors per plane
+  FastDiv div_plane, div_pv;
   FinArgs fin;
 };
 
-// Register rows per thread (the largest spill-free counts; LDS rows as in the
-// NHWC kernel).
-template <class Tr> struct OwnedRows { static constexpr int kFwd = 30, kGrad = 16; };
-template <> struct OwnedRows<TF16> { static constexpr int kFwd = 30, kGrad = 17; };
-template <> struct OwnedRows<TBF16> { static constexpr int kFwd = 31, kGrad = 15; };
+// Rows per thread.  The grad keeps the largest spill-free count of register
+// rows (LDS rows as in the NHWC kernel).  The forward keeps fewer, so that two
+// workgroups share a CU and one reads while the other writes: (12, 8) against
+// (30, 18), f16 [256,512,28,28] 104 -> 97 us, [256,300,28,28], whose 300
+// workgroups were two rounds, 77 -> 64, f32 [64,320,28,28] 31.4 -> 23.9; the
+// grads lose by it (f16 [256,512,28,28] 146 -> 154 us with (8, 4)).
+template <class Tr> struct OwnedRows { static constexpr int kFwd = 12, kFwdLds = 8, kGrad = 16; };
+template <> struct OwnedRows<TF16> { static constexpr int kFwd = 12, kFwdLds = 8, kGrad = 17; };
+template <> struct OwnedRows<TBF16> { static constexpr int kFwd = 11, kFwdLds = 8, kGrad = 14; };
 
 template <class Tr, bool kGrad, int KR, int KL>
 __global__ __launch_bounds__(kFusedThreads) void bn_nchw_owned_kernel(NchwArgs a) {
@@ -2476,10 +2576,10 @@ __global__ __launch_bounds__(kFusedThreads) void bn_nchw_owned_kernel(NchwArgs a
   // img * c * plane * s + v * 16 for channel vector (img, v).  Rows advance
   // by kFusedThreads vectors: dimg images and dv vectors (with carry).
   const uint32_t img_b = static_cast<uint32_t>(a.c * a.plane * static_cast<int64_t>(sizeof(S)));
-  const uint32_t dimg = static_cast<uint32_t>(kFusedThreads / a.pv);
-  const uint32_t dv = static_cast<uint32_t>(kFusedThreads % a.pv);
+  uint32_t dimg, dv, img0, v0;
+  a.div_pv.divmod(kFusedThreads, dimg, dv);
+  a.div_pv.divmod(static_cast<uint32_t>(tid), img0, v0);
   const uint32_t pv = static_cast<uint32_t>(a.pv);
-  uint32_t img0 = static_cast<uint32_t>(tid / a.pv), v0 = static_cast<uint32_t>(tid % a.pv);
   auto step = [&](uint32_t& img, uint32_t& v) {
     v += dv;
     const bool carry = v >= pv;
@@ -2498,8 +2598,9 @@ __global__ __launch_bounds__(kFusedThreads) void bn_nchw_owned_kernel(NchwArgs a
 
   // ---- phase 1: the channel's sums ----------------------------------------
   const float kk = kGrad ? a.fin.mean_in[ch]
-                         : chan_shift<Tr>(static_cast<const S*>(a.x), ch, a.n * a.plane, a.c,
-                                          a.plane);
+                         : chan_shift_nchw<Tr>(static_cast<const S*>(a.x), ch,
+                                               static_cast<uint32_t>(a.n * a.plane), a.c,
+                                               a.div_plane);
   float k[VEC], s1[VEC], s2[VEC];
 #pragma unroll
   for (int j = 0; j < VEC; ++j) {
@@ -2667,6 +2768,366 @@ __global__ __launch_bounds__(kFusedThreads) void bn_nchw_owned_kernel(NchwArgs a
     }
     step(img, v);
   }
+}
+
+// ---------------------------------------------------------------------------
+// 6. NCHW, channels shared between workgroups: every workgroup takes an equal
+//    share of the tensor's vectors in channel-major order (channel, image,
+//    vector of the plane), so it works on at most two channels, A and B, the
+//    last part of one and the first of the next.  It publishes a partial for
+//    each, and finishes both itself from all of their partials - a channel's
+//    are few, and each of its workgroups reading them saves the second
+//    hand-off, coefficients back from one finishing wave.  Coefficients are
+//    uniform, so the registers they take elsewhere hold rows.
+//    kTwo = false: a whole number of workgroups per channel instead, each
+//    within one (half the code: the resident rows' is unrolled).
+//    The grid may be larger than what is resident at once (more channels than
+//    CUs): a workgroup waits only for those of neighbouring ids, which are
+//    dispatched with it (in order, round-robin over the XCDs).
+//    kOdd: planes that are no multiple of a vector.  A plane's last vector
+//    then ends at the plane's end and overlaps the one before; its first
+//    elements are not summed and not stored.  Loads are not aligned there,
+//    which global memory allows.
+//    Bound by HBM; the split kernels read x (and dy) twice, in 2- or 4-byte
+//    accesses for odd planes, in three launches.  Forward / grad, back to
+//    back: f16 [256,64,56,56] 70.1 / 100 -> 44.1 / 59.7 us, f32 [64,96,56,56]
+//    52.5 / 77.4 -> 33.7 / 42.8, f16 [64,512,35,35] 127 / 145 -> 46.1 / 71.7,
+//    bf16 [32,192,28,28] 15.0 / 14.7 -> 8.9 / 9.5.
+// ---------------------------------------------------------------------------
+struct SharedNchwArgs {
+  FusedArgs f;
+  int64_t plane;    // elements per plane
+  uint32_t pv;      // vectors per plane (the last one partial for kOdd)
+  uint32_t nv;      // vectors per channel
+  uint32_t share;   // vectors per workgroup, at most nv
+  uint32_t parts;   // partial slots per channel
+  FastDiv div_pv, div_nv, div_share, div_parts, div_plane;
+};
+
+template <class Tr, bool kGrad, int KR, int KL, bool kOdd, bool kTwo>
+__global__ __launch_bounds__(kFusedThreads) void bn_nchw_shared_kernel(SharedNchwArgs na) {
+  using S = typename Tr::S;
+  constexpr int VEC = Tr::kVec;
+  constexpr int kIn = kGrad ? 2 : 1;
+  constexpr int U = kGrad ? 4 : 8;
+  constexpr int kWaves = kFusedThreads / 64;
+  extern __shared__ uint4 lds_rows[];  // [KL][kIn][kFusedThreads]
+  __shared__ float2 red[2][kWaves];
+  __shared__ float4 cfs[2];
+  const FusedArgs& a = na.f;
+  const int tid = threadIdx.x;
+  const int wave = tid >> 6, lane = tid & 63;
+  // Vectors [a0, a1) of channel ca, then (kTwo) [0, b1) of channel ca + 1.
+  const uint32_t b = blockIdx.x;
+  uint32_t ca, a0, a1, b1 = 0;
+  if constexpr (kTwo) {
+    const uint32_t v0 = b * na.share, total = static_cast<uint32_t>(a.c) * na.nv;
+    const uint32_t v1 = v0 + na.share < total ? v0 + na.share : total;
+    na.div_nv.divmod(v0, ca, a0);
+    const uint32_t a_end = (ca + 1) * na.nv;
+    a1 = v1 < a_end ? a0 + (v1 - v0) : na.nv;
+    b1 = v1 > a_end ? v1 - a_end : 0;
+  } else {
+    uint32_t g;
+    na.div_parts.divmod(b, ca, g);
+    a0 = g * na.share;
+    a1 = a0 + na.share < na.nv ? a0 + na.share : na.nv;
+  }
+  const bool two = kTwo && b1 > 0;
+  const uint32_t cb = two ? ca + 1 : ca;
+  const int qa = static_cast<int>((a1 - a0 + kFusedThreads - 1) / kFusedThreads);  // rows of A
+  const int nq = qa + static_cast<int>((b1 + kFusedThreads - 1) / kFusedThreads);  // all rows
+  const uint32_t plane_b = static_cast<uint32_t>(na.plane * static_cast<int64_t>(sizeof(S)));
+  const uint32_t img_b = static_cast<uint32_t>(a.c) * plane_b;
+  const int64_t bytes = static_cast<int64_t>(na.nv / na.pv) * img_b;
+  const auto rx = rows_rsrc(a.x, bytes);
+  const auto rd = rows_rsrc(kGrad ? a.dy : a.x, bytes);
+  const char* const px = static_cast<const char*>(a.x);
+  const char* const pd = static_cast<const char*>(kGrad ? a.dy : a.x);
+  char* const po = static_cast<char*>(a.out);
+  // Row q of thread t: its byte offset (kOutOfRange: no such row) and, for
+  // kOdd, how many elements of the vector are its own (the last ones).  t is an opaque copy of threadIdx.x made in
+  // each phase: the compiler otherwise keeps the resident rows' offsets from
+  // phase 1 to phase 3, a register each.
+  auto opaque_tid = []() {
+    uint32_t t = threadIdx.x;
+    asm volatile("" : "+v"(t));
+    return t;
+  };
+  uint32_t t = opaque_tid();
+  auto row_of = [&](int q, uint32_t& keep) -> uint32_t {
+    const bool in_a = !kTwo || q < qa;
+    // (Values, not variables, to choose from: a choice between two variables
+    // is one between their addresses, which puts them in scratch memory.)
+    const uint32_t i = (in_a ? a0 + static_cast<uint32_t>(q) * kFusedThreads
+                             : static_cast<uint32_t>(q - qa) * kFusedThreads) +
+                       t;
+    const uint32_t ch = ca + (in_a ? 0u : cb - ca), end = in_a ? +a1 : +b1;
+    uint32_t img, v;
+    na.div_pv.divmod(i, img, v);
+    uint32_t e = v * VEC;
+    keep = VEC;
+    if constexpr (kOdd) {
+      const uint32_t last = static_cast<uint32_t>(na.plane) - VEC;
+      keep = e > last ? VEC - (e - last) : VEC;
+      e = e > last ? last : e;
+    }
+    const uint32_t off = img * img_b + ch * plane_b + e * static_cast<uint32_t>(sizeof(S));
+    return q < nq && i < end ? off : kOutOfRange;
+  };
+  auto load = [&](bool last_use, const __amdgpu_buffer_rsrc_t& r, const char* p, uint32_t off) {
+    if constexpr (kOdd) {
+      // No row: the tensor's first vector, not used.
+      typedef u32x4 __attribute__((aligned(2))) any_u32x4;
+      const any_u32x4* const w =
+          reinterpret_cast<const any_u32x4*>(p + (off == kOutOfRange ? 0u : off));
+      const u32x4 d = last_use ? __builtin_nontemporal_load(w) : *w;
+      return make_uint4(d[0], d[1], d[2], d[3]);
+    } else {
+      return last_use ? bld16_last(r, off) : bld16(r, off);
+    }
+  };
+  auto store = [&](uint32_t off, uint32_t keep, const uint4& w) {
+    if constexpr (kOdd) {
+      typedef u32x4 __attribute__((aligned(2))) any_u32x4;
+      if (keep == VEC) {
+        __builtin_nontemporal_store(u32x4{w.x, w.y, w.z, w.w},
+                                    reinterpret_cast<any_u32x4*>(po + off));
+      } else {
+        S e[VEC];
+        __builtin_memcpy(e, &w, 16);
+#pragma unroll
+        for (int j = 1; j < VEC; ++j)
+          if (j >= VEC - static_cast<int>(keep)) reinterpret_cast<S*>(po + off)[j] = e[j];
+      }
+    } else {
+      st16(po + off, w);
+    }
+  };
+  auto lds = [&](int q2, int which) -> uint4& {
+    return lds_rows[(q2 * kIn + which) * kFusedThreads + tid];
+  };
+
+  // ---- phase 1 ----------------------------------------------------------
+  const S* const xs = static_cast<const S*>(a.x);
+  float ka, kb;
+  if constexpr (kGrad) {
+    ka = a.fin.mean_in[ca];
+    kb = a.fin.mean_in[cb];
+  } else {
+    const uint32_t n = static_cast<uint32_t>(a.fin.n);
+    ka = chan_shift_nchw<Tr>(xs, ca, n, a.c, na.div_plane);
+    kb = two ? chan_shift_nchw<Tr>(xs, cb, n, a.c, na.div_plane) : ka;
+  }
+  uint4 xr[KR];
+  uint4 dr[kGrad ? KR : 1];
+  uint4 xl[KL];
+  uint4 dl[kGrad ? KL : 1];
+#pragma unroll
+  for (int q = 0; q < KR; ++q) {
+    uint32_t keep;
+    const uint32_t o = row_of(q, keep);
+    xr[q] = load(true, rx, px, o);
+    if constexpr (kGrad) dr[q] = load(true, rd, pd, o);
+  }
+#pragma unroll
+  for (int q = 0; q < KL; ++q) {
+    uint32_t keep;
+    const uint32_t o = row_of(KR + q, keep);
+    xl[q] = load(true, rx, px, o);
+    if constexpr (kGrad) dl[q] = load(true, rd, pd, o);
+  }
+  const unsigned epoch =
+      a.epoch_dev ? 0x80000001u + __hip_atomic_load(a.epoch_dev, __ATOMIC_RELAXED,
+                                                    __HIP_MEMORY_SCOPE_AGENT) % 0x7fffffffu
+                  : a.epoch;
+  const uint64_t etag = static_cast<uint64_t>(epoch) << 32;
+  const uint32_t wtag = epoch ^ a.wait_xor;
+  // Sums of the segment in hand; at the first row of B those of A are put
+  // aside.
+  float s1 = 0.f, s2 = 0.f, a1s = 0.f, a2s = 0.f, k = ka;
+  t = opaque_tid();
+  auto accum_row = [&](int q, const uint4& xw, const uint4& dw) {
+    if (kTwo && two && q == qa) {  // uniform
+      a1s = s1;
+      a2s = s2;
+      s1 = s2 = 0.f;
+      k = kb;
+    }
+    uint32_t keep;
+    if (row_of(q, keep) == kOutOfRange) return;
+    S xv[VEC], dv[VEC];
+    __builtin_memcpy(xv, &xw, 16);
+    if constexpr (kGrad) __builtin_memcpy(dv, &dw, 16);
+    // Two chains of additions a sum: one of VEC is long for two waves a SIMD.
+    float t1[2] = {0.f, 0.f}, t2[2] = {0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) {
+      const float xc = Tr::ld(xv[j]) - k;
+      float f = kGrad ? Tr::ld(dv[j]) : xc;
+      float p = f * xc;
+      if constexpr (kOdd) {
+        const bool own = j >= VEC - static_cast<int>(keep);
+        f = own ? f : 0.f;
+        p = own ? p : 0.f;
+      }
+      t1[j & 1] += f;
+      t2[j & 1] += p;
+    }
+    s1 += t1[0] + t1[1];
+    s2 += t2[0] + t2[1];
+  };
+#pragma unroll
+  for (int q = 0; q < KR; ++q) {
+    accum_row(q, xr[q], dr[kGrad ? q : 0]);
+    asm volatile("" : "+v"(xr[q].x), "+v"(xr[q].y), "+v"(xr[q].z), "+v"(xr[q].w));
+    if constexpr (kGrad)
+      asm volatile("" : "+v"(dr[q].x), "+v"(dr[q].y), "+v"(dr[q].z), "+v"(dr[q].w));
+  }
+  const int kl_w = nq - KR < 0 ? 0 : (nq - KR < KL ? nq - KR : KL);
+#pragma unroll
+  for (int q = 0; q < KL; ++q) {
+    if (q < kl_w) {
+      lds(q, 0) = xl[q];
+      if constexpr (kGrad) lds(q, kGrad ? 1 : 0) = dl[kGrad ? q : 0];
+    }
+  }
+#pragma unroll 2
+  for (int q = 0; q < kl_w; ++q) {
+    const uint4 xw = lds(q, 0);
+    const uint4 dw = kGrad ? lds(q, kGrad ? 1 : 0) : xw;
+    accum_row(KR + q, xw, dw);
+  }
+#pragma unroll 1
+  for (int q = KR + KL; q < nq; q += U) {
+    uint4 xw[U], dw[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      uint32_t keep;
+      const uint32_t o = row_of(q + u, keep);
+      xw[u] = load(false, rx, px, o);
+      if constexpr (kGrad) dw[u] = load(false, rd, pd, o);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) accum_row(q + u, xw[u], dw[kGrad ? u : 0]);
+  }
+  if (!two) {  // the rows were all A's
+    a1s = s1;
+    a2s = s2;
+    s1 = s2 = 0.f;
+  }
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) {
+    a1s += __shfl_xor(a1s, off, 64);
+    a2s += __shfl_xor(a2s, off, 64);
+    s1 += __shfl_xor(s1, off, 64);
+    s2 += __shfl_xor(s2, off, 64);
+  }
+  if (lane == 0) {
+    red[0][wave] = make_float2(a1s, a2s);
+    red[1][wave] = make_float2(s1, s2);
+  }
+  __syncthreads();
+
+  // ---- phase 2: wave 0 publishes and finishes A, wave 1 B ----------------
+  if (wave < (two ? 2 : 1)) {
+    const uint32_t ch = wave == 0 ? ca : cb;
+    // The channel's workgroups: those of its first and its last vector.
+    const uint32_t w0 = kTwo ? na.div_share.div(ch * na.nv) : ca * na.parts;
+    const uint32_t w1 =
+        kTwo ? na.div_share.div(ch * na.nv + na.nv - 1) : w0 + na.parts - 1;
+    const uint32_t cnt = w1 - w0 + 1;
+    const auto rs = rows_rsrc(a.eslots, static_cast<int64_t>(a.c) * na.parts * 16);
+    if (lane == 0) {
+      float2 sum = red[wave][0];
+#pragma unroll
+      for (int i = 1; i < kWaves; ++i) {
+        sum.x += red[wave][i].x;
+        sum.y += red[wave][i].y;
+      }
+      store_pair(rs, static_cast<int64_t>(ch) * na.parts + (b - w0),
+                 static_cast<uint32_t>(etag >> 32), sum.x, sum.y);
+    }
+    const FinIn fin_in = fin_inputs<Tr, kGrad>(a.fin, static_cast<int>(ch), wave == 0 ? ka : kb);
+    double t1 = 0.0, t2 = 0.0;
+    for (uint32_t p0 = 0; p0 < cnt; p0 += 64) {
+      const uint32_t p = p0 + static_cast<uint32_t>(lane);
+      const bool has = p < cnt;
+      const int64_t slot =
+          has ? static_cast<int64_t>(ch) * na.parts + p : int64_t(kOutOfRange / 16);
+      u32x4 v = load_pair(rs, slot);
+      unsigned spins = 0;
+      while (has && !pair_tagged(v, wtag)) {
+        if (++spins > a.spin_limit) {
+          v = u32x4{0x7fc00000u, wtag, 0x7fc00000u, wtag};
+          __hip_atomic_store(a.gave_up, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+          break;
+        }
+        __builtin_amdgcn_s_sleep(1);
+        asm volatile("" ::: "memory");  // the reload is not the load above
+        v = load_pair(rs, slot);
+      }
+      if (has) {
+        t1 += bits_f32(v[0]);
+        t2 += bits_f32(v[2]);
+      }
+    }
+    const double2 w = wave_sum(t1, t2);
+    if (lane == 0)
+      cfs[wave] = finish_channel<Tr, kGrad>(a.fin, static_cast<int>(ch), w.x, w.y, fin_in,
+                                            b == w0);
+  }
+  zero_side_outputs<kGrad>(a.fin);
+
+  // ---- phase 3 ----------------------------------------------------------
+#pragma unroll
+  for (int r = 0; r < KR; ++r) {
+    asm volatile("" : "+v"(xr[r].x), "+v"(xr[r].y), "+v"(xr[r].z), "+v"(xr[r].w));
+    if constexpr (kGrad)
+      asm volatile("" : "+v"(dr[r].x), "+v"(dr[r].y), "+v"(dr[r].z), "+v"(dr[r].w));
+  }
+  __syncthreads();
+  const float4 fa = cfs[0], fb = cfs[two ? 1 : 0];
+  t = opaque_tid();
+  auto apply_row = [&](int q, uint32_t off, uint32_t keep, const uint4& xw, const uint4& dw) {
+    const bool in_a = !kTwo || q < qa;
+    const float4 cone = make_float4(in_a ? +fa.x : +fb.x, in_a ? +fa.y : +fb.y,
+                                    in_a ? +fa.z : +fb.z, in_a ? +fa.w : +fb.w);
+    float4 cf[VEC];
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) cf[j] = cone;
+    const uint4 o = apply_words<Tr, kGrad>(xw, dw, cf);
+    if (off != kOutOfRange) store(off, keep, o);
+  };
+#pragma unroll 1
+  for (int q = nq - 1; q >= KR + KL; q -= U) {
+    uint4 xw[U], dw[U];
+    uint32_t o[U], keep[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t at = row_of(q - u, keep[u]);
+      o[u] = q - u >= KR + KL ? at : kOutOfRange;
+      xw[u] = load(true, rx, px, o[u]);
+      if constexpr (kGrad) dw[u] = load(true, rd, pd, o[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) apply_row(q - u, o[u], keep[u], xw[u], dw[kGrad ? u : 0]);
+  }
+#pragma unroll
+  for (int r = 0; r < KR; ++r) {
+    uint32_t keep;
+    const uint32_t off = row_of(r, keep);
+    if (r < nq) apply_row(r, off, keep, xr[r], dr[kGrad ? r : 0]);
+  }
+#pragma unroll 2
+  for (int q2 = 0; q2 < kl_w; ++q2) {
+    uint32_t keep;
+    const uint32_t off = row_of(KR + q2, keep);
+    const uint4 xw = lds(q2, 0);
+    const uint4 dw = kGrad ? lds(q2, kGrad ? 1 : 0) : xw;
+    apply_row(KR + q2, off, keep, xw, dw);
+  }
+  recorded_exit(a, epoch);
 }
 
 // ---------------------------------------------------------------------------
@@ -2872,6 +3333,12 @@ struct FusedPlan {
   int fold = 1;
   int tw = 0;
   int64_t row_groups = 0;
+  // NCHW shared (share > 0): vectors per workgroup; groups is the number of
+  // partial slots per channel.
+  int64_t share = 0;
+  int64_t pv = 0;
+  bool two = false;
+  int unit = 0;  // NCHW units: channels of one (folded kernel, kUnit)
 };
 
 // Channels of the largest fused plan (at most 2 workgroups per CU, tiles of
@@ -2931,19 +3398,20 @@ constexpr int folded_kr() { return kGrad ? FoldedRows<Tr>::kGrad : FoldedRows<Tr
 template <class Tr, bool kGrad>
 constexpr int folded_kl() { return kGrad ? 8 : 16; }
 
-template <class Tr, bool kGrad, int KR = folded_kr<Tr, kGrad>(), int KL = folded_kl<Tr, kGrad>()>
+template <class Tr, bool kGrad, bool kUnit, int KR, int KL>
 const void* folded_kernel() {
-  return reinterpret_cast<const void*>(&bn_folded_nhwc_kernel<Tr, kGrad, KR, KL>);
+  return reinterpret_cast<const void*>(&bn_folded_nhwc_kernel<Tr, kGrad, KR, KL, kUnit>);
 }
-template <class Tr, bool kGrad>
+template <class Tr, bool kGrad, bool kUnit>
 FusedPick pick_folded(int64_t nk) {
   constexpr FewRows f1 = kGrad ? kFew1Grad : kFew1Fwd;
-  if (nk <= f1.most) return {folded_kernel<Tr, kGrad, f1.kr, f1.kl>(), f1.kr, f1.kl};
+  constexpr int kr = folded_kr<Tr, kGrad>(), kl = folded_kl<Tr, kGrad>();
+  if (nk <= f1.most) return {folded_kernel<Tr, kGrad, kUnit, f1.kr, f1.kl>(), f1.kr, f1.kl};
   if constexpr (!kGrad) {
     constexpr FewRows f2 = kFew2Fwd;
-    if (nk <= f2.most) return {folded_kernel<Tr, kGrad, f2.kr, f2.kl>(), f2.kr, f2.kl};
+    if (nk <= f2.most) return {folded_kernel<Tr, kGrad, kUnit, f2.kr, f2.kl>(), f2.kr, f2.kl};
   }
-  return {folded_kernel<Tr, kGrad>(), folded_kr<Tr, kGrad>(), folded_kl<Tr, kGrad>()};
+  return {folded_kernel<Tr, kGrad, kUnit, kr, kl>(), kr, kl};
 }
 template <class Tr, bool kGrad>
 size_t folded_smem() {
@@ -2961,14 +3429,16 @@ int folded_blocks_per_cu() {
   if (known != 0) return known;
   int count = 1;
   for (int64_t nk : {int64_t(1), kFew2Fwd.most, kFew2Fwd.most + 1}) {
-    const void* const k = pick_folded<Tr, kGrad>(nk).kernel;
-    int nb = 0;
-    hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       static_cast<int>(folded_smem<Tr, kGrad>()));
-    if (e == hipSuccess)
-      e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k, kFusedThreads,
-                                                       folded_smem<Tr, kGrad>());
-    if (e != hipSuccess || nb < 1) count = -1;
+    for (const void* k : {pick_folded<Tr, kGrad, false>(nk).kernel,
+                          pick_folded<Tr, kGrad, true>(nk).kernel}) {
+      int nb = 0;
+      hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                         static_cast<int>(folded_smem<Tr, kGrad>()));
+      if (e == hipSuccess)
+        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k, kFusedThreads,
+                                                         folded_smem<Tr, kGrad>());
+      if (e != hipSuccess || nb < 1) count = -1;
+    }
   }
   cached[dev].store(count, std::memory_order_release);
   return count;
@@ -3039,6 +3509,148 @@ bool make_folded_plan(const BnGeometry& g, int vec, int blocks_per_cu, FusedPlan
   fp->fold = F;
   fp->tw = static_cast<int>(tw);
   fp->row_groups = groups;
+  return true;
+}
+
+// The unit plan (16-byte aligned pointers): planes that are no multiple of a
+// vector, whole units of channels, and units of at most one pass of a
+// workgroup.
+bool make_unit_plan(const BnGeometry& g, int vec, int blocks_per_cu, FusedPlan* fp) {
+  const int64_t plane = g.h * g.w;
+  const int64_t esz = 16 / vec;
+  if (g.nhwc || blocks_per_cu < 1 || plane % vec == 0 || g.n < 1 ||
+      TuneValue(kTuneBnNchwOwned) == 0)
+    return false;
+  int gcd = vec;
+  while (plane % gcd != 0) gcd >>= 1;
+  const int u = vec / gcd;
+  const int64_t tw = u * plane / vec;
+  if (g.c % u != 0 || tw > kFusedThreads) return false;
+  const int64_t units = g.c / u;
+  const int64_t ry = kFusedThreads / tw;
+  const int64_t row_b = g.c * plane * esz;
+  int64_t groups = std::max<int64_t>(1, static_cast<int64_t>(DeviceCUs()) / units);
+  groups = std::min(groups, std::max<int64_t>(1, g.n / (2 * ry)));
+  const int64_t rpg = (g.n + groups - 1) / groups;
+  groups = (g.n + rpg - 1) / rpg;
+  if ((rpg + 64 * ry) * row_b >= (int64_t{1} << 31) || groups > kMaxEpochGroups ||
+      groups * g.c > 512 * static_cast<int64_t>(DeviceCUs()) || g.c > max_fused_channels() ||
+      units * groups >= (int64_t{1} << 30))
+    return false;
+  *fp = FusedPlan{};
+  fp->tx_shift = 0;
+  fp->ct = fp->ct_conc = static_cast<int>(units);
+  fp->cv = units * tw;
+  fp->groups = fp->row_groups = groups;
+  fp->rows_per_g = rpg;
+  fp->blocks = static_cast<int>(groups * units);
+  fp->dyn_rows = 0;
+  fp->dyn_chunk = 1;
+  fp->fold = 1;
+  fp->tw = static_cast<int>(tw);
+  fp->unit = u;
+  return true;
+}
+
+// Register rows per thread of the shared NCHW kernels (the largest spill-free
+// counts); ops with few rows per thread run the FewRows counts.
+template <class Tr, bool kGrad, bool kOdd>
+constexpr int shared_kr() {
+  constexpr bool half = std::is_same<Tr, TF16>::value, bf = std::is_same<Tr, TBF16>::value;
+  return kGrad ? (kOdd ? 14 : (half ? 17 : (bf ? 16 : 15))) : (kOdd ? 26 : (half ? 32 : 29));
+}
+
+template <class Tr, bool kGrad, bool kOdd, bool kTwo>
+FusedPick pick_shared(int64_t nk) {
+  constexpr FewRows f1 = kGrad ? kFew1Grad : kFew1Fwd;
+  constexpr FewRows f2 = kFew2Fwd;
+  constexpr int kr = shared_kr<Tr, kGrad, kOdd>(), kl = fused_kl<Tr, kGrad>();
+  if (nk <= f1.most)
+    return {reinterpret_cast<const void*>(&bn_nchw_shared_kernel<Tr, kGrad, f1.kr, f1.kl, kOdd, kTwo>),
+            f1.kr, f1.kl};
+  if constexpr (!kGrad) {
+    if (nk <= f2.most)
+      return {
+          reinterpret_cast<const void*>(&bn_nchw_shared_kernel<Tr, kGrad, f2.kr, f2.kl, kOdd, kTwo>),
+          f2.kr, f2.kl};
+  }
+  return {reinterpret_cast<const void*>(&bn_nchw_shared_kernel<Tr, kGrad, kr, kl, kOdd, kTwo>), kr, kl};
+}
+
+// Whether one workgroup of every shared NCHW kernel fits a CU (-1: no), once
+// per device.
+template <class Tr, bool kGrad>
+int shared_blocks_per_cu() {
+  static std::atomic<int> cached[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
+  const int known = cached[dev].load(std::memory_order_acquire);
+  if (known != 0) return known;
+  int count = 1;
+  for (int64_t nk : {int64_t(1), kFew2Fwd.most, kFew2Fwd.most + 1}) {
+    for (const void* k : {pick_shared<Tr, kGrad, false, false>(nk).kernel,
+                          pick_shared<Tr, kGrad, false, true>(nk).kernel,
+                          pick_shared<Tr, kGrad, true, false>(nk).kernel,
+                          pick_shared<Tr, kGrad, true, true>(nk).kernel}) {
+      int nb = 0;
+      hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                         static_cast<int>(fused_smem<Tr, kGrad>()));
+      if (e == hipSuccess)
+        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k, kFusedThreads,
+                                                         fused_smem<Tr, kGrad>());
+      if (e != hipSuccess || nb < 1) count = -1;
+    }
+  }
+  cached[dev].store(count, std::memory_order_release);
+  return count;
+}
+
+// The shared NCHW plan (16-byte aligned pointers, planes of at least a
+// vector): equal shares for as many workgroups as CUs, or a whole multiple
+// where there are more channels, so that no share exceeds a channel.  The
+// kernel's offsets are 32-bit over the whole tensor.
+bool make_shared_plan(const BnGeometry& g, int vec, int blocks_per_cu, FusedPlan* fp) {
+  const int64_t plane = g.h * g.w;
+  const int64_t esz = 16 / vec;
+  // Planes of a line or two are read in pieces of a line by different
+  // workgroups: with many channels the split kernels are as fast (f16
+  // [64,777,9,9] 23.9 / 22.0 us against 23.7 / 24.5).
+  if (g.c > DeviceCUs() && plane * esz < 192) return false;
+  if (g.nhwc || blocks_per_cu < 1 || plane < vec || g.n < 1 ||
+      TuneValue(kTuneBnNchwOwned) == 0 || (g.n + 16) * g.c * plane * esz >= (int64_t{1} << 31))
+    return false;
+  const int64_t cus = DeviceCUs();
+  const int64_t pv = (plane + vec - 1) / vec;
+  const int64_t nv = g.n * pv;
+  const int64_t wgs = (g.c + cus - 1) / cus * cus;
+  const int64_t least = 2 * kFusedThreads;  // two rows per thread, where a channel has them
+  // A whole number of workgroups per channel where that leaves at most an
+  // eighth of the CUs idle or the channels are short.
+  const int64_t whole = std::max<int64_t>(1, std::min(wgs / g.c, (nv + least - 1) / least));
+  const bool two = whole * g.c * 8 < wgs * 7 && whole == wgs / g.c;
+  int64_t share, blocks, parts;
+  if (two) {
+    share = std::min(nv, std::max((g.c * nv + wgs - 1) / wgs, least));
+    blocks = (g.c * nv + share - 1) / share;
+    parts = (nv + share - 1) / share + 1;
+  } else {
+    share = (nv + whole - 1) / whole;
+    parts = (nv + share - 1) / share;
+    blocks = parts * g.c;
+  }
+  if (blocks > wgs || parts > 255 || parts * g.c > 512 * cus) return false;
+  *fp = FusedPlan{};
+  fp->tx_shift = 0;
+  fp->ct = fp->ct_conc = 1;
+  fp->cv = pv;
+  fp->groups = parts;
+  fp->rows_per_g = share;
+  fp->blocks = static_cast<int>(blocks);
+  fp->dyn_rows = 0;
+  fp->dyn_chunk = 1;
+  fp->share = share;
+  fp->pv = pv;
+  fp->two = two;
   return true;
 }
 
@@ -3356,9 +3968,10 @@ hipError_t launch_fused(const FusedPlan& fp, const BnGeometry& g, const void* x,
   fa.epoch_dev = recorded ? reinterpret_cast<unsigned*>(reinterpret_cast<char*>(region) +
                                                         kEpochOffset)
                           : nullptr;
-  const bool folded = fp.tw > 0;
+  const bool folded = fp.tw > 0, shared = fp.share > 0;
   const int ry = folded ? kFusedThreads / fp.tw : kFusedThreads >> fp.tx_shift;
-  const int64_t nk_max = (fp.rows_per_g + ry - 1) / ry;  // rows of a thread
+  // Rows of a thread (two channels: the second's start anew).
+  const int64_t nk_max = (fp.rows_per_g + ry - 1) / ry + (fp.two ? 1 : 0);
   const bool sliced = kGrad && fp.slices > 1;
   FusedPick pick = pick_fused<Tr, kGrad>(nk_max);
   if constexpr (kGrad) {
@@ -3376,12 +3989,12 @@ hipError_t launch_fused(const FusedPlan& fp, const BnGeometry& g, const void* x,
     size_t shards = slots / per_shard;
     if (shards > 16) shards = 16;
     fa.shards = shards > 0 ? static_cast<int>(shards) : 1;
-    fa.dyn_rows = shards > 0 && !folded ? fd.dyn_rows : 0;
+    fa.dyn_rows = shards > 0 && !folded && !shared ? fd.dyn_rows : 0;
   }
   fa.tail = 0;
   fa.tail_row = 0;
   if (folded) {
-    fa.tail = static_cast<int>(g.rows % fp.fold);
+    fa.tail = static_cast<int>(g.rows % fp.fold);  // 0 for units
     fa.tail_row = g.rows - fa.tail;
     fa.coef_copies = static_cast<int>(std::min<int64_t>(
         kCoefCopies, std::max<int64_t>(1, fp.row_groups / kPollersPerCopy)));
@@ -3397,6 +4010,7 @@ hipError_t launch_fused(const FusedPlan& fp, const BnGeometry& g, const void* x,
   t_last_plan.dynamic_chunk = fa.dyn_chunk;
   t_last_plan.slices = fp.slices;
   const char* name = kGrad ? "tfma_bn_grad_fused" : "tfma_bn_fwd_fused";
+  if (shared) name = kGrad ? "tfma_bn_grad_nchw_shared" : "tfma_bn_fwd_nchw_shared";
   SetLastKernel(name);
   if constexpr (kGrad) {
     // No dynamic tail: the kernel that hides the slices' hand-offs.
@@ -3409,20 +4023,48 @@ hipError_t launch_fused(const FusedPlan& fp, const BnGeometry& g, const void* x,
   void* kargs[] = {&fa};
   FoldedArgs fo;
   if (folded) {
-    pick = pick_folded<Tr, kGrad>(nk_max);
+    pick = fp.unit > 0 ? pick_folded<Tr, kGrad, true>(nk_max)
+                       : pick_folded<Tr, kGrad, false>(nk_max);
     smem = folded_smem<Tr, kGrad>();
+    // Workgroups that wait for none may share a CU.
+    if (fp.unit > 0 && fp.groups == 1)
+      smem = static_cast<size_t>(pick.kl) * (kGrad ? 2 : 1) * kFusedThreads * 16;
     fo.f = fa;
-    fo.fold = fp.fold;
+    fo.fold = fp.unit > 0 ? fp.unit : fp.fold;
     fo.cv = static_cast<int>(fp.cv);
     fo.tw = fp.tw;
     fo.tiles = fp.ct;
     fo.ry = ry;
-    fo.rows = g.rows / fp.fold;
+    fo.rows = fp.unit > 0 ? g.n : g.rows / fp.fold;
     fo.rows_per_g = fp.rows_per_g;
+    fo.plane = g.h * g.w;
+    fo.row_bytes = g.c * g.h * g.w * static_cast<int64_t>(sizeof(typename Tr::S));
+    fo.own = fp.unit > 0 && fp.groups == 1;
     fo.div_tw = FastDiv(static_cast<uint32_t>(fp.tw));
     fo.div_ry = FastDiv(static_cast<uint32_t>(ry));
-    fo.div_c = FastDiv(static_cast<uint32_t>(g.c));
+    fo.div_c = FastDiv(static_cast<uint32_t>(fp.unit > 0 ? fo.plane : g.c));
     kargs[0] = &fo;
+  }
+  SharedNchwArgs sn;
+  if (shared) {
+    const int64_t plane = g.h * g.w;
+    const bool odd = plane % Tr::kVec != 0;
+    pick = fp.two ? (odd ? pick_shared<Tr, kGrad, true, true>(nk_max)
+                         : pick_shared<Tr, kGrad, false, true>(nk_max))
+                  : (odd ? pick_shared<Tr, kGrad, true, false>(nk_max)
+                         : pick_shared<Tr, kGrad, false, false>(nk_max));
+    sn.f = fa;
+    sn.plane = plane;
+    sn.pv = static_cast<uint32_t>(fp.pv);
+    sn.nv = static_cast<uint32_t>(g.n * fp.pv);
+    sn.share = static_cast<uint32_t>(fp.share);
+    sn.parts = static_cast<uint32_t>(fp.groups);
+    sn.div_pv = FastDiv(sn.pv);
+    sn.div_nv = FastDiv(sn.nv);
+    sn.div_share = FastDiv(sn.share);
+    sn.div_parts = FastDiv(sn.parts);
+    sn.div_plane = FastDiv(static_cast<uint32_t>(plane));
+    kargs[0] = &sn;
   }
   t_last_plan.register_rows = pick.kr;
   t_last_plan.lds_rows = pick.kl;
@@ -3523,20 +4165,45 @@ bool nchw_owned_ok(const BnGeometry& g, int vec, int elem) {
   return plane % vec == 0 && (g.n + 16) * g.c * plane * elem < (int64_t{1} << 31);
 }
 
+struct OwnedPick {
+  void (*kernel)(NchwArgs);
+  int kr, kl;
+};
+// Only the last one needs more LDS than a launch gets by default.
+template <class Tr, bool kGrad>
+OwnedPick pick_owned(int64_t nk) {
+  if constexpr (kGrad) {
+    constexpr FewRows f1 = kFew1Grad;
+    constexpr int kr = OwnedRows<Tr>::kGrad, kl = fused_kl<Tr, true>();
+    if (nk <= f1.most) return {&bn_nchw_owned_kernel<Tr, true, f1.kr, f1.kl>, f1.kr, f1.kl};
+    return {&bn_nchw_owned_kernel<Tr, true, kr, kl>, kr, kl};
+  } else {
+    constexpr FewRows f1 = kFew1Fwd, f2 = kFew2Fwd;
+    constexpr int kr = OwnedRows<Tr>::kFwd, kl = OwnedRows<Tr>::kFwdLds;
+    if (nk <= f1.most) return {&bn_nchw_owned_kernel<Tr, false, f1.kr, f1.kl>, f1.kr, f1.kl};
+    if (nk <= f2.most / 2) return {&bn_nchw_owned_kernel<Tr, false, f2.kr, f2.kl>, f2.kr, f2.kl};
+    return {&bn_nchw_owned_kernel<Tr, false, kr, kl>, kr, kl};
+  }
+}
+
 template <class Tr, bool kGrad>
 hipError_t launch_nchw_owned(const BnGeometry& g, const void* x, const void* dy, void* out,
                              const FinArgs& fin, hipStream_t stream) {
-  constexpr int KR = kGrad ? OwnedRows<Tr>::kGrad : OwnedRows<Tr>::kFwd;
-  constexpr int KL = fused_kl<Tr, kGrad>();
-  const auto kern = &bn_nchw_owned_kernel<Tr, kGrad, KR, KL>;
-  const size_t smem = static_cast<size_t>(KL) * (kGrad ? 2 : 1) * kFusedThreads * 16;
+  // Few rows per thread: kernels of few resident rows, and several workgroups
+  // per CU (no workgroup waits for another, so any number may be in flight).
+  // Forward / grad: f32 [32,1024,14,14] 38.2 / 31.6 -> 13.6 / 16.2 us, f16
+  // [32,512,28,28] 24.3 / 24.4 -> 11.4 / 15.1, f32 [8,2048,14,14] 71.8 / 56.2
+  // -> 16.5 / 17.9.
+  const int64_t nv = g.n * (g.h * g.w / Tr::kVec);
+  const OwnedPick p = pick_owned<Tr, kGrad>((nv + kFusedThreads - 1) / kFusedThreads);
+  const size_t smem = static_cast<size_t>(p.kl) * (kGrad ? 2 : 1) * kFusedThreads * 16;
   static std::atomic<bool> attr_set[64];
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return e;
   if (dev < 0 || dev >= 64) return hipErrorInvalidDevice;
-  if (!attr_set[dev].load(std::memory_order_acquire)) {
-    e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+  if (smem > 65536 && !attr_set[dev].load(std::memory_order_acquire)) {
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(p.kernel),
                             hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(smem));
     if (e != hipSuccess) return e;
     attr_set[dev].store(true, std::memory_order_release);
@@ -3549,16 +4216,18 @@ hipError_t launch_nchw_owned(const BnGeometry& g, const void* x, const void* dy,
   na.c = static_cast<int>(g.c);
   na.plane = g.h * g.w;
   na.pv = na.plane / Tr::kVec;
+  na.div_plane = FastDiv(static_cast<uint32_t>(na.plane));
+  na.div_pv = FastDiv(static_cast<uint32_t>(na.pv));
   na.fin = fin;
   t_last_plan = TFMA_FusedBatchNormPlan{};
   t_last_plan.fused = 2;
   t_last_plan.workgroups = static_cast<int32_t>(g.c);
   t_last_plan.row_groups = 1;
   t_last_plan.channel_tiles = static_cast<int32_t>(g.c);
-  t_last_plan.register_rows = KR;
-  t_last_plan.lds_rows = KL;
+  t_last_plan.register_rows = p.kr;
+  t_last_plan.lds_rows = p.kl;
   t_last_plan.slices = 1;
-  TFMA_LAUNCH(kGrad ? "tfma_bn_grad_nchw_owned" : "tfma_bn_fwd_nchw_owned", kern,
+  TFMA_LAUNCH(kGrad ? "tfma_bn_grad_nchw_owned" : "tfma_bn_fwd_nchw_owned", p.kernel,
               dim3(static_cast<unsigned>(g.c)), dim3(kFusedThreads), smem, stream, na);
   return hipGetLastError();
 }
@@ -3607,6 +4276,12 @@ hipError_t forward_t(const BnGeometry& g, const BnFwdArgs& a, void* ws,
     return launch_fused<Tr, false>(fp, g, a.x, nullptr, a.y, fa,
                                                   stream);
   }
+  if (a.is_training && aligned && fused_enabled() &&
+      make_unit_plan(g, Tr::kVec, folded_blocks_per_cu<Tr, false>(), &fp))
+    return launch_fused<Tr, false>(fp, g, a.x, nullptr, a.y, fa, stream);
+  if (a.is_training && aligned && fused_enabled() &&
+      make_shared_plan(g, Tr::kVec, shared_blocks_per_cu<Tr, false>(), &fp))
+    return launch_fused<Tr, false>(fp, g, a.x, nullptr, a.y, fa, stream);
   if (a.is_training && aligned && fused_enabled() &&
       make_folded_plan(g, Tr::kVec, folded_blocks_per_cu<Tr, false>(), &fp))
     return launch_fused<Tr, false>(fp, g, a.x, nullptr, a.y, fa, stream);
@@ -3661,6 +4336,12 @@ hipError_t grad_t(const BnGeometry& g, const BnGradArgs& a, void* ws,
     return launch_fused<Tr, true>(fp, g, a.x, a.dy, a.dx, fa,
                                                   stream);
   }
+  if (aligned && fused_enabled() &&
+      make_unit_plan(g, Tr::kVec, folded_blocks_per_cu<Tr, true>(), &fp))
+    return launch_fused<Tr, true>(fp, g, a.x, a.dy, a.dx, fa, stream);
+  if (aligned && fused_enabled() &&
+      make_shared_plan(g, Tr::kVec, shared_blocks_per_cu<Tr, true>(), &fp))
+    return launch_fused<Tr, true>(fp, g, a.x, a.dy, a.dx, fa, stream);
   if (aligned && fused_enabled() &&
       make_folded_plan(g, Tr::kVec, folded_blocks_per_cu<Tr, true>(), &fp))
     return launch_fused<Tr, true>(fp, g, a.x, a.dy, a.dx, fa, stream);

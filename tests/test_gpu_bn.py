@@ -833,3 +833,65 @@ def test_few_rows_kernels_match_oracle(dev, rows):
                            ("offset_backprop", grad.offset_backprop, rob)):
         err = np.abs(got.cpu().numpy().astype(np.float64) - ref).max()
         assert err <= STAT_TOL * max(np.abs(ref).max(), np.sqrt(rows)), name
+
+
+# NCHW: channels shared by a whole number of workgroups and by any number (two
+# channels in a workgroup), whole and partial last vectors of a plane, planes
+# of one vector, more channels than CUs; units of channels (planes that are no
+# multiple of a vector), with one row group and several; channels that are no
+# whole unit; all rows on chip and streamed ones.
+NCHW_CASES = [
+    ((5, 3, 4, 8), "float16"),
+    ((3, 1, 8, 8), "float32"),
+    ((64, 64, 28, 28), "float16"),
+    ((17, 96, 28, 28), "bfloat16"),    # 2.67 workgroups per channel
+    ((9, 200, 8, 9), "float32"),
+    ((16, 100, 5, 5), "float16"),      # 25 elements, no whole unit of 8
+    ((4, 99, 35, 35), "float32"),
+    ((3, 301, 13, 15), "bfloat16"),    # more channels than CUs, odd planes
+    ((16, 64, 112, 112), "float16"),   # streamed rows
+    ((8, 48, 99, 99), "bfloat16"),     # the same, odd planes
+    ((2, 8, 7, 7), "float16"),         # one unit
+    ((33, 512, 7, 7), "float16"),
+    ((40, 2048, 7, 7), "bfloat16"),    # one row group
+    ((64, 256, 14, 14), "float16"),
+    ((7, 36, 21, 21), "float32"),
+    ((256, 64, 21, 21), "float16"),    # 441 vectors of 512: streamed rows
+    ((6, 512, 14, 14), "float32"),     # a workgroup per channel, few rows
+    ((40, 256, 28, 28), "float16"),
+    ((90, 260, 28, 28), "bfloat16"),
+]
+
+
+@pytest.mark.parametrize("shape,dtype", NCHW_CASES)
+def test_nchw_matches_oracle(dev, shape, dtype):
+    rng = np.random.default_rng(zlib.crc32(repr((shape, dtype, "nchw")).encode()))
+    eps = 1e-3
+    x, scale, offset, _ = _inputs(rng, shape, dtype, "NCHW", loc=0.5)
+    dy = gen(rng, shape, dtype, loc=0.25)
+    c = shape[1]
+    mean = (0.1 * rng.standard_normal(c)).astype(np.float32)
+    var = rng.uniform(0.5, 2.0, c).astype(np.float32)
+    fwd, grad = _run_fwd_grad(dev, x, scale, offset, dy, dtype, "NCHW", eps, mean=mean, var=var,
+                              factor=0.75)
+    assert ops.fused_batch_norm_last_plan()["fused"] != 0
+    ry, rbm, rbv, rsm, rsv = oracle.bn_fwd(x, scale, offset, mean, var, epsilon=eps,
+                                          exponential_avg_factor=0.75, data_format="NCHW",
+                                          dtype=dtype)
+    assert_close(to_np(fwd.y, dtype), ry, dtype, ACT_TOL[dtype], "y")
+    for name, got, ref in (("batch_mean", fwd.batch_mean, rbm),
+                           ("batch_variance", fwd.batch_variance, rbv),
+                           ("reserve_space_1", fwd.reserve_space_1, rsm),
+                           ("reserve_space_2", fwd.reserve_space_2, rsv)):
+        assert_close(got.cpu().numpy(), ref, "float32", STAT_TOL, name)
+    rdx, rsb, rob = oracle.bn_grad(dy, x, scale, fwd.reserve_space_1.cpu().numpy(),
+                                   fwd.reserve_space_2.cpu().numpy(), epsilon=eps,
+                                   data_format="NCHW", dtype=dtype)
+    assert_close(to_np(grad.x_backprop, dtype), rdx, dtype, ACT_TOL[dtype], "x_backprop")
+    assert_close(grad.offset_backprop.cpu().numpy(), rob, "float32", STAT_TOL, "offset_backprop")
+    # scale_backprop cancels (dy is independent of x): relative to the spread
+    # of such a sum of N(0, 1) terms.
+    n = x.size // c
+    err = np.abs(grad.scale_backprop.cpu().numpy().astype(np.float64) - rsb).max()
+    assert err <= STAT_TOL * max(np.abs(rsb).max(), np.sqrt(n))
+    assert torch.all(grad.reserve_space_4 == 0) and torch.all(grad.reserve_space_5 == 0)

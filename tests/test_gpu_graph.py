@@ -95,7 +95,8 @@ def test_recorded_training_step_replays(dev, tune, shape, slice_tw, slices):
     assert not ops.fused_batch_norm_barrier_timed_out()
 
 
-@pytest.mark.parametrize("shape,fmt", [((8, 13, 13, 99), "NHWC"), ((2, 9, 7, 515), "NHWC")])
+@pytest.mark.parametrize("shape,fmt", [((8, 13, 13, 99), "NHWC"), ((2, 9, 7, 515), "NHWC"),
+                                       ((9, 96, 28, 28), "NCHW"), ((33, 512, 7, 7), "NCHW")])
 def test_recorded_batch_norm_replays(dev, shape, fmt):
     """The other batch-norm kernels whose workgroups wait for one another,
     recorded: three replays between eager launches, bit for bit."""
