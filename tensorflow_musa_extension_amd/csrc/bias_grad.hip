@@ -15,6 +15,7 @@
 //   stage 2: per channel, the partials in group order, cast to T.
 // Every sum runs in a fixed order, so results are deterministic.  Memory:
 // one read of x (s*E bytes), partials of G*C accumulators.
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 
@@ -62,6 +63,17 @@ struct TagArgs {
   unsigned spin_limit;
 };
 
+// What the finalizing code needs of a folded plan (BagPlan::fold): the real
+// channel count, the partials per channel (groups * fold, partial i of channel
+// ch at i * c + ch) and the rows past the last whole super-row, which it adds
+// itself.
+struct FinalArgs {
+  int c;
+  int64_t groups;
+  int64_t tail_row;
+  int tail;
+};
+
 // Tagged partial words: {value bits (low 32), epoch (high 32)}, written and
 // read with relaxed agent-scope atomics (coherent across the XCDs' L2s; one
 // single-copy-atomic word, so a word validates itself).  Float accumulators
@@ -80,21 +92,16 @@ inline size_t bag_rows_smem(int vec, size_t acc_bytes) {
   return static_cast<size_t>(kThreads) * (vec > 1 ? vec + 1 : 1) * acc_bytes;
 }
 
+template <class B, bool kTag>
+__device__ void bag_finalize_block(const typename B::A* __restrict__ partial,
+                                   const typename B::S* __restrict__ x, const FinalArgs& fa,
+                                   int fb, typename B::S* __restrict__ out, const TagArgs& tg);
+
+// rows and c: of the (super-)rows summed; fa: of the tensor.
 template <class B, int VEC, bool kTag = false>
 __global__ __launch_bounds__(kThreads) void bag_rows_kernel(
     const typename B::S* __restrict__ x, int64_t rows, int c, int64_t cv, int tx_shift,
-    int64_t rows_per_g, typename B::A* __restrict__ partial, TagArgs tg,
-    typename B::S* __restrict__ out);
-
-template <class B, bool kTag>
-__device__ void bag_finalize_block(const typename B::A* __restrict__ partial, int64_t groups,
-                                   int c, int fb, typename B::S* __restrict__ out,
-                                   const TagArgs& tg);
-
-template <class B, int VEC, bool kTag>
-__global__ __launch_bounds__(kThreads) void bag_rows_kernel(
-    const typename B::S* __restrict__ x, int64_t rows, int c, int64_t cv, int tx_shift,
-    int64_t rows_per_g, typename B::A* __restrict__ partial, TagArgs tg,
+    int64_t rows_per_g, typename B::A* __restrict__ partial, TagArgs tg, FinalArgs fa,
     typename B::S* __restrict__ out) {
   using S = typename B::S;
   using A = typename B::A;
@@ -104,8 +111,7 @@ __global__ __launch_bounds__(kThreads) void bag_rows_kernel(
   if constexpr (kTag) {
     const int64_t b = blockIdx.x;
     if (b >= tg.ct * tg.groups) {
-      bag_finalize_block<B, true>(nullptr, tg.groups, c, static_cast<int>(b - tg.ct * tg.groups),
-                                  out, tg);
+      bag_finalize_block<B, true>(nullptr, x, fa, static_cast<int>(b - tg.ct * tg.groups), out, tg);
       return;
     }
     bx = b % tg.ct;
@@ -219,8 +225,8 @@ __global__ __launch_bounds__(kThreads) void bag_planes_kernel(
   if constexpr (kTag) {
     const int64_t b = blockIdx.x;
     if (b >= tg.ct * tg.groups) {
-      bag_finalize_block<B, true>(nullptr, tg.groups, c, static_cast<int>(b - tg.ct * tg.groups),
-                                  out, tg);
+      bag_finalize_block<B, true>(nullptr, x, FinalArgs{c, tg.groups, 0, 0},
+                                  static_cast<int>(b - tg.ct * tg.groups), out, tg);
       return;
     }
     bx = b % tg.ct;
@@ -293,10 +299,12 @@ constexpr int kTagFinLoads = sizeof(S) == 2 ? 4 : 8;
 // nothing, so they all run; the spin is bounded all the same, and a partial
 // that never arrives is taken as NaN).
 template <class B, bool kTag>
-__device__ void bag_finalize_block(const typename B::A* __restrict__ partial, int64_t groups,
-                                   int c, int fb, typename B::S* __restrict__ out,
-                                   const TagArgs& tg) {
+__device__ void bag_finalize_block(const typename B::A* __restrict__ partial,
+                                   const typename B::S* __restrict__ x, const FinalArgs& fa,
+                                   int fb, typename B::S* __restrict__ out, const TagArgs& tg) {
   using A = typename B::A;
+  const int64_t groups = fa.groups;
+  const int c = fa.c;
   constexpr int kWaves = kThreads / 64;
   __shared__ A fred[kWaves][64];
   const int lane = threadIdx.x & 63;
@@ -359,15 +367,16 @@ __device__ void bag_finalize_block(const typename B::A* __restrict__ partial, in
     A t = fred[0][lane];
 #pragma unroll
     for (int k = 1; k < kWaves; ++k) t += fred[k][lane];
+    for (int r = 0; r < fa.tail; ++r) t += B::ld(x[(fa.tail_row + r) * c + ch]);
     out[ch] = B::out(t);
   }
 }
 
 template <class B>
 __global__ __launch_bounds__(kThreads) void bag_finalize_kernel(
-    const typename B::A* __restrict__ partial, int64_t groups, int c,
+    const typename B::A* __restrict__ partial, const typename B::S* __restrict__ x, FinalArgs fa,
     typename B::S* __restrict__ out) {
-  bag_finalize_block<B, false>(partial, groups, c, blockIdx.x, out, TagArgs{});
+  bag_finalize_block<B, false>(partial, x, fa, blockIdx.x, out, TagArgs{});
 }
 
 __global__ __launch_bounds__(kThreads) void zero_bytes_kernel(uint8_t* __restrict__ p, int64_t n) {
@@ -384,6 +393,7 @@ struct BagPlan {
   int ct;
   int64_t per_g;     // rows (or images) per group
   int64_t groups;
+  int fold;          // rows of a super-row (rows form), 1: none
 };
 
 // Reducing workgroups aimed for: 1024, and 256 for the rows form with 2-byte
@@ -393,12 +403,34 @@ struct BagPlan {
 // (256: 63.7, 512: 66.1, 1024: 65.5-66.5, 2048: 65.7-67.3).
 constexpr int64_t kTargetBlocks = 1024;
 constexpr int64_t kTargetBlocksRows16 = 256;
+// Columns of the widest folded super-row: its partials (at most 2^17 words)
+// then fit the tagged slots and the allocation-free scratch.
+constexpr int64_t kMinFoldChannels = 512;
+constexpr int64_t kMinFoldBytes = int64_t(4) << 20;
+constexpr int64_t kMaxFoldColumns = int64_t(1) << 16;
 
 BagPlan make_bag_plan(int64_t outer, int64_t c, int64_t inner, int esize, bool aligned) {
   BagPlan p{};
   p.rows = inner == 1;
+  p.fold = 1;
   if (p.rows) {
     const int kv = 16 / esize;
+    // A channel count that is no multiple of a vector: `fold` rows are a
+    // whole number of vectors, one super-row of fold * c columns, each of one
+    // channel; the columns are summed as channels and a channel's `fold`
+    // columns added at the end.  Back to back, against 2- and 4-byte loads:
+    // f32 [8191,4095] 44.2 -> 30.0 us, f16 35.4 -> 18.1, bf16 [3000,8191] 28.0
+    // -> 14.5, f32 [4001,1021] 10.2 -> 8.8.  Few channels or little data leave
+    // many partials per channel to too few finalizing waves (f16 [65536,33]
+    // 10.7 -> 33.8, [256,2047] 3.8 -> 4.6): those keep the narrow loads.
+    int gcd = kv;
+    while (c % gcd != 0) gcd >>= 1;
+    if (aligned && gcd < kv && c >= kMinFoldChannels && outer * c * esize >= kMinFoldBytes &&
+        c * (kv / gcd) <= kMaxFoldColumns) {
+      p.fold = kv / gcd;
+      outer /= p.fold;
+      c *= p.fold;
+    }
     p.vec = (aligned && c % kv == 0) ? kv : 1;
     p.cv = c / p.vec;
     int s = 0;
@@ -409,7 +441,7 @@ BagPlan make_bag_plan(int64_t outer, int64_t c, int64_t inner, int esize, bool a
     int64_t gt = (esize == 2 ? kTargetBlocksRows16 : kTargetBlocks) / p.ct;
     if (gt < 1) gt = 1;
     int64_t rpg = (outer + gt - 1) / gt;
-    const int64_t min_rows = static_cast<int64_t>(ry) * kUnroll;
+    const int64_t min_rows = static_cast<int64_t>(ry) * (kUnroll / p.fold > 1 ? kUnroll / p.fold : 1);
     if (rpg < min_rows) rpg = min_rows;
     p.per_g = rpg;
     p.groups = (outer + rpg - 1) / rpg;
@@ -430,6 +462,11 @@ BagPlan make_bag_plan(int64_t outer, int64_t c, int64_t inner, int esize, bool a
   }
   if (p.groups < 1) p.groups = 1;
   return p;
+}
+
+FinalArgs final_args(const BagPlan& p, int64_t outer, int64_t c) {
+  const int64_t tail = outer % p.fold;
+  return FinalArgs{static_cast<int>(c), p.groups * p.fold, outer - tail, static_cast<int>(tail)};
 }
 
 // ---- one launch: tagged partials and trailing finalizing workgroups ------
@@ -464,7 +501,7 @@ bool tag_applies(const BagPlan& p, int64_t c, hipStream_t stream) {
     return false;
   } else {
     if (TuneValue(kTuneBagFused) == 0) return false;
-    if (static_cast<size_t>(p.groups) * static_cast<size_t>(c) > kTagSlots) return false;
+    if (static_cast<size_t>(p.groups) * p.fold * static_cast<size_t>(c) > kTagSlots) return false;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(stream, &cap) != hipSuccess) return false;
     return cap == hipStreamCaptureStatusNone;
@@ -514,18 +551,19 @@ hipError_t launch_bag_tagged(const BagPlan& p, const void* x, int64_t outer, int
   const TraceEvents tev = TraceTake(kName);
   hipEvent_t end = ts->chain.end_event(tev.end);
   constexpr int V = 16 / sizeof(S);
+  const FinalArgs fa = final_args(p, outer, c);
   if (p.rows) {
     tg.ct = p.ct;
     const dim3 grid(static_cast<unsigned>(p.ct * p.groups + fin));
     const size_t smem = bag_rows_smem(p.vec, sizeof(float));
     if (p.vec == V)
       hipExtLaunchKernelGGL((bag_rows_kernel<B, V, true>), grid, dim3(kThreads), smem, stream,
-                            tev.start, end, 0, xs, outer, static_cast<int>(c), p.cv, p.tx_shift,
-                            p.per_g, static_cast<float*>(nullptr), tg, o);
+                            tev.start, end, 0, xs, outer / p.fold, static_cast<int>(c) * p.fold,
+                            p.cv, p.tx_shift, p.per_g, static_cast<float*>(nullptr), tg, fa, o);
     else
       hipExtLaunchKernelGGL((bag_rows_kernel<B, 1, true>), grid, dim3(kThreads), smem, stream,
                             tev.start, end, 0, xs, outer, static_cast<int>(c), p.cv, p.tx_shift,
-                            p.per_g, static_cast<float*>(nullptr), tg, o);
+                            p.per_g, static_cast<float*>(nullptr), tg, fa, o);
   } else {
     tg.ct = static_cast<int>(c);
     const dim3 grid(static_cast<unsigned>(c * p.groups + fin));
@@ -565,6 +603,7 @@ hipError_t launch_bag(const void* x, int64_t outer, int64_t c, int64_t inner, vo
       return launch_bag_tagged<B>(p, x, outer, c, inner, out, stream);
   }
   A* partial = static_cast<A*>(workspace);
+  const FinalArgs fa = final_args(p, outer, c);
   const S* xs = static_cast<const S*>(x);
   {
     if (p.rows) {
@@ -572,12 +611,12 @@ hipError_t launch_bag(const void* x, int64_t outer, int64_t c, int64_t inner, vo
       constexpr int V = 16 / sizeof(S);
       if (p.vec == V) {
         TFMA_LAUNCH("tfma_bias_add_grad_reduce", (bag_rows_kernel<B, V>), dim3(p.ct, p.groups), dim3(kThreads), smem,
-                           stream, xs, outer, static_cast<int>(c), p.cv, p.tx_shift, p.per_g,
-                           partial, TagArgs{}, static_cast<S*>(nullptr));
+                           stream, xs, outer / p.fold, static_cast<int>(c) * p.fold, p.cv,
+                           p.tx_shift, p.per_g, partial, TagArgs{}, fa, static_cast<S*>(nullptr));
       } else {
         TFMA_LAUNCH("tfma_bias_add_grad_reduce", (bag_rows_kernel<B, 1>), dim3(p.ct, p.groups), dim3(kThreads), smem,
                            stream, xs, outer, static_cast<int>(c), p.cv, p.tx_shift, p.per_g,
-                           partial, TagArgs{}, static_cast<S*>(nullptr));
+                           partial, TagArgs{}, fa, static_cast<S*>(nullptr));
       }
     } else if (p.vec > 1) {
       constexpr int V = 16 / sizeof(S);
@@ -598,15 +637,14 @@ hipError_t launch_bag(const void* x, int64_t outer, int64_t c, int64_t inner, vo
   constexpr const char* kFinalize = "tfma_bias_add_grad_finalize";
   if (!chain_end) {
     TFMA_LAUNCH(kFinalize, (bag_finalize_kernel<B>), dim3((c + 63) / 64), dim3(kThreads), 0,
-                stream, partial, p.groups, static_cast<int>(c), static_cast<S*>(out));
+                stream, partial, xs, fa, static_cast<S*>(out));
     return hipGetLastError();
   }
   SetLastKernel(kFinalize);
   const TraceEvents tev = TraceTake(kFinalize);
   hipEvent_t end = tev.end ? tev.end : *chain_end;  // may be null: no end event
   hipExtLaunchKernelGGL((bag_finalize_kernel<B>), dim3((c + 63) / 64), dim3(kThreads), 0, stream,
-                        tev.start, end, 0, partial, p.groups, static_cast<int>(c),
-                        static_cast<S*>(out));
+                        tev.start, end, 0, partial, xs, fa, static_cast<S*>(out));
   TraceCommit(tev);
   *chain_end = end;
   return hipGetLastError();
@@ -647,7 +685,7 @@ hipError_t BiasAddGradScratch(void** ptr) {
 size_t BiasAddGradWorkspaceBytes(int dt, int64_t outer, int64_t c, int64_t inner, int esize) {
   const BagPlan p = make_bag_plan(outer, c, inner, esize, true);
   const BagPlan q = make_bag_plan(outer, c, inner, esize, false);
-  const int64_t g = p.groups > q.groups ? p.groups : q.groups;
+  const int64_t g = std::max(p.groups * p.fold, q.groups * q.fold);
   return (static_cast<size_t>(g) * c * acc_bytes(dt) + 255) & ~size_t(255);
 }
 

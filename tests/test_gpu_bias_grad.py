@@ -162,3 +162,29 @@ def test_one_launch_calls_on_two_streams(dev):
     torch.cuda.synchronize()
     for i, (o, w) in enumerate(zip(outs, wants)):
         assert torch.equal(o.view(torch.int16), w.view(torch.int16)), f"call {i} {shapes[i]}"
+
+
+# Super-rows of 2, 4 and 8 rows, every kind of remainder, the fewest channels
+# and bytes that fold and just fewer, the most columns.
+@pytest.mark.parametrize("dtype", ["float32", "float16", "bfloat16", "float64", "int32"])
+@pytest.mark.parametrize("shape", [(4101, 513), (4099, 514), (4098, 516), (4096, 511),
+                                   (2051, 1021), (2047, 1021), (259, 8191), (130, 16387)])
+def test_folded_rows(dev, tune, dtype, shape):
+    rng = np.random.default_rng(14)
+    x = gen(rng, shape, dtype)
+    xd = to_dev(x, dtype, dev)
+    one = ops.BiasAddGrad(xd)
+    tune("bag_fused", 0)
+    two = ops.BiasAddGrad(xd)
+    out = torch.empty_like(one)
+    ops.bias_add_grad_no_alloc(xd, out)
+    torch.cuda.synchronize()
+    assert torch.equal(one, two) and torch.equal(one, out)
+    if dtype in ("float64", "int32"):
+        want = torch.from_numpy(x).sum(0)
+        got = one.cpu()
+        assert torch.equal(got, want.int()) if dtype == "int32" else torch.allclose(
+            got, want, rtol=0, atol=1e-11 * shape[0])
+    else:
+        ref = oracle.bias_add_grad(x, "NHWC", dtype)
+        assert_close(to_np(one, dtype), ref, dtype, TOL[dtype], f"{dtype} {shape}")
