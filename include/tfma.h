@@ -416,7 +416,7 @@ int TFMA_FusedBatchNormBarrierTimedOut(int32_t* timed_out, int32_t reset, TFMA_S
 
 /* Launch plan of the calling thread's last FusedBatchNormV3 /
  * FusedBatchNormGradV3 call (for tests that check which path ran).
- * fused = 1: the persistent kernel ran with `workgroups` workgroups over
+ * fused = 1: one of the one-launch kernels ran with `workgroups` workgroups over
  * row_groups x channel_tiles; dynamic_rows > 0: each thread's lowest
  * dynamic_rows streamed phase-3 rows were handed out in chunks of
  * dynamic_chunk rows; register_rows / lds_rows: rows per thread kept on chip;
@@ -455,7 +455,8 @@ const char* TFMA_LastKernelName(void);
  *   "bn_sliced_overlap" 0: sliced gradients run the plain sliced pass
  *                       instead of hiding each slice's hand-off.
  *   "bn_nchw_owned"     0: NCHW training keeps the split kernels instead of
- *                       one workgroup per channel.
+ *                       one workgroup per channel, shared channels or units
+ *                       of channels.
  *   "bag_fused"         0: BiasAddGrad runs as two kernels (partials, then
  *                       per-channel finals) instead of one launch.
  * Each starts from the environment variable TFMA_<NAME in upper case>,

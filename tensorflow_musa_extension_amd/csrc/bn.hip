@@ -34,7 +34,6 @@
 // workgroup uses the same K.
 #include <hip/hip_ext.h>
 
-
 #include <atomic>
 #include <mutex>
 
@@ -4232,6 +4231,15 @@ hipError_t launch_nchw_owned(const BnGeometry& g, const void* x, const void* dy,
   return hipGetLastError();
 }
 
+// Launches recorded into a graph are not chained to other launches, so a
+// replay of a kernel whose workgroups wait for one another must not overlap
+// other such work.  The ops that run the folded super-rows, units and shared
+// channels when eager are recorded as the split kernels, whose replays may.
+bool recording(hipStream_t stream) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone;
+}
+
 bool ptr_aligned(const void* p) {
   return (reinterpret_cast<uintptr_t>(p) & 15) == 0;
 }
@@ -4276,13 +4284,14 @@ hipError_t forward_t(const BnGeometry& g, const BnFwdArgs& a, void* ws,
     return launch_fused<Tr, false>(fp, g, a.x, nullptr, a.y, fa,
                                                   stream);
   }
-  if (a.is_training && aligned && fused_enabled() &&
+  const bool eager = a.is_training && aligned && fused_enabled() && !recording(stream);
+  if (eager &&
       make_unit_plan(g, Tr::kVec, folded_blocks_per_cu<Tr, false>(), &fp))
     return launch_fused<Tr, false>(fp, g, a.x, nullptr, a.y, fa, stream);
-  if (a.is_training && aligned && fused_enabled() &&
+  if (eager &&
       make_shared_plan(g, Tr::kVec, shared_blocks_per_cu<Tr, false>(), &fp))
     return launch_fused<Tr, false>(fp, g, a.x, nullptr, a.y, fa, stream);
-  if (a.is_training && aligned && fused_enabled() &&
+  if (eager && g.c % Tr::kVec != 0 &&
       make_folded_plan(g, Tr::kVec, folded_blocks_per_cu<Tr, false>(), &fp))
     return launch_fused<Tr, false>(fp, g, a.x, nullptr, a.y, fa, stream);
   note_split_plan(p);
@@ -4336,13 +4345,14 @@ hipError_t grad_t(const BnGeometry& g, const BnGradArgs& a, void* ws,
     return launch_fused<Tr, true>(fp, g, a.x, a.dy, a.dx, fa,
                                                   stream);
   }
-  if (aligned && fused_enabled() &&
+  const bool eager = aligned && fused_enabled() && !recording(stream);
+  if (eager &&
       make_unit_plan(g, Tr::kVec, folded_blocks_per_cu<Tr, true>(), &fp))
     return launch_fused<Tr, true>(fp, g, a.x, a.dy, a.dx, fa, stream);
-  if (aligned && fused_enabled() &&
+  if (eager &&
       make_shared_plan(g, Tr::kVec, shared_blocks_per_cu<Tr, true>(), &fp))
     return launch_fused<Tr, true>(fp, g, a.x, a.dy, a.dx, fa, stream);
-  if (aligned && fused_enabled() &&
+  if (eager && g.c % Tr::kVec != 0 &&
       make_folded_plan(g, Tr::kVec, folded_blocks_per_cu<Tr, true>(), &fp))
     return launch_fused<Tr, true>(fp, g, a.x, a.dy, a.dx, fa, stream);
   note_split_plan(p);

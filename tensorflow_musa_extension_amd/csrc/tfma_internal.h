@@ -226,8 +226,9 @@ hipError_t LaunchElementwise(DType t, EwOp op, int64_t n,
                              const BcastOperand& c, void* out,
                              hipStream_t stream);
 
-// General strided broadcast fallback (rank <= 8): strides are in elements,
-// 0 on broadcast dimensions.
+// General broadcasts (rank <= 8), by row of the innermost merged dimension:
+// strides are in elements, 0 on broadcast dimensions; every operand is
+// contiguous in its own order.
 struct StridedShape {
   int ndims;
   int64_t dims[TFMA_MAX_DIMS];

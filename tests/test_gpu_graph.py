@@ -95,11 +95,17 @@ def test_recorded_training_step_replays(dev, tune, shape, slice_tw, slices):
     assert not ops.fused_batch_norm_barrier_timed_out()
 
 
-@pytest.mark.parametrize("shape,fmt", [((8, 13, 13, 99), "NHWC"), ((2, 9, 7, 515), "NHWC"),
-                                       ((9, 96, 28, 28), "NCHW"), ((33, 512, 7, 7), "NCHW")])
-def test_recorded_batch_norm_replays(dev, shape, fmt):
-    """The other batch-norm kernels whose workgroups wait for one another,
-    recorded: three replays between eager launches, bit for bit."""
+# (8,13,13,72): the folded kernel, recorded as it runs.  The others run kernels
+# whose workgroups wait for one another when eager and are recorded as the
+# split kernels (a replay may overlap other work).
+@pytest.mark.parametrize("shape,fmt,same", [((8, 13, 13, 72), "NHWC", True),
+                                            ((8, 13, 13, 99), "NHWC", False),
+                                            ((2, 9, 7, 515), "NHWC", False),
+                                            ((9, 96, 28, 28), "NCHW", False),
+                                            ((33, 512, 7, 7), "NCHW", False)])
+def test_recorded_batch_norm_replays(dev, shape, fmt, same):
+    """Three replays between eager launches: bit for bit the eager results, or
+    one another and within rounding of the eager results."""
     gen_ = torch.Generator(device=dev)
     gen_.manual_seed(33)
     c = shape[-1] if fmt == "NHWC" else shape[1]
@@ -108,10 +114,11 @@ def test_recorded_batch_norm_replays(dev, shape, fmt):
     offset = torch.randn(c, generator=gen_, device=dev)
     e = torch.empty(0, device=dev)
     kw = dict(epsilon=EPS, data_format=fmt)
+    plans = []
 
     def step():
         f = ops.FusedBatchNormV3(x, scale, offset, e, e, **kw)
-        assert ops.fused_batch_norm_last_plan()["fused"] != 0
+        plans.append(ops.fused_batch_norm_last_plan()["fused"])
         return tuple(f) + tuple(ops.FusedBatchNormGradV3(
             dy, x, scale, f.reserve_space_1, f.reserve_space_2, f.reserve_space_3, **kw))
 
@@ -120,12 +127,23 @@ def test_recorded_batch_norm_replays(dev, shape, fmt):
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
         outs = step()
+    assert plans == [1, 1 if same else 0]
+    first = None
     for _ in range(3):
         for t in outs:
             t.fill_(float("nan"))
         graph.replay()
         torch.cuda.synchronize()
-        assert all(torch.equal(a, b) for a, b in zip(outs, want))
+        if first is None:
+            first = [t.clone() for t in outs]
+        for got, one, w in zip(outs, first, want):
+            assert torch.equal(got, one)
+            if same:
+                assert torch.equal(got, w)
+            elif w.dtype == torch.float16:  # one ulp of the largest value
+                assert (got.float() - w.float()).abs().max() <= 2 ** -10 * w.float().abs().max()
+            else:  # float32 sums of the same terms in another order
+                assert (got - w).abs().max() <= 1e-5 * max(w.abs().max().item(), 1.0)
         assert all(torch.equal(a, b) for a, b in zip(step(), want))
         torch.cuda.synchronize()
     assert not ops.fused_batch_norm_barrier_timed_out()
