@@ -14,7 +14,9 @@
 //     offset_backprop = sum(dy), scale_backprop = k * sum(dy * xc)
 //     dx = scale*k * ((dy - sum(dy)/n) - xc * (k*k * sum(dy*xc)/n))
 //
-// Structure: three kernels per op.
+// Structure: one launch per op where it can be (sections 4 to 6 below); what
+// is left (inference, unaligned pointers, and other forms those exclude) runs
+// three kernels per op.
 //   1. reduce:   each workgroup owns a row range x channel tile and writes
 //                one float2 partial per channel (shifted sums for the
 //                forward, sum(dy) / sum(dy*xc) for the grad).  16-byte loads,

@@ -15,8 +15,9 @@
 // vector when its period is a multiple of the vector width (row vectors such
 // as a BiasAdd bias over the last dimension), as one value per vector when
 // its inner extent is (NCHW bias), and gathered per element otherwise (odd
-// shapes such as [8191, 4095]).  Broadcast operands are tiny and stay in
-// L1/L2, so HBM traffic is the compulsory stream of the full-size tensors.
+// shapes such as [8191, 4095]); broadcasts of several runs are walked by row
+// (ew_rows_kernel).  Broadcast operands are tiny and stay in L1/L2, so HBM
+// traffic is the compulsory stream of the full-size tensors.
 #include <atomic>
 #include <type_traits>
 
