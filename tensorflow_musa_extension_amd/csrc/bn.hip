@@ -3514,13 +3514,14 @@ bool make_folded_plan(const BnGeometry& g, int vec, int blocks_per_cu, FusedPlan
 }
 
 // The unit plan (16-byte aligned pointers): planes that are no multiple of a
-// vector, whole units of channels, and units of at most one pass of a
-// workgroup.
+// vector, whole units of channels, units of at most one pass of a workgroup,
+// and a tensor of fewer than 2^31 elements: every workgroup's shift samples
+// (chan_shift_nchw) are anywhere in it, whatever its own rows span.
 bool make_unit_plan(const BnGeometry& g, int vec, int blocks_per_cu, FusedPlan* fp) {
   const int64_t plane = g.h * g.w;
   const int64_t esz = 16 / vec;
   if (g.nhwc || blocks_per_cu < 1 || plane % vec == 0 || g.n < 1 ||
-      TuneValue(kTuneBnNchwOwned) == 0)
+      g.n * g.c * plane >= (int64_t{1} << 31) || TuneValue(kTuneBnNchwOwned) == 0)
     return false;
   int gcd = vec;
   while (plane % gcd != 0) gcd >>= 1;

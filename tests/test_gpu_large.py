@@ -225,3 +225,41 @@ def test_batch_norm_wide_channels_group_span(dev, rows, kernel):
     assert torch.allclose(g.scale_backprop.double(), sbp, rtol=1e-5, atol=5e-2)
     ref = bn_grad_ref32(dy, x, scale, mu, sig, g.offset_backprop, g.scale_backprop, eps, rows, c)
     assert bn_max_ulp(g.x_backprop, ref, rows, c, rows_per=2048) <= 1
+
+
+@pytest.mark.parametrize("n,kernel", [(342387, "fused"), (1_500_000, "apply_nchw")])
+def test_batch_norm_nchw_odd_planes_over_2_31(dev, n, kernel):
+    """FusedBatchNormV3 on [n, 128, 7, 7] f16, whose channels lie 8 apart with
+    a spread of 0.8: an element of another channel as the sums' shift would
+    leave the variance a difference of numbers 10^6 times its size.  Below 2^31
+    elements (342387 images) the unit kernel's 32-bit sample positions hold; at
+    1.5 million images (9.4e9 elements) three of the five samples lie past
+    2^32 and the op must take the split path's 64-bit ones.  The images repeat
+    a block of 1000, so the statistics are known in float64: mean 1e-5 of its
+    largest value, variance 5e-5 relative (as above)."""
+    _need(n * 128 * 49 * 4 / 2**30 + 2)
+    c, block = 128, 1000
+    torch.manual_seed(16)
+    noise = torch.randint(-1, 2, (block, c, 7, 7), device=dev, dtype=torch.float16)
+    tile = noise + (8.0 * torch.arange(c, device=dev) - 512).half().view(1, c, 1, 1)
+    x = torch.empty((n, c, 7, 7), device=dev, dtype=torch.float16)
+    for i in range(0, n, block):
+        x[i:i + block] = tile[:n - i]
+    t = torch.cat([tile.double()] * 2)[:block + n % block]
+    count = torch.full((t.shape[0], 1, 1, 1), float(n // block), device=dev, dtype=torch.float64)
+    count[block:] = 1.0
+    mean = (t * count).sum((0, 2, 3)) / (n * 49)
+    var = ((t - mean.view(1, c, 1, 1)) ** 2 * count).sum((0, 2, 3)) / (n * 49)
+    e = torch.empty(0, device=dev)
+    scale = torch.rand(c, device=dev) + 0.5
+    offset = torch.randn(c, device=dev)
+    eps = 1.001e-5
+    f = ops.FusedBatchNormV3(x, scale, offset, e, e, epsilon=eps, data_format="NCHW")
+    assert torch.allclose(f.reserve_space_1.double(), mean, rtol=0, atol=512e-5)
+    assert torch.allclose(f.reserve_space_2.double(), var, rtol=5e-5, atol=0)
+    assert ops.last_kernel_name() == f"tfma_bn_fwd_{kernel}"
+    k = (scale / torch.sqrt(f.reserve_space_2 + eps)).view(1, c, 1, 1)
+    for i in (0, n // 2 // block * block, (n - 1) // block * block):  # one ulp at most 4
+        want = (x[i:i + block].float() - f.reserve_space_1.view(1, c, 1, 1)) * k \
+            + offset.view(1, c, 1, 1)
+        assert (f.y[i:i + block].float() - want).abs().max() <= 2 ** -8
