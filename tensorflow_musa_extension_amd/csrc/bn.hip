@@ -937,6 +937,15 @@ __device__ inline double2 wave_sum(double a, double b) {
   }
   return make_double2(a, b);
 }
+// The same of float sums, added in float32.
+__device__ inline double2 wave_sum_f32(float a, float b) {
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) {
+    a += __shfl_xor(a, off, 64);
+    b += __shfl_xor(b, off, 64);
+  }
+  return make_double2(a, b);
+}
 
 // Coherent (agent-scope) 8-byte store/load for values shared across XCDs.
 __device__ inline void store_shared(void* p, uint64_t v) {
@@ -2368,7 +2377,10 @@ __global__ __launch_bounds__(kFusedThreads) void bn_folded_nhwc_kernel(FoldedArg
     pl = static_cast<uint32_t>(tid) - part * nl;
   }
   const bool adds = part < parts && pl < nl;
-  float sum[2];
+  // Units add across threads in double: the sums of a unit's only row group go
+  // to the statistics as they are, not as one of several partials.
+  using Sum = typename std::conditional<kUnit, double, float>::type;
+  Sum sum[2];
 #pragma unroll
   for (int w = 0; w < 2; ++w) {
     __syncthreads();
@@ -2377,7 +2389,7 @@ __global__ __launch_bounds__(kFusedThreads) void bn_folded_nhwc_kernel(FoldedArg
       for (int j = 0; j < VEC; ++j) red[tid * VEC + j] = w == 0 ? s1[j] : s2[j];
     }
     __syncthreads();
-    float t = 0.f;
+    Sum t = 0;
     if (adds) {
       if constexpr (kUnit) {
         const uint32_t pl0 = pl * static_cast<uint32_t>(fa.plane);
@@ -2400,20 +2412,21 @@ __global__ __launch_bounds__(kFusedThreads) void bn_folded_nhwc_kernel(FoldedArg
   }
   if (parts > 1) {
     __syncthreads();
+    Sum* const rs = reinterpret_cast<Sum*>(red);
     if (kUnit ? adds && part == 0 : adds) {
       const uint32_t at = kUnit ? pl : static_cast<uint32_t>(tid);
-      red[2 * at] = sum[0];
-      red[2 * at + 1] = sum[1];
+      rs[2 * at] = sum[0];
+      rs[2 * at + 1] = sum[1];
     }
     __syncthreads();
     if (owner) {
-      sum[0] = red[2 * tid];
-      sum[1] = red[2 * tid + 1];
+      sum[0] = rs[2 * tid];
+      sum[1] = rs[2 * tid + 1];
       if constexpr (!kUnit) {
 #pragma unroll 4
         for (uint32_t p = 1; p < parts; ++p) {
-          sum[0] += red[2 * (p * nl + tid)];
-          sum[1] += red[2 * (p * nl + tid) + 1];
+          sum[0] += rs[2 * (p * nl + tid)];
+          sum[1] += rs[2 * (p * nl + tid) + 1];
         }
       }
     }
@@ -2435,7 +2448,7 @@ __global__ __launch_bounds__(kFusedThreads) void bn_folded_nhwc_kernel(FoldedArg
       const int64_t slot =
           kUnit ? g * C + ch_t : (single ? g * C + tid : g * fa.fold * C + ve);
       store_pair(slots_rsrc(a.eslots, a.groups, a.c), slot, static_cast<uint32_t>(etag >> 32),
-                 sum[0], sum[1]);
+                 static_cast<float>(sum[0]), static_cast<float>(sum[1]));
     }
     finish_channel_blocks<Tr, kGrad, !kUnit>(a, 0, a.c, wave, lane, wtag, etag, epoch);
   }
@@ -2813,7 +2826,8 @@ __global__ __launch_bounds__(kFusedThreads) void bn_nchw_shared_kernel(SharedNch
   constexpr int U = kGrad ? 4 : 8;
   constexpr int kWaves = kFusedThreads / 64;
   extern __shared__ uint4 lds_rows[];  // [KL][kIn][kFusedThreads]
-  __shared__ float2 red[2][kWaves];
+  using Sums = typename std::conditional<kTwo, float2, double2>::type;
+  __shared__ Sums red[2][kWaves];
   __shared__ float4 cfs[2];
   const FusedArgs& a = na.f;
   const int tid = threadIdx.x;
@@ -3017,16 +3031,23 @@ __global__ __launch_bounds__(kFusedThreads) void bn_nchw_shared_kernel(SharedNch
     a2s = s2;
     s1 = s2 = 0.f;
   }
+  // Across threads in double where a channel has one workgroup, whose sums go
+  // to the statistics as they are; else they are published in float32.
+  if constexpr (!kTwo) {
+    const double2 w = na.parts == 1 ? wave_sum(a1s, a2s) : wave_sum_f32(a1s, a2s);
+    if (lane == 0) red[0][wave] = w;
+  } else {
 #pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) {
-    a1s += __shfl_xor(a1s, off, 64);
-    a2s += __shfl_xor(a2s, off, 64);
-    s1 += __shfl_xor(s1, off, 64);
-    s2 += __shfl_xor(s2, off, 64);
-  }
-  if (lane == 0) {
-    red[0][wave] = make_float2(a1s, a2s);
-    red[1][wave] = make_float2(s1, s2);
+    for (int off = 32; off >= 1; off >>= 1) {
+      a1s += __shfl_xor(a1s, off, 64);
+      a2s += __shfl_xor(a2s, off, 64);
+      s1 += __shfl_xor(s1, off, 64);
+      s2 += __shfl_xor(s2, off, 64);
+    }
+    if (lane == 0) {
+      red[0][wave] = make_float2(a1s, a2s);
+      red[1][wave] = make_float2(s1, s2);
+    }
   }
   __syncthreads();
 
@@ -3039,41 +3060,46 @@ __global__ __launch_bounds__(kFusedThreads) void bn_nchw_shared_kernel(SharedNch
         kTwo ? na.div_share.div(ch * na.nv + na.nv - 1) : w0 + na.parts - 1;
     const uint32_t cnt = w1 - w0 + 1;
     const auto rs = rows_rsrc(a.eslots, static_cast<int64_t>(a.c) * na.parts * 16);
-    if (lane == 0) {
-      float2 sum = red[wave][0];
+    typename std::conditional<kTwo, float, double>::type o1 = 0, o2 = 0;
 #pragma unroll
-      for (int i = 1; i < kWaves; ++i) {
-        sum.x += red[wave][i].x;
-        sum.y += red[wave][i].y;
-      }
+    for (int i = 0; i < kWaves; ++i) {
+      o1 += red[wave][i].x;
+      o2 += red[wave][i].y;
+    }
+    // (The plan gives two channels to a workgroup only where each has several.)
+    const bool several = kTwo || cnt > 1;
+    if (several && lane == 0)
       store_pair(rs, static_cast<int64_t>(ch) * na.parts + (b - w0),
-                 static_cast<uint32_t>(etag >> 32), sum.x, sum.y);
-    }
+                 static_cast<uint32_t>(etag >> 32), static_cast<float>(o1),
+                 static_cast<float>(o2));
     const FinIn fin_in = fin_inputs<Tr, kGrad>(a.fin, static_cast<int>(ch), wave == 0 ? ka : kb);
-    double t1 = 0.0, t2 = 0.0;
-    for (uint32_t p0 = 0; p0 < cnt; p0 += 64) {
-      const uint32_t p = p0 + static_cast<uint32_t>(lane);
-      const bool has = p < cnt;
-      const int64_t slot =
-          has ? static_cast<int64_t>(ch) * na.parts + p : int64_t(kOutOfRange / 16);
-      u32x4 v = load_pair(rs, slot);
-      unsigned spins = 0;
-      while (has && !pair_tagged(v, wtag)) {
-        if (++spins > a.spin_limit) {
-          v = u32x4{0x7fc00000u, wtag, 0x7fc00000u, wtag};
-          __hip_atomic_store(a.gave_up, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-          break;
+    double2 w = make_double2(o1, o2);
+    if (several) {
+      double t1 = 0.0, t2 = 0.0;
+      for (uint32_t p0 = 0; p0 < cnt; p0 += 64) {
+        const uint32_t p = p0 + static_cast<uint32_t>(lane);
+        const bool has = p < cnt;
+        const int64_t slot =
+            has ? static_cast<int64_t>(ch) * na.parts + p : int64_t(kOutOfRange / 16);
+        u32x4 v = load_pair(rs, slot);
+        unsigned spins = 0;
+        while (has && !pair_tagged(v, wtag)) {
+          if (++spins > a.spin_limit) {
+            v = u32x4{0x7fc00000u, wtag, 0x7fc00000u, wtag};
+            __hip_atomic_store(a.gave_up, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            break;
+          }
+          __builtin_amdgcn_s_sleep(1);
+          asm volatile("" ::: "memory");  // the reload is not the load above
+          v = load_pair(rs, slot);
         }
-        __builtin_amdgcn_s_sleep(1);
-        asm volatile("" ::: "memory");  // the reload is not the load above
-        v = load_pair(rs, slot);
+        if (has) {
+          t1 += bits_f32(v[0]);
+          t2 += bits_f32(v[2]);
+        }
       }
-      if (has) {
-        t1 += bits_f32(v[0]);
-        t2 += bits_f32(v[2]);
-      }
+      w = wave_sum(t1, t2);
     }
-    const double2 w = wave_sum(t1, t2);
     if (lane == 0)
       cfs[wave] = finish_channel<Tr, kGrad>(a.fin, static_cast<int>(ch), w.x, w.y, fin_in,
                                             b == w0);
@@ -3558,8 +3584,8 @@ bool make_unit_plan(const BnGeometry& g, int vec, int blocks_per_cu, FusedPlan* 
 // counts); ops with few rows per thread run the FewRows counts.
 template <class Tr, bool kGrad, bool kOdd>
 constexpr int shared_kr() {
-  constexpr bool half = std::is_same<Tr, TF16>::value, bf = std::is_same<Tr, TBF16>::value;
-  return kGrad ? (kOdd ? 14 : (half ? 17 : (bf ? 16 : 15))) : (kOdd ? 26 : (half ? 32 : 29));
+  constexpr bool half = std::is_same<Tr, TF16>::value;
+  return kGrad ? (kOdd ? 14 : (half ? 17 : 15)) : (kOdd ? 26 : (half ? 32 : 29));
 }
 
 template <class Tr, bool kGrad, bool kOdd, bool kTwo>
@@ -3629,10 +3655,9 @@ bool make_shared_plan(const BnGeometry& g, int vec, int blocks_per_cu, FusedPlan
   // A whole number of workgroups per channel where that leaves at most an
   // eighth of the CUs idle or the channels are short.
   const int64_t whole = std::max<int64_t>(1, std::min(wgs / g.c, (nv + least - 1) / least));
-  const bool two = whole * g.c * 8 < wgs * 7 && whole == wgs / g.c;
-  int64_t share, blocks, parts;
+  int64_t share = std::max((g.c * nv + wgs - 1) / wgs, least), blocks, parts;
+  const bool two = whole * g.c * 8 < wgs * 7 && whole == wgs / g.c && share < nv;
   if (two) {
-    share = std::min(nv, std::max((g.c * nv + wgs - 1) / wgs, least));
     blocks = (g.c * nv + share - 1) / share;
     parts = (nv + share - 1) / share + 1;
   } else {

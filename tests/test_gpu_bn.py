@@ -895,3 +895,24 @@ def test_nchw_matches_oracle(dev, shape, dtype):
     err = np.abs(grad.scale_backprop.cpu().numpy().astype(np.float64) - rsb).max()
     assert err <= STAT_TOL * max(np.abs(rsb).max(), np.sqrt(n))
     assert torch.all(grad.reserve_space_4 == 0) and torch.all(grad.reserve_space_5 == 0)
+
+
+@pytest.mark.parametrize("shape", [(256, 260, 14, 14), (64, 230, 28, 28), (64, 260, 28, 28)])
+def test_nchw_one_workgroup_channels_sum_in_double(dev, shape):
+    """Channels that one workgroup finishes alone (a unit, a shared channel of
+    one part, an owned channel): a thread sums at most 128 values of [1, 2) in
+    steps of 2^-10, which float32 holds exactly (18 bits); a channel's 50176
+    take 27 bits, so offset_backprop is the correctly rounded sum only if the
+    threads' sums are added in more than float32."""
+    n = shape[0] * shape[2] * shape[3]
+    assert n == 50176
+    g = torch.Generator(device=dev)
+    g.manual_seed(5)
+    x = torch.randn(shape, generator=g, device=dev).half()
+    dy = (torch.randint(1024, 2048, shape, generator=g, device=dev) / 1024).half()
+    c = shape[1]
+    one, zero = torch.ones(c, device=dev), torch.zeros(c, device=dev)
+    got = ops.FusedBatchNormGradV3(dy, x, one, zero, one, torch.zeros((), device=dev),
+                                   epsilon=1e-3, data_format="NCHW")
+    assert ops.fused_batch_norm_last_plan()["workgroups"] <= max(c, 256)
+    assert torch.equal(got.offset_backprop, dy.double().sum((0, 2, 3)).float())
