@@ -4268,6 +4268,29 @@ bool recording(hipStream_t stream) {
   return hipStreamIsCapturing(stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone;
 }
 
+// Whether a per-channel output lies over a per-channel input.  Such calls keep
+// the kernels in which one thread reads a channel's inputs and writes its
+// outputs: in the shared NCHW kernel the first of a channel's workgroups may
+// write them before another has read.
+bool channel_outputs_over_inputs(const FinArgs& f) {
+  const size_t bytes = static_cast<size_t>(f.c) * sizeof(float);
+  struct Range {
+    const void* p;
+    size_t n;
+  };
+  const Range in[] = {{f.scale, bytes}, {f.offset, bytes}, {f.mean_in, bytes}, {f.var_in, bytes}};
+  const Range out[] = {{f.batch_mean, bytes}, {f.batch_var, bytes}, {f.saved_mean, bytes},
+                       {f.saved_var, bytes}, {f.reserve3, sizeof(float)}, {f.scale_bp, bytes},
+                       {f.offset_bp, bytes}, {f.reserve4, f.reserve4_n * sizeof(float)},
+                       {f.reserve5, f.reserve5_n * sizeof(float)}};
+  for (const Range& i : in)
+    for (const Range& o : out) {
+      const uintptr_t a = reinterpret_cast<uintptr_t>(i.p), b = reinterpret_cast<uintptr_t>(o.p);
+      if (i.p && o.p && a < b + o.n && b < a + i.n) return true;
+    }
+  return false;
+}
+
 bool ptr_aligned(const void* p) {
   return (reinterpret_cast<uintptr_t>(p) & 15) == 0;
 }
@@ -4316,7 +4339,7 @@ hipError_t forward_t(const BnGeometry& g, const BnFwdArgs& a, void* ws,
   if (eager &&
       make_unit_plan(g, Tr::kVec, folded_blocks_per_cu<Tr, false>(), &fp))
     return launch_fused<Tr, false>(fp, g, a.x, nullptr, a.y, fa, stream);
-  if (eager &&
+  if (eager && !channel_outputs_over_inputs(fa) &&
       make_shared_plan(g, Tr::kVec, shared_blocks_per_cu<Tr, false>(), &fp))
     return launch_fused<Tr, false>(fp, g, a.x, nullptr, a.y, fa, stream);
   if (eager && g.c % Tr::kVec != 0 &&
@@ -4377,7 +4400,7 @@ hipError_t grad_t(const BnGeometry& g, const BnGradArgs& a, void* ws,
   if (eager &&
       make_unit_plan(g, Tr::kVec, folded_blocks_per_cu<Tr, true>(), &fp))
     return launch_fused<Tr, true>(fp, g, a.x, a.dy, a.dx, fa, stream);
-  if (eager &&
+  if (eager && !channel_outputs_over_inputs(fa) &&
       make_shared_plan(g, Tr::kVec, shared_blocks_per_cu<Tr, true>(), &fp))
     return launch_fused<Tr, true>(fp, g, a.x, a.dy, a.dx, fa, stream);
   if (eager && g.c % Tr::kVec != 0 &&

@@ -916,3 +916,45 @@ def test_nchw_one_workgroup_channels_sum_in_double(dev, shape):
                                    epsilon=1e-3, data_format="NCHW")
     assert ops.fused_batch_norm_last_plan()["workgroups"] <= max(c, 256)
     assert torch.equal(got.offset_backprop, dy.double().sum((0, 2, 3)).float())
+
+
+def test_nchw_channel_outputs_over_inputs(dev):
+    """Per-channel outputs written over per-channel inputs: several workgroups
+    read a shared channel's inputs and one writes its outputs, so such calls
+    run the split kernels, in which one thread does both."""
+    shape, dtype, eps = (9, 96, 28, 28), "float16", 1e-3
+    rng = np.random.default_rng(6)
+    x, scale, offset, dy = _inputs(rng, shape, dtype, "NCHW", loc=0.5)
+    mean = (0.1 * rng.standard_normal(96)).astype(np.float32)
+    var = rng.uniform(0.5, 2.0, 96).astype(np.float32)
+    xd, dyd = to_dev(x, dtype, dev), to_dev(dy, dtype, dev)
+    f32 = lambda a: torch.from_numpy(a.copy()).to(dev)
+    new = lambda: torch.empty(96, device=dev)
+
+    # Running statistics updated in place.
+    m, v = f32(mean), f32(var)
+    fwd = ops.FusedBatchNormV3(
+        xd, f32(scale), f32(offset), m, v, epsilon=eps, exponential_avg_factor=0.75,
+        data_format="NCHW", out=ops.FusedBatchNormV3Result(
+            torch.empty_like(xd), m, v, new(), new(), torch.empty((), device=dev)))
+    assert ops.fused_batch_norm_last_plan()["fused"] == 0
+    ry, rbm, rbv, rsm, rsv = oracle.bn_fwd(x, scale, offset, mean, var, epsilon=eps,
+                                          exponential_avg_factor=0.75, data_format="NCHW",
+                                          dtype=dtype)
+    assert_close(to_np(fwd.y, dtype), ry, dtype, ACT_TOL[dtype], "y")
+    for got, ref in ((m, rbm), (v, rbv), (fwd.reserve_space_1, rsm), (fwd.reserve_space_2, rsv)):
+        assert_close(got.cpu().numpy(), ref, "float32", STAT_TOL, "statistics")
+
+    # The gradients over the saved statistics.
+    sm, sv, sc = f32(rsm), f32(rsv), f32(scale)
+    grad = ops.FusedBatchNormGradV3(
+        dyd, xd, sc, sm, sv, torch.zeros((), device=dev), epsilon=eps, data_format="NCHW",
+        out=ops.FusedBatchNormGradV3Result(torch.empty_like(xd), sm, sv, new(), new()))
+    assert ops.fused_batch_norm_last_plan()["fused"] == 0
+    rdx, rsb, rob = oracle.bn_grad(dy, x, scale, rsm, rsv, epsilon=eps, data_format="NCHW",
+                                   dtype=dtype)
+    assert_close(to_np(grad.x_backprop, dtype), rdx, dtype, ACT_TOL[dtype], "x_backprop")
+    # Both cancel (dy is independent of x): relative to the spread of such a sum.
+    for got, ref in ((sm, rsb), (sv, rob)):
+        err = np.abs(got.cpu().numpy().astype(np.float64) - ref).max()
+        assert err <= STAT_TOL * max(np.abs(ref).max(), np.sqrt(x.size // 96))
