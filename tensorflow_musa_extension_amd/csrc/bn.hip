@@ -770,6 +770,9 @@ constexpr int kFusedThreads = 512;
 // into a host-visible word; the host reports it as an error from the next
 // FusedBatchNorm call on the device (BnPendingGiveUp).
 constexpr unsigned kSpinLimit = 1u << 24;
+// The same for the folded and shared kernels, whose workgroups then work out
+// what they miss themselves.
+constexpr unsigned kMakeUpSpins = 1u << 16;
 // Epoch-tagged partials: at most 8 row groups per lane of a finishing wave.
 constexpr int kEpochPerLane = 8;
 constexpr int64_t kMaxEpochGroups = 64 * kEpochPerLane;
@@ -932,15 +935,6 @@ __device__ inline void stamp(int) {}
 __device__ inline double2 wave_sum(double a, double b) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
-    a += __shfl_xor(a, off, 64);
-    b += __shfl_xor(b, off, 64);
-  }
-  return make_double2(a, b);
-}
-// The same of float sums, added in float32.
-__device__ inline double2 wave_sum_f32(float a, float b) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) {
     a += __shfl_xor(a, off, 64);
     b += __shfl_xor(b, off, 64);
   }
@@ -1241,7 +1235,9 @@ __device__ __forceinline__ void finish_channels(const FusedArgs& a, int cs0, int
 // finish_channels.
 // kFold: the channel's elements in the tail rows are added to its sums here,
 // and written once its coefficients are known.
-template <class Tr, bool kGrad, bool kFold = false>
+// kLeave: a channel whose partials do not come is left unfinished, to the
+// workgroups that wait for its coefficients.
+template <class Tr, bool kGrad, bool kFold = false, bool kLeave = false>
 __device__ __forceinline__ void finish_channel_blocks(const FusedArgs& a, int cs0, int cs1,
                                                       int wave, int lane, uint32_t wtag,
                                                       uint64_t etag, unsigned epoch) {
@@ -1255,7 +1251,7 @@ __device__ __forceinline__ void finish_channel_blocks(const FusedArgs& a, int cs
   auto tagged = [&](uint64_t v) { return (v >> 32) == (tag >> 32); };
   for (int blk = blockIdx.x + wave * gridDim.x; blk < nb; blk += kWaves * gridDim.x) {
     const int ch = cs0 + blk * B + cl;
-    const bool chv = ch < cs1;
+    bool chv = ch < cs1;
     FinIn fin_in = fin_inputs<Tr, kGrad>(a.fin, chv ? ch : cs1 - 1, 0.f);
     uint64_t vk = !kGrad && chv ? load_shared(a.ekey + ch) : tag;
     // Slots of absent channels or past the groups are out of range: they
@@ -1279,7 +1275,8 @@ __device__ __forceinline__ void finish_channel_blocks(const FusedArgs& a, int cs
       if (ready) break;
       if (++spins > a.spin_limit) {
         lost = true;
-        __hip_atomic_store(a.gave_up, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        if constexpr (!kLeave)
+          __hip_atomic_store(a.gave_up, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         break;
       }
       __builtin_amdgcn_s_sleep(1);
@@ -1303,6 +1300,13 @@ __device__ __forceinline__ void finish_channel_blocks(const FusedArgs& a, int cs
     for (int off = 32; off >= B; off >>= 1) {
       t1 += __shfl_xor(t1, off, 64);
       t2 += __shfl_xor(t2, off, 64);
+    }
+    if constexpr (kLeave) {
+      if (__any(lost)) {
+        int n = lost;
+        for (int off = 32; off >= B; off >>= 1) n += __shfl_xor(n, off, 64);
+        chv = chv && n == 0;
+      }
     }
     float4 cfc = make_float4(0.f, 0.f, 0.f, 0.f);
     if constexpr (kFold) {
@@ -2177,7 +2181,7 @@ constexpr int kFoldParts = 32;     // most threads that share one channel's sums
 // Register rows per thread (the largest spill-free counts); ops with few rows
 // per thread run the FewRows counts.
 template <class Tr> struct FoldedRows { static constexpr int kFwd = 24, kGrad = 11; };
-template <> struct FoldedRows<TF32> { static constexpr int kFwd = 28, kGrad = 13; };
+template <> struct FoldedRows<TF32> { static constexpr int kFwd = 28, kGrad = 12; };
 template <> struct FoldedRows<TBF16> { static constexpr int kFwd = 24, kGrad = 9; };
 
 struct FoldedArgs {
@@ -2189,6 +2193,7 @@ struct FoldedArgs {
   int ry;              // super-rows of one pass
   int64_t rows;        // whole super-rows
   int64_t rows_per_g;
+  int64_t row_groups;
   FastDiv div_tw, div_ry, div_c;
   // NCHW units (kUnit): rows are images, tiles units of `fold` channels, div_c
   // divides by the plane.
@@ -2196,6 +2201,89 @@ struct FoldedArgs {
   int64_t row_bytes;   // one image
   int own;             // one row group: the workgroup finishes its channels
 };
+
+// The kernel's argument (its only one), read anew: code that hardly ever runs
+// then keeps none of its values in registers from the kernel's start.
+template <class A>
+__device__ __forceinline__ const A& arguments_again() {
+  const void* p = (const void*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *static_cast<const A*>(p);
+}
+
+// Partial i of channel ch, summed by one thread from the rows (images) that
+// its workgroup sums.
+template <class Tr, bool kGrad, bool kUnit>
+__device__ inline float2 folded_partial(const FoldedArgs& fa, int64_t i, uint32_t ch, float k) {
+  using S = typename Tr::S;
+  const FusedArgs& a = fa.f;
+  // One tile: a group's partial is of all its rows; several: of every fold-th.
+  const int64_t fold = kUnit ? 1 : fa.fold;
+  const int64_t step = kUnit || fa.tiles == 1 ? 1 : fold;
+  const int64_t g = i / step;
+  const int64_t end = (g + 1) * fa.rows_per_g < fa.rows ? (g + 1) * fa.rows_per_g : fa.rows;
+  double t1 = 0.0, t2 = 0.0;
+  auto add = [&](int64_t at) {
+    const float xc = Tr::ld(static_cast<const S*>(a.x)[at]) - k;
+    const float f = kGrad ? Tr::ld(static_cast<const S*>(a.dy)[at]) : xc;
+    t1 += f;
+    t2 += f * xc;
+  };
+  const int64_t first = g * fa.rows_per_g * fold + i % step;
+  if constexpr (kUnit) {
+    for (int64_t r = first; r < end; ++r) {
+#pragma unroll 4
+      for (int e = 0; e < static_cast<int>(fa.plane); ++e) add((r * a.c + ch) * fa.plane + e);
+    }
+  } else {
+#pragma unroll 4
+    for (int64_t r = first; r < end * fold; r += step) add(r * a.c + ch);
+  }
+  return make_float2(static_cast<float>(t1), static_cast<float>(t2));
+}
+
+// A channel whose coefficients do not come, finished by one thread of a
+// workgroup that needs them: from the partials, of which it sums those that
+// are not there itself (and publishes them; the workgroups start at different
+// ones, so they share the work).  Several workgroups may do so and write the
+// same outputs; the channel's rows past the last super-row too.
+template <class Tr, bool kGrad, bool kUnit>
+__device__ __forceinline__ float4 folded_rescue(const FoldedArgs& fa, int64_t first, uint32_t ch,
+                                             float k, uint32_t wtag, uint32_t epoch) {
+  using S = typename Tr::S;
+  const FusedArgs& a = fa.f;
+  const auto rs = slots_rsrc(a.eslots, a.groups, a.c);
+  double t1 = 0.0, t2 = 0.0;
+  for (int64_t n = 0; n < a.groups; ++n) {
+    const int64_t i = first + n < a.groups ? first + n : first + n - a.groups;
+    const u32x4 v = load_pair(rs, i * a.c + ch);
+    if (pair_tagged(v, wtag)) {
+      t1 += bits_f32(v[0]);
+      t2 += bits_f32(v[2]);
+    } else {
+      const float2 p = folded_partial<Tr, kGrad, kUnit>(fa, i, ch, k);
+      store_pair(rs, i * a.c + ch, epoch, p.x, p.y);
+      t1 += p.x;
+      t2 += p.y;
+    }
+  }
+  const int64_t at = a.tail_row * a.c + ch;
+  const S* const xt = static_cast<const S*>(a.x) + at;
+  const S* const dt = static_cast<const S*>(kGrad ? a.dy : a.x) + at;
+  const int tail = kUnit ? 0 : a.tail;
+  for (int64_t r = 0; r < tail; ++r) {
+    const float xc = Tr::ld(xt[r * a.c]) - k;
+    const float f = kGrad ? Tr::ld(dt[r * a.c]) : xc;
+    t1 += f;
+    t2 += f * xc;
+  }
+  const float4 cf = finish_channel<Tr, kGrad>(a.fin, static_cast<int>(ch), t1, t2,
+                                              fin_inputs<Tr, kGrad>(a.fin, ch, k));
+  S* const ot = static_cast<S*>(a.out) + at;
+  for (int64_t r = 0; r < tail; ++r)
+    ot[r * a.c] = apply_one<Tr, kGrad>(xt[r * a.c], dt[r * a.c], cf);
+  return cf;
+}
 
 template <class Tr, bool kGrad, int KR, int KL, bool kUnit = false>
 __global__ __launch_bounds__(kFusedThreads) void bn_folded_nhwc_kernel(FoldedArgs fa) {
@@ -2450,7 +2538,7 @@ __global__ __launch_bounds__(kFusedThreads) void bn_folded_nhwc_kernel(FoldedArg
       store_pair(slots_rsrc(a.eslots, a.groups, a.c), slot, static_cast<uint32_t>(etag >> 32),
                  static_cast<float>(sum[0]), static_cast<float>(sum[1]));
     }
-    finish_channel_blocks<Tr, kGrad, !kUnit>(a, 0, a.c, wave, lane, wtag, etag, epoch);
+    finish_channel_blocks<Tr, kGrad, !kUnit, true>(a, 0, a.c, wave, lane, wtag, etag, epoch);
   }
   zero_side_outputs<kGrad>(a.fin);
 
@@ -2462,28 +2550,19 @@ __global__ __launch_bounds__(kFusedThreads) void bn_folded_nhwc_kernel(FoldedArg
       asm volatile("" : "+v"(dr[r].x), "+v"(dr[r].y), "+v"(dr[r].z), "+v"(dr[r].w));
   }
   // The local channels' coefficients, one channel per thread, polled until
-  // tagged (as tile_coefs); coefficients that never arrive are used as NaN.
-  if (finish_own) {
-    __syncthreads();
-    if (owner) {
-      float* const c = red + tid + tid / VEC;
-      c[0] = own_cf.x;
-      c[kComp] = own_cf.y;
-      c[2 * kComp] = own_cf.z;
-      c[3 * kComp] = own_cf.w;
-    }
-    __syncthreads();
-  } else {
+  // tagged (as tile_coefs); those that do not come (the workgroups that they
+  // wait for are not running) are worked out here.
+  if (!finish_own) {
     const int64_t copy0 = (g % a.coef_copies) * a.coef_copy;
     const auto rc = rows_rsrc(a.ecoef, a.coef_copies * a.coef_copy * 8);
     const int64_t pr =
         owner ? (copy0 + 4 * static_cast<int64_t>(ch_t)) / 2 : int64_t(kOutOfRange / 16);
     u32x4 v0 = load_pair(rc, pr), v1 = load_pair(rc, pr + 1);
     unsigned spins = 0;
+    bool lost = false;
     while (owner && !(pair_tagged(v0, wtag) && pair_tagged(v1, wtag))) {
       if (++spins > a.spin_limit) {
-        v0 = v1 = u32x4{0x7fc00000u, wtag, 0x7fc00000u, wtag};
-        __hip_atomic_store(a.gave_up, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        lost = true;
         break;
       }
       __builtin_amdgcn_s_sleep(1);
@@ -2491,16 +2570,21 @@ __global__ __launch_bounds__(kFusedThreads) void bn_folded_nhwc_kernel(FoldedArg
       v0 = load_pair(rc, pr);
       v1 = load_pair(rc, pr + 1);
     }
-    __syncthreads();
-    if (owner) {
-      float* const c = red + tid + tid / VEC;
-      c[0] = bits_f32(v0[0]);
-      c[kComp] = bits_f32(v0[2]);
-      c[2 * kComp] = bits_f32(v1[0]);
-      c[3 * kComp] = bits_f32(v1[2]);
-    }
-    __syncthreads();
+    own_cf = make_float4(bits_f32(v0[0]), bits_f32(v0[2]), bits_f32(v1[0]), bits_f32(v1[2]));
+    if (__builtin_expect(lost, 0))
+      own_cf = folded_rescue<Tr, kGrad, kUnit>(
+          arguments_again<FoldedArgs>(), g + 1 < fa.row_groups ? (g + 1) * (a.groups / fa.row_groups) : 0, ch_t, k_own, wtag,
+          static_cast<uint32_t>(etag >> 32));
   }
+  __syncthreads();
+  if (owner) {
+    float* const c = red + tid + tid / VEC;
+    c[0] = own_cf.x;
+    c[kComp] = own_cf.y;
+    c[2 * kComp] = own_cf.z;
+    c[3 * kComp] = own_cf.w;
+  }
+  __syncthreads();
   float4 cf[VEC];
 #pragma unroll
   for (int j = 0; j < VEC; ++j) {
@@ -2818,6 +2902,35 @@ struct SharedNchwArgs {
   FastDiv div_pv, div_nv, div_share, div_parts, div_plane;
 };
 
+// Partial `part` of channel ch, summed by one wave element by element from the
+// vectors of the workgroup that would publish it.
+template <class Tr, bool kGrad, bool kTwo>
+__device__ __forceinline__ float2 shared_partial(const SharedNchwArgs& na, uint32_t ch,
+                                                 uint32_t part, int lane, float k) {
+  using S = typename Tr::S;
+  const uint32_t vec = Tr::kVec, plane = static_cast<uint32_t>(na.plane);
+  uint32_t lo = part * na.share, hi = lo + na.share;
+  if constexpr (kTwo) {  // counted from the workgroup of the channel's first vector
+    const uint32_t c0 = ch * na.nv, v0 = (c0 / na.share + part) * na.share;
+    lo = v0 > c0 ? v0 - c0 : 0;
+    hi = v0 + na.share - c0;
+  }
+  hi = hi < na.nv ? hi : na.nv;
+  double t1 = 0.0, t2 = 0.0;
+#pragma unroll 1
+  for (uint32_t i = lo * vec + static_cast<uint32_t>(lane); i < hi * vec; i += 64) {
+    const uint32_t img = i / (na.pv * vec), e = i - img * na.pv * vec;
+    if (e >= plane) continue;  // past a partial last vector
+    const uint32_t at = (img * static_cast<uint32_t>(na.f.c) + ch) * plane + e;
+    const float xc = Tr::ld(static_cast<const S*>(na.f.x)[at]) - k;
+    const float f = kGrad ? Tr::ld(static_cast<const S*>(na.f.dy)[at]) : xc;
+    t1 += f;
+    t2 += f * xc;
+  }
+  const double2 w = wave_sum(t1, t2);
+  return make_float2(static_cast<float>(w.x), static_cast<float>(w.y));
+}
+
 template <class Tr, bool kGrad, int KR, int KL, bool kOdd, bool kTwo>
 __global__ __launch_bounds__(kFusedThreads) void bn_nchw_shared_kernel(SharedNchwArgs na) {
   using S = typename Tr::S;
@@ -2826,8 +2939,8 @@ __global__ __launch_bounds__(kFusedThreads) void bn_nchw_shared_kernel(SharedNch
   constexpr int U = kGrad ? 4 : 8;
   constexpr int kWaves = kFusedThreads / 64;
   extern __shared__ uint4 lds_rows[];  // [KL][kIn][kFusedThreads]
-  using Sums = typename std::conditional<kTwo, float2, double2>::type;
-  __shared__ Sums red[2][kWaves];
+  __shared__ float2 red[2][kWaves];
+  __shared__ double2 red_alone[kWaves];
   __shared__ float4 cfs[2];
   const FusedArgs& a = na.f;
   const int tid = threadIdx.x;
@@ -3032,21 +3145,25 @@ __global__ __launch_bounds__(kFusedThreads) void bn_nchw_shared_kernel(SharedNch
     s1 = s2 = 0.f;
   }
   // Across threads in double where a channel has one workgroup, whose sums go
-  // to the statistics as they are; else they are published in float32.
-  if constexpr (!kTwo) {
-    const double2 w = na.parts == 1 ? wave_sum(a1s, a2s) : wave_sum_f32(a1s, a2s);
-    if (lane == 0) red[0][wave] = w;
+  // to the statistics as they are; else they are published in float32.  (The
+  // plan gives two channels to a workgroup only where each has several.)
+  const bool alone = !kTwo && na.parts == 1;
+  if (alone) {
+    const double2 w = wave_sum(a1s, a2s);
+    if (lane == 0) red_alone[wave] = w;
   } else {
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) {
       a1s += __shfl_xor(a1s, off, 64);
       a2s += __shfl_xor(a2s, off, 64);
-      s1 += __shfl_xor(s1, off, 64);
-      s2 += __shfl_xor(s2, off, 64);
+      if constexpr (kTwo) {
+        s1 += __shfl_xor(s1, off, 64);
+        s2 += __shfl_xor(s2, off, 64);
+      }
     }
     if (lane == 0) {
       red[0][wave] = make_float2(a1s, a2s);
-      red[1][wave] = make_float2(s1, s2);
+      if constexpr (kTwo) red[1][wave] = make_float2(s1, s2);
     }
   }
   __syncthreads();
@@ -3060,22 +3177,25 @@ __global__ __launch_bounds__(kFusedThreads) void bn_nchw_shared_kernel(SharedNch
         kTwo ? na.div_share.div(ch * na.nv + na.nv - 1) : w0 + na.parts - 1;
     const uint32_t cnt = w1 - w0 + 1;
     const auto rs = rows_rsrc(a.eslots, static_cast<int64_t>(a.c) * na.parts * 16);
-    typename std::conditional<kTwo, float, double>::type o1 = 0, o2 = 0;
+    if (!alone && lane == 0) {
+      float2 sum = red[wave][0];
 #pragma unroll
-    for (int i = 0; i < kWaves; ++i) {
-      o1 += red[wave][i].x;
-      o2 += red[wave][i].y;
-    }
-    // (The plan gives two channels to a workgroup only where each has several.)
-    const bool several = kTwo || cnt > 1;
-    if (several && lane == 0)
+      for (int i = 1; i < kWaves; ++i) {
+        sum.x += red[wave][i].x;
+        sum.y += red[wave][i].y;
+      }
       store_pair(rs, static_cast<int64_t>(ch) * na.parts + (b - w0),
-                 static_cast<uint32_t>(etag >> 32), static_cast<float>(o1),
-                 static_cast<float>(o2));
+                 static_cast<uint32_t>(etag >> 32), sum.x, sum.y);
+    }
     const FinIn fin_in = fin_inputs<Tr, kGrad>(a.fin, static_cast<int>(ch), wave == 0 ? ka : kb);
-    double2 w = make_double2(o1, o2);
-    if (several) {
-      double t1 = 0.0, t2 = 0.0;
+    double t1 = 0.0, t2 = 0.0;
+    if (alone) {
+#pragma unroll
+      for (int i = 0; i < kWaves; ++i) {
+        t1 += red_alone[i].x;
+        t2 += red_alone[i].y;
+      }
+    } else {
       for (uint32_t p0 = 0; p0 < cnt; p0 += 64) {
         const uint32_t p = p0 + static_cast<uint32_t>(lane);
         const bool has = p < cnt;
@@ -3083,25 +3203,40 @@ __global__ __launch_bounds__(kFusedThreads) void bn_nchw_shared_kernel(SharedNch
             has ? static_cast<int64_t>(ch) * na.parts + p : int64_t(kOutOfRange / 16);
         u32x4 v = load_pair(rs, slot);
         unsigned spins = 0;
+        bool lost = false;
         while (has && !pair_tagged(v, wtag)) {
           if (++spins > a.spin_limit) {
-            v = u32x4{0x7fc00000u, wtag, 0x7fc00000u, wtag};
-            __hip_atomic_store(a.gave_up, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            lost = true;
             break;
           }
           __builtin_amdgcn_s_sleep(1);
           asm volatile("" ::: "memory");  // the reload is not the load above
           v = load_pair(rs, slot);
         }
+        // Partials that do not come (their workgroups are not running): the
+        // wave sums those workgroups' vectors itself and publishes them.
+        for (uint64_t left = __ballot(lost); __builtin_expect(left != 0, 0); left &= left - 1) {
+          const int src = __builtin_ctzll(left);
+          const float2 m = shared_partial<Tr, kGrad, kTwo>(
+              arguments_again<SharedNchwArgs>(), ch, p0 + static_cast<uint32_t>(src), lane,
+              wave == 0 ? ka : kb);
+          if (lane == src) {
+            v = u32x4{__builtin_bit_cast(uint32_t, m.x), wtag, __builtin_bit_cast(uint32_t, m.y),
+                      wtag};
+            store_pair(rs, slot, static_cast<uint32_t>(etag >> 32), m.x, m.y);
+          }
+        }
         if (has) {
           t1 += bits_f32(v[0]);
           t2 += bits_f32(v[2]);
         }
       }
-      w = wave_sum(t1, t2);
+      const double2 w = wave_sum(t1, t2);
+      t1 = w.x;
+      t2 = w.y;
     }
     if (lane == 0)
-      cfs[wave] = finish_channel<Tr, kGrad>(a.fin, static_cast<int>(ch), w.x, w.y, fin_in,
+      cfs[wave] = finish_channel<Tr, kGrad>(a.fin, static_cast<int>(ch), t1, t2, fin_in,
                                             b == w0);
   }
   zero_side_outputs<kGrad>(a.fin);
@@ -3367,6 +3502,10 @@ struct FusedPlan {
   bool two = false;
   int unit = 0;  // NCHW units: channels of one (folded kernel, kUnit)
 };
+
+// Odd channel counts, NCHW units and shared channels, which are recorded as
+// the split kernels.
+bool eager_only(const FusedPlan& fp) { return fp.fold > 1 || fp.unit > 0 || fp.share > 0; }
 
 // Channels of the largest fused plan (at most 2 workgroups per CU, tiles of
 // at most 256 channels), and the words from one copy of the epoch-tagged
@@ -3825,10 +3964,14 @@ struct BarrierState {
   unsigned long long base = 0;
   unsigned sub_base[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // class counters (mod 2^32)
   LaunchChain chain;           // orders launches from different streams
-  unsigned long long* eslots = nullptr;  // epoch-tagged partials, zeroed at creation
+  // Epoch-tagged partials and coefficients, zeroed at creation: [0] for every
+  // kernel that may be recorded, [1] for those that run only eagerly (a replay
+  // may overlap them, and they must not touch its words).
+  unsigned long long* eslots[2] = {nullptr, nullptr};
+  unsigned long long* ecoef[2] = {nullptr, nullptr};
   size_t eslot_bytes = 0;
-  unsigned long long* ecoef = nullptr;   // epoch-tagged coefficients, zeroed at creation
   size_t ecoef_bytes = 0;
+  bool epoch_started = false;
   unsigned epoch = 0;                    // last epoch handed to a launch (< 2^31)
   // Give-up word in pinned host memory (coherent, mapped): a launch whose
   // wait ran out stores its epoch there; the host reads it without any
@@ -3911,7 +4054,8 @@ hipError_t launch_fused(const FusedPlan& fp, const BnGeometry& g, const void* x,
   // 512 * CUs), tagged with the launch's epoch, so a value from an earlier
   // launch never matches.  Eager epochs stay below 2^31; at the wrap both
   // regions are zeroed again.
-  if (!bs->eslots) {
+  const int own_values = eager_only(fp) ? 1 : 0;
+  if (!bs->eslots[own_values]) {
     const size_t slot_bytes = static_cast<size_t>(2 * DeviceCUs()) * 256 * 16;
     // kCoefCopies copies of 4 words per channel, then 1 key word per channel.
     const size_t coef_bytes =
@@ -3924,15 +4068,19 @@ hipError_t launch_fused(const FusedPlan& fp, const BnGeometry& g, const void* x,
       (void)hipFree(p);
       return e;
     }
-    bs->eslots = static_cast<unsigned long long*>(p);
+    bs->eslots[own_values] = static_cast<unsigned long long*>(p);
     bs->eslot_bytes = slot_bytes;
-    bs->ecoef = reinterpret_cast<unsigned long long*>(static_cast<char*>(p) + slot_bytes);
+    bs->ecoef[own_values] =
+        reinterpret_cast<unsigned long long*>(static_cast<char*>(p) + slot_bytes);
     bs->ecoef_bytes = coef_bytes;
+  }
+  if (!bs->epoch_started) {
     // First eager epoch - 1 (TFMA_BN_EPOCH_START, default 0): a test starts
     // just below the wrap to run launches across it.
     const char* es = getenv("TFMA_BN_EPOCH_START");
     const unsigned long long start = es ? strtoull(es, nullptr, 10) : 0ull;
     bs->epoch = start < (1ull << 31) ? static_cast<unsigned>(start) : 0u;
+    bs->epoch_started = true;
   }
   if (fp.groups > kMaxEpochGroups || fp.ct_conc < 1 ||
       static_cast<size_t>(fp.groups) * g.c * 16 > bs->eslot_bytes ||
@@ -3951,8 +4099,11 @@ hipError_t launch_fused(const FusedPlan& fp, const BnGeometry& g, const void* x,
   unsigned epoch = 0;
   if (!recorded) {
     if (bs->epoch + 1 >= (1u << 31)) {
-      hipError_t e = hipMemsetAsync(bs->eslots, 0, bs->eslot_bytes + bs->ecoef_bytes, stream);
-      if (e != hipSuccess) return e;
+      for (unsigned long long* values : bs->eslots) {
+        if (!values) continue;
+        hipError_t e = hipMemsetAsync(values, 0, bs->eslot_bytes + bs->ecoef_bytes, stream);
+        if (e != hipSuccess) return e;
+      }
       bs->epoch = 0;
     }
     epoch = ++bs->epoch;
@@ -3980,17 +4131,19 @@ hipError_t launch_fused(const FusedPlan& fp, const BnGeometry& g, const void* x,
   }
   fa.gave_up = bs->gave_up_dev;
   const bool forced = force_give_up() && !recorded;
-  fa.spin_limit = forced ? 2000u : kSpinLimit;
+  // The kernels that make up for what does not come need not wait long.
+  const bool makes_up = fp.tw > 0 || fp.share > 0;
+  fa.spin_limit = forced ? 2000u : (makes_up ? kMakeUpSpins : kSpinLimit);
   fa.wait_xor = forced ? 0x40000000u : 0u;
   fa.queues = reinterpret_cast<unsigned*>(reinterpret_cast<char*>(region) + kQueueOffset);
   fa.reset_at_exit = recorded ? 1 : 0;
-  fa.eslots = bs->eslots;
-  fa.ecoef = bs->ecoef;
+  fa.eslots = bs->eslots[own_values];
+  fa.ecoef = bs->ecoef[own_values];
   fa.coef_copy = static_cast<int64_t>(coef_copy_words());
   fa.coef_copies = static_cast<int>(std::min<int64_t>(
       kCoefCopies, std::max<int64_t>(1, fp.groups / kPollersPerCopy)));
   // The key words after the last copy of the coefficients.
-  fa.ekey = bs->ecoef + kCoefCopies * coef_copy_words();
+  fa.ekey = bs->ecoef[own_values] + kCoefCopies * coef_copy_words();
   fa.epoch = epoch;
   fa.epoch_dev = recorded ? reinterpret_cast<unsigned*>(reinterpret_cast<char*>(region) +
                                                         kEpochOffset)
@@ -4064,6 +4217,7 @@ hipError_t launch_fused(const FusedPlan& fp, const BnGeometry& g, const void* x,
     fo.ry = ry;
     fo.rows = fp.unit > 0 ? g.n : g.rows / fp.fold;
     fo.rows_per_g = fp.rows_per_g;
+    fo.row_groups = fp.row_groups;
     fo.plane = g.h * g.w;
     fo.row_bytes = g.c * g.h * g.w * static_cast<int64_t>(sizeof(typename Tr::S));
     fo.own = fp.unit > 0 && fp.groups == 1;
@@ -4268,23 +4422,28 @@ bool recording(hipStream_t stream) {
   return hipStreamIsCapturing(stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone;
 }
 
-// Whether a per-channel output lies over a per-channel input.  Such calls keep
-// the kernels in which one thread reads a channel's inputs and writes its
-// outputs: in the shared NCHW kernel the first of a channel's workgroups may
-// write them before another has read.
-bool channel_outputs_over_inputs(const FinArgs& f) {
+// Whether an output lies over an input.  Such calls keep the kernels in which
+// every element and every channel's inputs are read before they are written
+// whatever the workgroups' order: in the shared NCHW kernel the first of a
+// channel's workgroups may write the channel's outputs before another has read
+// its inputs, and where a workgroup makes up for one that is not running
+// (folded_rescue), it reads rows that others may have written.
+bool outputs_over_inputs(const FinArgs& f, const void* x, const void* dy, const void* out,
+                         size_t tensor_bytes) {
   const size_t bytes = static_cast<size_t>(f.c) * sizeof(float);
   struct Range {
     const void* p;
     size_t n;
   };
-  const Range in[] = {{f.scale, bytes}, {f.offset, bytes}, {f.mean_in, bytes}, {f.var_in, bytes}};
-  const Range out[] = {{f.batch_mean, bytes}, {f.batch_var, bytes}, {f.saved_mean, bytes},
-                       {f.saved_var, bytes}, {f.reserve3, sizeof(float)}, {f.scale_bp, bytes},
-                       {f.offset_bp, bytes}, {f.reserve4, f.reserve4_n * sizeof(float)},
-                       {f.reserve5, f.reserve5_n * sizeof(float)}};
+  const Range in[] = {{x, tensor_bytes}, {dy, tensor_bytes}, {f.scale, bytes},
+                      {f.offset, bytes}, {f.mean_in, bytes}, {f.var_in, bytes}};
+  const Range to[] = {{out, tensor_bytes}, {f.batch_mean, bytes}, {f.batch_var, bytes},
+                      {f.saved_mean, bytes}, {f.saved_var, bytes}, {f.reserve3, sizeof(float)},
+                      {f.scale_bp, bytes}, {f.offset_bp, bytes},
+                      {f.reserve4, f.reserve4_n * sizeof(float)},
+                      {f.reserve5, f.reserve5_n * sizeof(float)}};
   for (const Range& i : in)
-    for (const Range& o : out) {
+    for (const Range& o : to) {
       const uintptr_t a = reinterpret_cast<uintptr_t>(i.p), b = reinterpret_cast<uintptr_t>(o.p);
       if (i.p && o.p && a < b + o.n && b < a + i.n) return true;
     }
@@ -4327,7 +4486,9 @@ hipError_t forward_t(const BnGeometry& g, const BnFwdArgs& a, void* ws,
   FusedPlan fp;
   if (a.is_training && nchw_owned_ok(g, p.vec, sizeof(typename Tr::S)))
     return launch_nchw_owned<Tr, false>(g, a.x, nullptr, a.y, fa, stream);
-  if (a.is_training && p.vec > 1 && fused_enabled() && prefer_folded(g, p.vec) &&
+  const bool apart = !outputs_over_inputs(
+      fa, a.x, nullptr, a.y, static_cast<size_t>(g.rows) * g.c * sizeof(typename Tr::S));
+  if (a.is_training && p.vec > 1 && fused_enabled() && apart && prefer_folded(g, p.vec) &&
       make_folded_plan(g, p.vec, folded_blocks_per_cu<Tr, false>(), &fp))
     return launch_fused<Tr, false>(fp, g, a.x, nullptr, a.y, fa, stream);
   if (a.is_training && p.vec > 1 && fused_enabled() &&
@@ -4335,11 +4496,11 @@ hipError_t forward_t(const BnGeometry& g, const BnFwdArgs& a, void* ws,
     return launch_fused<Tr, false>(fp, g, a.x, nullptr, a.y, fa,
                                                   stream);
   }
-  const bool eager = a.is_training && aligned && fused_enabled() && !recording(stream);
+  const bool eager = a.is_training && aligned && fused_enabled() && apart && !recording(stream);
   if (eager &&
       make_unit_plan(g, Tr::kVec, folded_blocks_per_cu<Tr, false>(), &fp))
     return launch_fused<Tr, false>(fp, g, a.x, nullptr, a.y, fa, stream);
-  if (eager && !channel_outputs_over_inputs(fa) &&
+  if (eager &&
       make_shared_plan(g, Tr::kVec, shared_blocks_per_cu<Tr, false>(), &fp))
     return launch_fused<Tr, false>(fp, g, a.x, nullptr, a.y, fa, stream);
   if (eager && g.c % Tr::kVec != 0 &&
@@ -4388,7 +4549,9 @@ hipError_t grad_t(const BnGeometry& g, const BnGradArgs& a, void* ws,
   FusedPlan fp;
   if (nchw_owned_ok(g, p.vec, sizeof(typename Tr::S)))
     return launch_nchw_owned<Tr, true>(g, a.x, a.dy, a.dx, fa, stream);
-  if (p.vec > 1 && fused_enabled() && prefer_folded(g, p.vec) &&
+  const bool apart = !outputs_over_inputs(
+      fa, a.x, a.dy, a.dx, static_cast<size_t>(g.rows) * g.c * sizeof(typename Tr::S));
+  if (p.vec > 1 && fused_enabled() && apart && prefer_folded(g, p.vec) &&
       make_folded_plan(g, p.vec, folded_blocks_per_cu<Tr, true>(), &fp))
     return launch_fused<Tr, true>(fp, g, a.x, a.dy, a.dx, fa, stream);
   if (p.vec > 1 && fused_enabled() &&
@@ -4396,11 +4559,11 @@ hipError_t grad_t(const BnGeometry& g, const BnGradArgs& a, void* ws,
     return launch_fused<Tr, true>(fp, g, a.x, a.dy, a.dx, fa,
                                                   stream);
   }
-  const bool eager = aligned && fused_enabled() && !recording(stream);
+  const bool eager = aligned && fused_enabled() && apart && !recording(stream);
   if (eager &&
       make_unit_plan(g, Tr::kVec, folded_blocks_per_cu<Tr, true>(), &fp))
     return launch_fused<Tr, true>(fp, g, a.x, a.dy, a.dx, fa, stream);
-  if (eager && !channel_outputs_over_inputs(fa) &&
+  if (eager &&
       make_shared_plan(g, Tr::kVec, shared_blocks_per_cu<Tr, true>(), &fp))
     return launch_fused<Tr, true>(fp, g, a.x, a.dy, a.dx, fa, stream);
   if (eager && g.c % Tr::kVec != 0 &&

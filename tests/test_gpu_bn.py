@@ -958,3 +958,78 @@ def test_nchw_channel_outputs_over_inputs(dev):
     for got, ref in ((sm, rsb), (sv, rob)):
         err = np.abs(got.cpu().numpy().astype(np.float64) - ref).max()
         assert err <= STAT_TOL * max(np.abs(ref).max(), np.sqrt(x.size // 96))
+
+
+# Whole channels in one tile and in several, rows past the last super-row,
+# whole vectors; several row groups of units; shared channels of a whole number
+# of workgroups and of any number, whole and partial last vectors, more
+# channels than CUs.
+_MADE_UP_FOR = [
+    ((4, 9, 9, 63), "float16", "NHWC"),
+    ((3, 5, 7, 3), "float32", "NHWC"),
+    ((2, 17, 19, 130), "bfloat16", "NHWC"),
+    ((2, 9, 7, 513), "float16", "NHWC"),
+    ((4, 9, 9, 72), "float16", "NHWC"),
+    ((33, 512, 7, 7), "float16", "NCHW"),
+    ((7, 36, 21, 21), "float32", "NCHW"),
+    ((5, 3, 16, 24), "float16", "NCHW"),
+    ((17, 96, 28, 28), "bfloat16", "NCHW"),
+    ((4, 99, 35, 35), "float32", "NCHW"),
+    ((11, 301, 13, 15), "float16", "NCHW"),
+]
+
+_MADE_UP_FOR_SCRIPT = """
+import sys, zlib
+sys.path.insert(0, sys.argv[1])
+import numpy as np
+import torch
+from tensorflow_musa_extension_amd import raw_ops as ops
+from tests.test_gpu_bn import _MADE_UP_FOR, _inputs, _run_fwd_grad, ACT_TOL, STAT_TOL
+from tests.helpers import assert_close, gen, to_np
+from oracle import oracle
+
+dev = torch.device("cuda:0")
+for shape, dtype, fmt in _MADE_UP_FOR:
+    print(shape, dtype, flush=True)
+    rng = np.random.default_rng(zlib.crc32(repr((shape, dtype)).encode()))
+    x, scale, offset, _ = _inputs(rng, shape, dtype, fmt, loc=0.5)
+    dy = gen(rng, shape, dtype, loc=0.25)
+    fwd, grad = _run_fwd_grad(dev, x, scale, offset, dy, dtype, fmt, 1e-3)
+    assert ops.fused_batch_norm_last_plan()["fused"] == 1
+    ry, rbm, rbv, rsm, rsv = oracle.bn_fwd(x, scale, offset, epsilon=1e-3, data_format=fmt,
+                                          dtype=dtype)
+    rdx, rsb, rob = oracle.bn_grad(dy, x, scale, fwd.reserve_space_1.cpu().numpy(),
+                                   fwd.reserve_space_2.cpu().numpy(), epsilon=1e-3,
+                                   data_format=fmt, dtype=dtype)
+    assert_close(to_np(fwd.y, dtype), ry, dtype, ACT_TOL[dtype], "y")
+    assert_close(to_np(grad.x_backprop, dtype), rdx, dtype, ACT_TOL[dtype], "x_backprop")
+    for got, ref in ((fwd.batch_mean, rbm), (fwd.batch_variance, rbv),
+                     (fwd.reserve_space_1, rsm), (fwd.reserve_space_2, rsv)):
+        assert_close(got.cpu().numpy(), ref, "float32", STAT_TOL, "statistics")
+    n = x.size // scale.size
+    for got, ref in ((grad.scale_backprop, rsb), (grad.offset_backprop, rob)):
+        err = np.abs(got.cpu().numpy().astype(np.float64) - ref).max()
+        assert err <= STAT_TOL * max(np.abs(ref).max(), np.sqrt(n)), (err, n)
+assert not ops.fused_batch_norm_barrier_timed_out()
+print("made up for", flush=True)
+"""
+
+
+def test_waits_that_run_out_are_made_up_for(tmp_path):
+    """Odd channel counts, NCHW units and shared channels ran kernels without
+    cross-workgroup waits once and may overlap any other work on the device: a
+    wait that runs out (forced: every eager launch waits, briefly, for an epoch
+    that no launch publishes) leaves the outputs correct and raises no error -
+    the workgroups sum what they miss themselves.  Fresh process, since the
+    hook is read once."""
+    import os
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    script = tmp_path / "made_up_for.py"
+    script.write_text(_MADE_UP_FOR_SCRIPT)
+    env = dict(os.environ, TFMA_BN_FORCE_GIVE_UP="1")
+    r = subprocess.run([sys.executable, "-u", str(script), root], env=env, capture_output=True,
+                       text=True, timeout=100)
+    assert r.returncode == 0, r.stdout + r.stderr
+    assert "made up for" in r.stdout

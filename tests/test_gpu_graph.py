@@ -184,3 +184,56 @@ def test_grouped_adam_recorded_replays(dev, gdtype):
     for i, (v, m, w) in enumerate(zip(vars_, ms, vs)):
         for name, t, r in (("var", v, refs[i][0]), ("m", m, refs[i][1]), ("v", w, refs[i][2])):
             assert np.array_equal(t.cpu().numpy().view(np.uint32), r.view(np.uint32)), (i, name)
+
+
+@pytest.mark.parametrize("shape,fmt", [((8, 13, 13, 99), "NHWC"), ((17, 96, 28, 28), "NCHW"),
+                                       ((33, 512, 7, 7), "NCHW")])
+def test_replays_overlap_eager_odd_shapes(dev, shape, fmt):
+    """A replay of a fused batch norm on one stream and eager calls of shapes
+    that are not recorded as such (odd channels, shared channels, units) on
+    another, in no order: neither touches the other's words, and a workgroup
+    that misses what another has no room to run makes up for it."""
+    g = torch.Generator(device=dev)
+    g.manual_seed(35)
+    kw = dict(epsilon=EPS)
+    e = torch.empty(0, device=dev)
+
+    def op(shape, fmt):
+        c = shape[-1] if fmt == "NHWC" else shape[1]
+        x, dy = (torch.randn(shape, generator=g, device=dev).half() for _ in range(2))
+        scale = torch.rand(c, generator=g, device=dev) + 0.5
+        offset = torch.randn(c, generator=g, device=dev)
+
+        def step():
+            f = ops.FusedBatchNormV3(x, scale, offset, e, e, data_format=fmt, **kw)
+            return tuple(f) + tuple(ops.FusedBatchNormGradV3(
+                dy, x, scale, f.reserve_space_1, f.reserve_space_2, f.reserve_space_3,
+                data_format=fmt, **kw))
+        return step
+
+    fused, odd = op((64, 28, 28, 512), "NHWC"), op(shape, fmt)
+    want_fused = [t.clone() for t in fused()]
+    want_odd = [t.clone() for t in odd()]
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        outs = fused()
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    for _ in range(5):
+        for t in outs:
+            t.fill_(float("nan"))
+        torch.cuda.synchronize()
+        with torch.cuda.stream(streams[0]):
+            for _ in range(4):
+                graph.replay()
+        with torch.cuda.stream(streams[1]):
+            odds = [odd() for _ in range(12)]
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(outs, want_fused))
+        for got in odds:
+            for a, b in zip(got, want_odd):
+                # Partials that were made up for may differ in the last bit.
+                tol = 2 ** -10 if a.dtype == torch.float16 else 1e-6
+                assert (a.float() - b.float()).abs().max() <= tol * max(b.abs().max().item(), 1.0)
+    assert not ops.fused_batch_norm_barrier_timed_out()
