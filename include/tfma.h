@@ -407,6 +407,9 @@ int TFMA_StreamCopy(void* stream, void* dst, const void* src, uint64_t bytes,
  * stores its epoch in a host-visible word; the next FusedBatchNormV3 /
  * FusedBatchNormGradV3 call on the device then returns TFMA_INTERNAL instead
  * of launching (once per such launch; no device synchronization).
+ * That is the kernel for NHWC channel counts of whole 16-byte vectors.  Odd
+ * channel counts, and NCHW ops whose channels several workgroups share, make
+ * up for what does not come after a short spin: correct outputs, no error.
  * This query: *timed_out = 1 if any fused launch on the current device gave
  * up since the last reset; reset != 0 clears it.  Waits for the device to go
  * idle (hipDeviceSynchronize) first: a diagnostic, not for hot loops.

@@ -2174,6 +2174,9 @@ __device__ inline void recorded_exit(const FusedArgs& a, unsigned epoch) {
 //     itself and waits for none.  Forward / grad: f16 [256,2048,7,7] 57.7 /
 //     69.7 -> 28.5 / 39.4 us, bf16 [64,1024,14,14] 41.4 / 40.7 -> 21.8 / 26.0,
 //     f16 [32,512,7,7] 11.9 / 11.1 -> 7.4 / 8.1.
+//     Coefficients that do not come within kMakeUpSpins polls are worked out
+//     by the workgroup that waits for them (folded_rescue), as in the shared
+//     NCHW kernel below.
 // ---------------------------------------------------------------------------
 constexpr int kFoldChannels = 512; // most channels (one tile) or columns of a tile
 constexpr int kFoldParts = 32;     // most threads that share one channel's sums
@@ -2882,6 +2885,10 @@ __global__ __launch_bounds__(kFusedThreads) void bn_nchw_owned_kernel(NchwArgs a
 //    The grid may be larger than what is resident at once (more channels than
 //    CUs): a workgroup waits only for those of neighbouring ids, which are
 //    dispatched with it (in order, round-robin over the XCDs).
+//    A partial that does not come within kMakeUpSpins polls - other work on
+//    the device holds the CU that its workgroup needs - is summed by the wave
+//    that waits for it (shared_partial), so a launch may overlap anything;
+//    that needs inputs that no output lies over (outputs_over_inputs).
 //    kOdd: planes that are no multiple of a vector.  A plane's last vector
 //    then ends at the plane's end and overlaps the one before; its first
 //    elements are not summed and not stored.  Loads are not aligned there,
