@@ -2391,10 +2391,11 @@ __global__ __launch_bounds__(kFusedThreads) void bn_folded_nhwc_kernel(FoldedArg
     xl[q] = bld16_last(rx, roff(KR + q));
     if constexpr (kGrad) dl[q] = bld16_last(rd, roff(KR + q));
   }
-  const unsigned epoch =
-      a.epoch_dev ? 0x80000001u + __hip_atomic_load(a.epoch_dev, __ATOMIC_RELAXED,
-                                                    __HIP_MEMORY_SCOPE_AGENT) % 0x7fffffffu
-                  : a.epoch;
+  unsigned epoch = a.epoch;
+  if (!kUnit && a.epoch_dev)
+    epoch = 0x80000001u + __hip_atomic_load(a.epoch_dev, __ATOMIC_RELAXED,
+                                            __HIP_MEMORY_SCOPE_AGENT) % 0x7fffffffu;
+  asm volatile("" : "+v"(epoch));  // the scalar registers are short
   const uint64_t etag = static_cast<uint64_t>(epoch) << 32;
   const uint32_t wtag = epoch ^ a.wait_xor;
   if constexpr (!kGrad && !kUnit) {
@@ -2620,7 +2621,7 @@ __global__ __launch_bounds__(kFusedThreads) void bn_folded_nhwc_kernel(FoldedArg
 #pragma unroll
   for (int r = 0; r < KR; ++r)
     if (r < nk) st16(obase + roff(r), apply_words<Tr, kGrad>(xr[r], dr[kGrad ? r : 0], cf));
-  recorded_exit(a, epoch);
+  if constexpr (!kUnit) recorded_exit(a, epoch);
 }
 
 // ---------------------------------------------------------------------------
@@ -3072,10 +3073,9 @@ __global__ __launch_bounds__(kFusedThreads) void bn_nchw_shared_kernel(SharedNch
     xl[q] = load(true, rx, px, o);
     if constexpr (kGrad) dl[q] = load(true, rd, pd, o);
   }
-  const unsigned epoch =
-      a.epoch_dev ? 0x80000001u + __hip_atomic_load(a.epoch_dev, __ATOMIC_RELAXED,
-                                                    __HIP_MEMORY_SCOPE_AGENT) % 0x7fffffffu
-                  : a.epoch;
+  // In vector registers: the scalar ones are short (they hold the positions).
+  unsigned epoch = a.epoch;
+  asm volatile("" : "+v"(epoch));
   const uint64_t etag = static_cast<uint64_t>(epoch) << 32;
   const uint32_t wtag = epoch ^ a.wait_xor;
   // Sums of the segment in hand; at the first row of B those of A are put
@@ -3296,7 +3296,6 @@ __global__ __launch_bounds__(kFusedThreads) void bn_nchw_shared_kernel(SharedNch
     const uint4 dw = kGrad ? lds(q2, kGrad ? 1 : 0) : xw;
     apply_row(KR + q2, off, keep, xw, dw);
   }
-  recorded_exit(a, epoch);
 }
 
 // ---------------------------------------------------------------------------
@@ -3510,8 +3509,8 @@ struct FusedPlan {
   int unit = 0;  // NCHW units: channels of one (folded kernel, kUnit)
 };
 
-// Odd channel counts, NCHW units and shared channels, which are recorded as
-// the split kernels.
+// Odd channel counts, and NCHW units and channels of several workgroups, which
+// are recorded as the split kernels.
 bool eager_only(const FusedPlan& fp) { return fp.fold > 1 || fp.unit > 0 || fp.share > 0; }
 
 // Channels of the largest fused plan (at most 2 workgroups per CU, tiles of
@@ -3730,8 +3729,8 @@ bool make_unit_plan(const BnGeometry& g, int vec, int blocks_per_cu, FusedPlan* 
 // counts); ops with few rows per thread run the FewRows counts.
 template <class Tr, bool kGrad, bool kOdd>
 constexpr int shared_kr() {
-  constexpr bool half = std::is_same<Tr, TF16>::value;
-  return kGrad ? (kOdd ? 14 : (half ? 17 : 15)) : (kOdd ? 26 : (half ? 32 : 29));
+  constexpr bool half = std::is_same<Tr, TF16>::value, bf = std::is_same<Tr, TBF16>::value;
+  return kGrad ? (kOdd ? 14 : (half ? 17 : 15)) : (kOdd ? 26 : (half ? 32 : (bf ? 28 : 29)));
 }
 
 template <class Tr, bool kGrad, bool kOdd, bool kTwo>
@@ -4017,6 +4016,104 @@ BarrierState* barrier_state() {
   return &states[dev];
 }
 
+// Rows of a thread (two channels: the second's start anew).
+int64_t thread_rows(const FusedPlan& fp) {
+  const int ry = fp.tw > 0 ? kFusedThreads / fp.tw : kFusedThreads >> fp.tx_shift;
+  return (fp.rows_per_g + ry - 1) / ry + (fp.two ? 1 : 0);
+}
+
+template <class Tr>
+FoldedArgs folded_args(const FusedPlan& fp, const BnGeometry& g, const FusedArgs& fa) {
+  FoldedArgs fo;
+  fo.f = fa;
+  fo.fold = fp.unit > 0 ? fp.unit : fp.fold;
+  fo.cv = static_cast<int>(fp.cv);
+  fo.tw = fp.tw;
+  fo.tiles = fp.ct;
+  fo.ry = kFusedThreads / fp.tw;
+  fo.rows = fp.unit > 0 ? g.n : g.rows / fp.fold;
+  fo.rows_per_g = fp.rows_per_g;
+  fo.row_groups = fp.row_groups;
+  fo.plane = g.h * g.w;
+  fo.row_bytes = g.c * g.h * g.w * static_cast<int64_t>(sizeof(typename Tr::S));
+  fo.own = fp.unit > 0 && fp.groups == 1;
+  fo.div_tw = FastDiv(static_cast<uint32_t>(fp.tw));
+  fo.div_ry = FastDiv(static_cast<uint32_t>(fo.ry));
+  fo.div_c = FastDiv(static_cast<uint32_t>(fp.unit > 0 ? fo.plane : g.c));
+  return fo;
+}
+
+SharedNchwArgs shared_args(const FusedPlan& fp, const BnGeometry& g, const FusedArgs& fa) {
+  SharedNchwArgs sn;
+  sn.f = fa;
+  sn.plane = g.h * g.w;
+  sn.pv = static_cast<uint32_t>(fp.pv);
+  sn.nv = static_cast<uint32_t>(g.n * fp.pv);
+  sn.share = static_cast<uint32_t>(fp.share);
+  sn.parts = static_cast<uint32_t>(fp.groups);
+  sn.div_pv = FastDiv(sn.pv);
+  sn.div_nv = FastDiv(sn.nv);
+  sn.div_share = FastDiv(sn.share);
+  sn.div_parts = FastDiv(sn.parts);
+  sn.div_plane = FastDiv(static_cast<uint32_t>(sn.plane));
+  return sn;
+}
+
+template <class Tr, bool kGrad>
+FusedPick pick_shared(const FusedPlan& fp, const BnGeometry& g, int64_t nk) {
+  if (g.h * g.w % Tr::kVec != 0)
+    return fp.two ? pick_shared<Tr, kGrad, true, true>(nk) : pick_shared<Tr, kGrad, true, false>(nk);
+  return fp.two ? pick_shared<Tr, kGrad, false, true>(nk) : pick_shared<Tr, kGrad, false, false>(nk);
+}
+
+template <bool kGrad>
+const char* fused_name(const FusedPlan& fp) {
+  if (fp.share > 0) return kGrad ? "tfma_bn_grad_nchw_shared" : "tfma_bn_fwd_nchw_shared";
+  return kGrad ? "tfma_bn_grad_fused" : "tfma_bn_fwd_fused";
+}
+
+// NCHW ops whose channels are one workgroup's each (units of one row group,
+// shared channels of one part): no workgroup waits for another, so they are
+// launched and recorded like any other kernel - no chain, no words of the
+// library's - and several may share a CU.
+bool waits_for_none(const FusedPlan& fp) { return fp.groups == 1 && (fp.unit > 0 || fp.share > 0); }
+
+template <class Tr, bool kGrad>
+hipError_t launch_waiting_for_none(const FusedPlan& fp, const BnGeometry& g, const void* x,
+                                   const void* dy, void* out, const FinArgs& fin,
+                                   hipStream_t stream) {
+  FusedArgs fa{};
+  fa.x = x;
+  fa.dy = dy;
+  fa.out = out;
+  fa.rows = g.rows;
+  fa.c = static_cast<int>(g.c);
+  fa.groups = 1;
+  fa.fin = fin;
+  fa.fin.groups = 1;
+  const int64_t nk = thread_rows(fp);
+  const FusedPick pick =
+      fp.unit > 0 ? pick_folded<Tr, kGrad, true>(nk) : pick_shared<Tr, kGrad>(fp, g, nk);
+  t_last_plan = TFMA_FusedBatchNormPlan{};
+  t_last_plan.fused = 1;
+  t_last_plan.workgroups = fp.blocks;
+  t_last_plan.row_groups = 1;
+  t_last_plan.channel_tiles = fp.ct;
+  t_last_plan.slices = fp.slices;
+  t_last_plan.register_rows = pick.kr;
+  t_last_plan.lds_rows = pick.kl;
+  const size_t smem = static_cast<size_t>(pick.kl) * (kGrad ? 2 : 1) * kFusedThreads * 16;
+  const dim3 grid(static_cast<unsigned>(fp.blocks)), block(kFusedThreads);
+  void* const kern = const_cast<void*>(pick.kernel);
+  if (fp.unit > 0)
+    TFMA_LAUNCH(fused_name<kGrad>(fp), reinterpret_cast<void (*)(FoldedArgs)>(kern), grid,
+                block, smem, stream, folded_args<Tr>(fp, g, fa));
+  else
+    TFMA_LAUNCH(fused_name<kGrad>(fp), reinterpret_cast<void (*)(SharedNchwArgs)>(kern),
+                grid, block, smem, stream, shared_args(fp, g, fa));
+  return hipGetLastError();
+}
+
 template <class Tr, bool kGrad>
 hipError_t launch_fused(const FusedPlan& fp, const BnGeometry& g, const void* x,
                         const void* dy, void* out, const FinArgs& fin, hipStream_t stream) {
@@ -4054,6 +4151,7 @@ hipError_t launch_fused(const FusedPlan& fp, const BnGeometry& g, const void* x,
     if (e != hipSuccess) return e;
   }
   const bool recorded = cap != hipStreamCaptureStatusNone;
+  if (recorded && eager_only(fp)) return hipErrorStreamCaptureUnsupported;
   // Epoch-tagged values: partial slots for every (group, channel) and
   // coefficient words for every channel of the largest fused plan (at most
   // 2 workgroups per CU, each channel tile at most 256 channels wide and
@@ -4156,9 +4254,7 @@ hipError_t launch_fused(const FusedPlan& fp, const BnGeometry& g, const void* x,
                                                         kEpochOffset)
                           : nullptr;
   const bool folded = fp.tw > 0, shared = fp.share > 0;
-  const int ry = folded ? kFusedThreads / fp.tw : kFusedThreads >> fp.tx_shift;
-  // Rows of a thread (two channels: the second's start anew).
-  const int64_t nk_max = (fp.rows_per_g + ry - 1) / ry + (fp.two ? 1 : 0);
+  const int64_t nk_max = thread_rows(fp);
   const bool sliced = kGrad && fp.slices > 1;
   FusedPick pick = pick_fused<Tr, kGrad>(nk_max);
   if constexpr (kGrad) {
@@ -4196,8 +4292,7 @@ hipError_t launch_fused(const FusedPlan& fp, const BnGeometry& g, const void* x,
   t_last_plan.dynamic_rows = fa.dyn_rows;
   t_last_plan.dynamic_chunk = fa.dyn_chunk;
   t_last_plan.slices = fp.slices;
-  const char* name = kGrad ? "tfma_bn_grad_fused" : "tfma_bn_fwd_fused";
-  if (shared) name = kGrad ? "tfma_bn_grad_nchw_shared" : "tfma_bn_fwd_nchw_shared";
+  const char* const name = fused_name<kGrad>(fp);
   SetLastKernel(name);
   if constexpr (kGrad) {
     // No dynamic tail: the kernel that hides the slices' hand-offs.
@@ -4210,48 +4305,16 @@ hipError_t launch_fused(const FusedPlan& fp, const BnGeometry& g, const void* x,
   void* kargs[] = {&fa};
   FoldedArgs fo;
   if (folded) {
+    fo = folded_args<Tr>(fp, g, fa);
     pick = fp.unit > 0 ? pick_folded<Tr, kGrad, true>(nk_max)
                        : pick_folded<Tr, kGrad, false>(nk_max);
     smem = folded_smem<Tr, kGrad>();
-    // Workgroups that wait for none may share a CU.
-    if (fp.unit > 0 && fp.groups == 1)
-      smem = static_cast<size_t>(pick.kl) * (kGrad ? 2 : 1) * kFusedThreads * 16;
-    fo.f = fa;
-    fo.fold = fp.unit > 0 ? fp.unit : fp.fold;
-    fo.cv = static_cast<int>(fp.cv);
-    fo.tw = fp.tw;
-    fo.tiles = fp.ct;
-    fo.ry = ry;
-    fo.rows = fp.unit > 0 ? g.n : g.rows / fp.fold;
-    fo.rows_per_g = fp.rows_per_g;
-    fo.row_groups = fp.row_groups;
-    fo.plane = g.h * g.w;
-    fo.row_bytes = g.c * g.h * g.w * static_cast<int64_t>(sizeof(typename Tr::S));
-    fo.own = fp.unit > 0 && fp.groups == 1;
-    fo.div_tw = FastDiv(static_cast<uint32_t>(fp.tw));
-    fo.div_ry = FastDiv(static_cast<uint32_t>(ry));
-    fo.div_c = FastDiv(static_cast<uint32_t>(fp.unit > 0 ? fo.plane : g.c));
     kargs[0] = &fo;
   }
   SharedNchwArgs sn;
   if (shared) {
-    const int64_t plane = g.h * g.w;
-    const bool odd = plane % Tr::kVec != 0;
-    pick = fp.two ? (odd ? pick_shared<Tr, kGrad, true, true>(nk_max)
-                         : pick_shared<Tr, kGrad, false, true>(nk_max))
-                  : (odd ? pick_shared<Tr, kGrad, true, false>(nk_max)
-                         : pick_shared<Tr, kGrad, false, false>(nk_max));
-    sn.f = fa;
-    sn.plane = plane;
-    sn.pv = static_cast<uint32_t>(fp.pv);
-    sn.nv = static_cast<uint32_t>(g.n * fp.pv);
-    sn.share = static_cast<uint32_t>(fp.share);
-    sn.parts = static_cast<uint32_t>(fp.groups);
-    sn.div_pv = FastDiv(sn.pv);
-    sn.div_nv = FastDiv(sn.nv);
-    sn.div_share = FastDiv(sn.share);
-    sn.div_parts = FastDiv(sn.parts);
-    sn.div_plane = FastDiv(static_cast<uint32_t>(plane));
+    sn = shared_args(fp, g, fa);
+    pick = pick_shared<Tr, kGrad>(fp, g, nk_max);
     kargs[0] = &sn;
   }
   t_last_plan.register_rows = pick.kr;
@@ -4422,8 +4485,9 @@ hipError_t launch_nchw_owned(const BnGeometry& g, const void* x, const void* dy,
 
 // Launches recorded into a graph are not chained to other launches, so a
 // replay of a kernel whose workgroups wait for one another must not overlap
-// other such work.  The ops that run the folded super-rows, units and shared
-// channels when eager are recorded as the split kernels, whose replays may.
+// other such work.  The ops that run the folded super-rows, or units and
+// channels of several workgroups, when eager are recorded as the split kernels,
+// whose replays may.
 bool recording(hipStream_t stream) {
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   return hipStreamIsCapturing(stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone;
@@ -4503,16 +4567,16 @@ hipError_t forward_t(const BnGeometry& g, const BnFwdArgs& a, void* ws,
     return launch_fused<Tr, false>(fp, g, a.x, nullptr, a.y, fa,
                                                   stream);
   }
-  const bool eager = a.is_training && aligned && fused_enabled() && apart && !recording(stream);
-  if (eager &&
-      make_unit_plan(g, Tr::kVec, folded_blocks_per_cu<Tr, false>(), &fp))
-    return launch_fused<Tr, false>(fp, g, a.x, nullptr, a.y, fa, stream);
-  if (eager &&
-      make_shared_plan(g, Tr::kVec, shared_blocks_per_cu<Tr, false>(), &fp))
-    return launch_fused<Tr, false>(fp, g, a.x, nullptr, a.y, fa, stream);
-  if (eager && g.c % Tr::kVec != 0 &&
-      make_folded_plan(g, Tr::kVec, folded_blocks_per_cu<Tr, false>(), &fp))
-    return launch_fused<Tr, false>(fp, g, a.x, nullptr, a.y, fa, stream);
+  if (a.is_training && aligned && fused_enabled() &&
+      (make_unit_plan(g, Tr::kVec, folded_blocks_per_cu<Tr, false>(), &fp) ||
+       make_shared_plan(g, Tr::kVec, shared_blocks_per_cu<Tr, false>(), &fp) ||
+       (g.c % Tr::kVec != 0 &&
+        make_folded_plan(g, Tr::kVec, folded_blocks_per_cu<Tr, false>(), &fp)))) {
+    if (waits_for_none(fp))
+      return launch_waiting_for_none<Tr, false>(fp, g, a.x, nullptr, a.y, fa, stream);
+    if (apart && !recording(stream))
+      return launch_fused<Tr, false>(fp, g, a.x, nullptr, a.y, fa, stream);
+  }
   note_split_plan(p);
   if (!a.is_training)
     return p.vec == 1
@@ -4566,16 +4630,16 @@ hipError_t grad_t(const BnGeometry& g, const BnGradArgs& a, void* ws,
     return launch_fused<Tr, true>(fp, g, a.x, a.dy, a.dx, fa,
                                                   stream);
   }
-  const bool eager = aligned && fused_enabled() && apart && !recording(stream);
-  if (eager &&
-      make_unit_plan(g, Tr::kVec, folded_blocks_per_cu<Tr, true>(), &fp))
-    return launch_fused<Tr, true>(fp, g, a.x, a.dy, a.dx, fa, stream);
-  if (eager &&
-      make_shared_plan(g, Tr::kVec, shared_blocks_per_cu<Tr, true>(), &fp))
-    return launch_fused<Tr, true>(fp, g, a.x, a.dy, a.dx, fa, stream);
-  if (eager && g.c % Tr::kVec != 0 &&
-      make_folded_plan(g, Tr::kVec, folded_blocks_per_cu<Tr, true>(), &fp))
-    return launch_fused<Tr, true>(fp, g, a.x, a.dy, a.dx, fa, stream);
+  if (aligned && fused_enabled() &&
+      (make_unit_plan(g, Tr::kVec, folded_blocks_per_cu<Tr, true>(), &fp) ||
+       make_shared_plan(g, Tr::kVec, shared_blocks_per_cu<Tr, true>(), &fp) ||
+       (g.c % Tr::kVec != 0 &&
+        make_folded_plan(g, Tr::kVec, folded_blocks_per_cu<Tr, true>(), &fp)))) {
+    if (waits_for_none(fp))
+      return launch_waiting_for_none<Tr, true>(fp, g, a.x, a.dy, a.dx, fa, stream);
+    if (apart && !recording(stream))
+      return launch_fused<Tr, true>(fp, g, a.x, a.dy, a.dx, fa, stream);
+  }
   note_split_plan(p);
   hipError_t e =
       p.vec == 1 ? launch_reduce<Tr, 1, true>(p, g, a.x, a.dy, a.saved_mean, partial, stream)

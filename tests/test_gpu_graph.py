@@ -95,14 +95,19 @@ def test_recorded_training_step_replays(dev, tune, shape, slice_tw, slices):
     assert not ops.fused_batch_norm_barrier_timed_out()
 
 
-# (8,13,13,72): the folded kernel, recorded as it runs.  The others run kernels
-# whose workgroups wait for one another when eager and are recorded as the
-# split kernels (a replay may overlap other work).
+# (8,13,13,72): the folded kernel, recorded as it runs, and so are the kernels
+# whose workgroups wait for none: units of one row group (33 images of 7x7) and
+# shared channels of one part (9 images of 28x28).  The others run kernels whose
+# workgroups wait for one another when eager and are recorded as the split
+# kernels (a replay may overlap other work).
 @pytest.mark.parametrize("shape,fmt,same", [((8, 13, 13, 72), "NHWC", True),
                                             ((8, 13, 13, 99), "NHWC", False),
                                             ((2, 9, 7, 515), "NHWC", False),
-                                            ((9, 96, 28, 28), "NCHW", False),
-                                            ((33, 512, 7, 7), "NCHW", False)])
+                                            ((9, 96, 28, 28), "NCHW", True),
+                                            ((17, 96, 28, 28), "NCHW", False),
+                                            ((64, 512, 7, 7), "NCHW", False),
+                                            ((33, 512, 7, 7), "NCHW", True),
+                                            ((9, 230, 28, 28), "NCHW", True)])
 def test_recorded_batch_norm_replays(dev, shape, fmt, same):
     """Three replays between eager launches: bit for bit the eager results, or
     one another and within rounding of the eager results."""
@@ -187,7 +192,7 @@ def test_grouped_adam_recorded_replays(dev, gdtype):
 
 
 @pytest.mark.parametrize("shape,fmt", [((8, 13, 13, 99), "NHWC"), ((17, 96, 28, 28), "NCHW"),
-                                       ((33, 512, 7, 7), "NCHW")])
+                                       ((64, 512, 7, 7), "NCHW")])
 def test_replays_overlap_eager_odd_shapes(dev, shape, fmt):
     """A replay of a fused batch norm on one stream and eager calls of shapes
     that are not recorded as such (odd channels, shared channels, units) on
