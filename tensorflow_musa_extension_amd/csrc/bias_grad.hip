@@ -406,10 +406,26 @@ constexpr int64_t kTargetBlocksRows16 = 256;
 // Columns of the widest folded super-row: its partials (at most 2^17 words)
 // then fit the tagged slots and the allocation-free scratch.
 constexpr int64_t kMinFoldChannels = 512;
-constexpr int64_t kMinFoldBytes = int64_t(4) << 20;
 constexpr int64_t kMaxFoldColumns = int64_t(1) << 16;
 
-BagPlan make_bag_plan(int64_t outer, int64_t c, int64_t inner, int esize, bool aligned) {
+// From how many bytes folding pays: the fewer the channels, the more partials
+// a channel has and the fewer waves finalize.  Back to back, narrow loads ->
+// folded: f16 [6823,513] 7.7 -> 11.4 us, [15600,513] 12.4 -> 10.4, [2100,1021]
+// 6.8 -> 7.4, [3428,1021] 10.0 -> 8.9; f32 [11696,513], 24 MB, 11.8 -> 12.8,
+// [19493,513] 16.3 -> 14.7, [1102,1021] 4.9 -> 5.8, [1714,1021] 7.8 -> 6.8; f64
+// [1224,1021], 10 MB, 7.5 -> 9.3, [2091,777], 13 MB, 11.1 -> 7.5; int32
+// [855,2047] 7.6 -> 9.5, [1954,2047], 16 MB, 11.7 -> 7.3.
+int64_t min_fold_bytes(int64_t c, int esize, bool is_float) {
+  int64_t mib = 4;
+  if (esize == 2) mib = c < 768 ? 14 : (c < 1280 ? 6 : 4);
+  if (esize == 4 && is_float) mib = c < 768 ? 32 : (c < 896 ? 14 : (c < 1280 ? 6 : 4));
+  if (esize == 4 && !is_float) mib = c < 1024 || c >= 8192 ? 4 : 12;
+  if (esize == 8) mib = c < 4096 ? 12 : 8;
+  return mib << 20;
+}
+
+BagPlan make_bag_plan(int64_t outer, int64_t c, int64_t inner, int esize, bool is_float,
+                      bool aligned) {
   BagPlan p{};
   p.rows = inner == 1;
   p.fold = 1;
@@ -422,11 +438,12 @@ BagPlan make_bag_plan(int64_t outer, int64_t c, int64_t inner, int esize, bool a
     // f32 [8191,4095] 44.2 -> 30.0 us, f16 35.4 -> 18.1, bf16 [3000,8191] 28.0
     // -> 14.5, f32 [4001,1021] 10.2 -> 8.8.  Few channels or little data leave
     // many partials per channel to too few finalizing waves (f16 [65536,33]
-    // 10.7 -> 33.8, [256,2047] 3.8 -> 4.6): those keep the narrow loads.
+    // 10.7 -> 33.8, [256,2047] 3.8 -> 4.6): those keep the narrow loads
+    // (min_fold_bytes).
     int gcd = kv;
     while (c % gcd != 0) gcd >>= 1;
-    if (aligned && gcd < kv && c >= kMinFoldChannels && outer * c * esize >= kMinFoldBytes &&
-        c * (kv / gcd) <= kMaxFoldColumns) {
+    if (aligned && gcd < kv && c >= kMinFoldChannels && c * (kv / gcd) <= kMaxFoldColumns &&
+        outer * c * esize >= min_fold_bytes(c, esize, is_float)) {
       p.fold = kv / gcd;
       outer /= p.fold;
       c *= p.fold;
@@ -597,7 +614,7 @@ hipError_t launch_bag(const void* x, int64_t outer, int64_t c, int64_t inner, vo
   using S = typename B::S;
   using A = typename B::A;
   const bool aligned = (reinterpret_cast<uintptr_t>(x) & 15) == 0;
-  const BagPlan p = make_bag_plan(outer, c, inner, sizeof(S), aligned);
+  const BagPlan p = make_bag_plan(outer, c, inner, sizeof(S), !std::is_integral<S>::value, aligned);
   if constexpr (std::is_same<A, float>::value) {
     if (!chain_end && tag_applies<B>(p, c, stream))
       return launch_bag_tagged<B>(p, x, outer, c, inner, out, stream);
@@ -683,8 +700,9 @@ hipError_t BiasAddGradScratch(void** ptr) {
 }
 
 size_t BiasAddGradWorkspaceBytes(int dt, int64_t outer, int64_t c, int64_t inner, int esize) {
-  const BagPlan p = make_bag_plan(outer, c, inner, esize, true);
-  const BagPlan q = make_bag_plan(outer, c, inner, esize, false);
+  const bool is_float = dt != TFMA_INT32 && dt != TFMA_INT64;
+  const BagPlan p = make_bag_plan(outer, c, inner, esize, is_float, true);
+  const BagPlan q = make_bag_plan(outer, c, inner, esize, is_float, false);
   const int64_t g = std::max(p.groups * p.fold, q.groups * q.fold);
   return (static_cast<size_t>(g) * c * acc_bytes(dt) + 255) & ~size_t(255);
 }

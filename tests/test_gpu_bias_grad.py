@@ -165,10 +165,12 @@ def test_one_launch_calls_on_two_streams(dev):
 
 
 # Super-rows of 2, 4 and 8 rows, every kind of remainder, the fewest channels
-# and bytes that fold and just fewer, the most columns.
+# that fold and just fewer, the most columns; sizes that fold in every type
+# (16403x513, 3203x1021, 2047x2047, 2051x2046) and in some.
 @pytest.mark.parametrize("dtype", ["float32", "float16", "bfloat16", "float64", "int32"])
 @pytest.mark.parametrize("shape", [(4101, 513), (4099, 514), (4098, 516), (4096, 511),
-                                   (2051, 1021), (2047, 1021), (259, 8191), (130, 16387)])
+                                   (2051, 1021), (2047, 1021), (259, 8191), (130, 16387),
+                                   (16403, 513), (3203, 1021), (2047, 2047), (2051, 2046)])
 def test_folded_rows(dev, tune, dtype, shape):
     rng = np.random.default_rng(14)
     x = gen(rng, shape, dtype)
