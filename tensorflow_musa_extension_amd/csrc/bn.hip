@@ -2650,15 +2650,31 @@ struct NchwArgs {
   FinArgs fin;
 };
 
-// Rows per thread.  The grad keeps the largest spill-free count of register
-// rows (LDS rows as in the NHWC kernel).  The forward keeps fewer, so that two
+// Rows per thread: the largest spill-free counts of register rows (LDS rows as
+// in the NHWC kernel), and for the forward fewer (kFwd2), with which two
 // workgroups share a CU and one reads while the other writes: (12, 8) against
 // (30, 18), f16 [256,512,28,28] 104 -> 97 us, [256,300,28,28], whose 300
-// workgroups were two rounds, 77 -> 64, f32 [64,320,28,28] 31.4 -> 23.9; the
-// grads lose by it (f16 [256,512,28,28] 146 -> 154 us with (8, 4)).
-template <class Tr> struct OwnedRows { static constexpr int kFwd = 12, kFwdLds = 8, kGrad = 16; };
-template <> struct OwnedRows<TF16> { static constexpr int kFwd = 12, kFwdLds = 8, kGrad = 17; };
-template <> struct OwnedRows<TBF16> { static constexpr int kFwd = 11, kFwdLds = 8, kGrad = 14; };
+// workgroups were two rounds, 77 -> 64.  They read the rest again, which costs
+// more than the overlap gives with many rows, unless the rounds are far from
+// full (f16 [128,512,56,56], 98 rows, 170 -> 186, [80,768,56,56], 62 rows, 171
+// -> 180; [128,384,56,56] 148 -> 159, [96,384,56,56], 74 rows, 112 -> 108;
+// [128,300,56,56], 98 rows, 133 -> 126); in f32, whose rows are computed faster, from 49 rows (f32 [64,256,56,56] 80.4
+// -> 85.5, [256,384,28,28] 149 -> 169, [128,320,28,28], 49 rows, 60.8 -> 64.9;
+// [90,260,28,28], 35, 40.6 -> 33.6); and where planes are shorter than a cache
+// line, which workgroups of other channels read too (f32 [4096,512,4,4], 32
+// rows, 90.8 -> 104, f16 [16384,512,2,4] 411 -> 524; in planes of one vector
+// even with all rows resident, [4096,512,2,4] forward 91 -> 103, grad 121 -> 138).
+// The other grads lose by fewer rows (f16 [256,512,28,28] 146 -> 154 us with
+// (8, 4)).
+template <class Tr> struct OwnedRows {
+  static constexpr int kFwd = 30, kFwdLds = 18, kFwd2 = 12, kFwd2Lds = 8, kGrad = 16;
+};
+template <> struct OwnedRows<TF16> {
+  static constexpr int kFwd = 30, kFwdLds = 18, kFwd2 = 12, kFwd2Lds = 8, kGrad = 17;
+};
+template <> struct OwnedRows<TBF16> {
+  static constexpr int kFwd = 31, kFwdLds = 18, kFwd2 = 11, kFwd2Lds = 8, kGrad = 14;
+};
 
 template <class Tr, bool kGrad, int KR, int KL>
 __global__ __launch_bounds__(kFusedThreads) void bn_nchw_owned_kernel(NchwArgs a) {
@@ -4420,20 +4436,25 @@ struct OwnedPick {
   void (*kernel)(NchwArgs);
   int kr, kl;
 };
-// Only the last one needs more LDS than a launch gets by default.
+// nk: rows per thread; pv: vectors of a plane.  Only the last one needs more
+// LDS than a launch gets by default.
 template <class Tr, bool kGrad>
-OwnedPick pick_owned(int64_t nk) {
+OwnedPick pick_owned(int64_t nk, int64_t c, int64_t pv) {
+  // Rounds of one workgroup per CU that are at least two thirds full.
+  const int64_t cus = DeviceCUs(), slots = (c + cus - 1) / cus * cus;
+  const bool full = c * 3 >= slots * 2;
   if constexpr (kGrad) {
     constexpr FewRows f1 = kFew1Grad;
     constexpr int kr = OwnedRows<Tr>::kGrad, kl = fused_kl<Tr, true>();
-    if (nk <= f1.most) return {&bn_nchw_owned_kernel<Tr, true, f1.kr, f1.kl>, f1.kr, f1.kl};
+    const bool alone = nk > f1.most || (pv == 1 && full && nk > 4);
+    if (!alone) return {&bn_nchw_owned_kernel<Tr, true, f1.kr, f1.kl>, f1.kr, f1.kl};
     return {&bn_nchw_owned_kernel<Tr, true, kr, kl>, kr, kl};
   } else {
     constexpr FewRows f1 = kFew1Fwd, f2 = kFew2Fwd;
     constexpr int kr = OwnedRows<Tr>::kFwd, kl = OwnedRows<Tr>::kFwdLds;
     if (nk <= f1.most) return {&bn_nchw_owned_kernel<Tr, false, f1.kr, f1.kl>, f1.kr, f1.kl};
     if (nk <= f2.most / 2) return {&bn_nchw_owned_kernel<Tr, false, f2.kr, f2.kl>, f2.kr, f2.kl};
-    return {&bn_nchw_owned_kernel<Tr, false, kr, kl>, kr, kl};
+    return {&bn_nchw_owned_kernel<Tr, false, kr2, kl2>, kr2, kl2};
   }
 }
 
@@ -4446,7 +4467,8 @@ hipError_t launch_nchw_owned(const BnGeometry& g, const void* x, const void* dy,
   // [32,512,28,28] 24.3 / 24.4 -> 11.4 / 15.1, f32 [8,2048,14,14] 71.8 / 56.2
   // -> 16.5 / 17.9.
   const int64_t nv = g.n * (g.h * g.w / Tr::kVec);
-  const OwnedPick p = pick_owned<Tr, kGrad>((nv + kFusedThreads - 1) / kFusedThreads);
+  const OwnedPick p = pick_owned<Tr, kGrad>((nv + kFusedThreads - 1) / kFusedThreads, g.c,
+                                             g.h * g.w / Tr::kVec);
   const size_t smem = static_cast<size_t>(p.kl) * (kGrad ? 2 : 1) * kFusedThreads * 16;
   static std::atomic<bool> attr_set[64];
   int dev = 0;
@@ -4468,7 +4490,11 @@ hipError_t launch_nchw_owned(const BnGeometry& g, const void* x, const void* dy,
   na.plane = g.h * g.w;
   na.pv = na.plane / Tr::kVec;
   na.div_plane = FastDiv(static_cast<uint32_t>(na.plane));
+    constexpr int kr2 = OwnedRows<Tr>::kFwd2, kl2 = OwnedRows<Tr>::kFwd2Lds;
   na.div_pv = FastDiv(static_cast<uint32_t>(na.pv));
+    const bool alone = (Tr::kVec == 4 ? nk > 48 : nk > (c * 8 >= slots * 7 ? 56 : 76) && full) ||
+                       (pv < 8 && full && nk > (pv == 1 ? 4 : f1.most));
+    if (alone) return {&bn_nchw_owned_kernel<Tr, false, kr, kl>, kr, kl};
   na.fin = fin;
   t_last_plan = TFMA_FusedBatchNormPlan{};
   t_last_plan.fused = 2;
