@@ -3704,7 +3704,18 @@ bool make_folded_plan(const BnGeometry& g, int vec, int blocks_per_cu, FusedPlan
 // vector, whole units of channels, units of at most one pass of a workgroup,
 // and a tensor of fewer than 2^31 elements: every workgroup's shift samples
 // (chan_shift_nchw) are anywhere in it, whatever its own rows span.
-bool make_unit_plan(const BnGeometry& g, int vec, int blocks_per_cu, FusedPlan* fp) {
+// A unit's segment of an image is longer than a cache line, or with many units
+// most of one: shorter ones leave each line to several workgroups (against the
+// split kernels, forward / grad: f16 [1024,512,1,1] 12.0 / 13.2 -> 26.0 / 32.0
+// us, [1024,512,1,3] 15.1 / 16.1 -> 20.7 / 22.7, [1024,64,1,7], 8 units of 7
+// vectors, 10.8 / 10.5 -> 15.0 / 16.3, [1024,512,1,7], 64 units, 21.3 / 21.3 ->
+// 15.6 / 17.7, [1024,64,3,3], 9 vectors, 12.2 / 11.4 -> 10.7 / 11.8).  Small
+// 16-bit grads of several row groups are as fast in the split kernels, whose
+// launches cost less than the hand-off (f16 [64,8,14,14] 9.3 -> 11.0 us,
+// [128,64,7,7] 9.4 -> 9.7, [64,512,7,7], 3.2 MB, 12.9 -> 10.4).
+constexpr int64_t kUnitVectors = 9, kUnitVectorsMany = 5, kUnitsMany = 64;
+constexpr int64_t kUnitGradBytes = int64_t(3) << 19;
+bool make_unit_plan(const BnGeometry& g, int vec, bool grad, int blocks_per_cu, FusedPlan* fp) {
   const int64_t plane = g.h * g.w;
   const int64_t esz = 16 / vec;
   if (g.nhwc || blocks_per_cu < 1 || plane % vec == 0 || g.n < 1 ||
@@ -3741,12 +3752,14 @@ bool make_unit_plan(const BnGeometry& g, int vec, int blocks_per_cu, FusedPlan* 
   return true;
 }
 
+  if (tw < kUnitVectors && (tw < kUnitVectorsMany || units < kUnitsMany)) return false;
 // Register rows per thread of the shared NCHW kernels (the largest spill-free
 // counts); ops with few rows per thread run the FewRows counts.
 template <class Tr, bool kGrad, bool kOdd>
 constexpr int shared_kr() {
   constexpr bool half = std::is_same<Tr, TF16>::value, bf = std::is_same<Tr, TBF16>::value;
   return kGrad ? (kOdd ? 14 : (half ? 17 : 15)) : (kOdd ? 26 : (half ? 32 : (bf ? 28 : 29)));
+  if (grad && vec == 8 && groups > 1 && g.n * row_b < kUnitGradBytes) return false;
 }
 
 template <class Tr, bool kGrad, bool kOdd, bool kTwo>
@@ -4594,7 +4607,7 @@ hipError_t forward_t(const BnGeometry& g, const BnFwdArgs& a, void* ws,
                                                   stream);
   }
   if (a.is_training && aligned && fused_enabled() &&
-      (make_unit_plan(g, Tr::kVec, folded_blocks_per_cu<Tr, false>(), &fp) ||
+      (make_unit_plan(g, Tr::kVec, false, folded_blocks_per_cu<Tr, false>(), &fp) ||
        make_shared_plan(g, Tr::kVec, shared_blocks_per_cu<Tr, false>(), &fp) ||
        (g.c % Tr::kVec != 0 &&
         make_folded_plan(g, Tr::kVec, folded_blocks_per_cu<Tr, false>(), &fp)))) {
@@ -4657,7 +4670,7 @@ hipError_t grad_t(const BnGeometry& g, const BnGradArgs& a, void* ws,
                                                   stream);
   }
   if (aligned && fused_enabled() &&
-      (make_unit_plan(g, Tr::kVec, folded_blocks_per_cu<Tr, true>(), &fp) ||
+      (make_unit_plan(g, Tr::kVec, true, folded_blocks_per_cu<Tr, true>(), &fp) ||
        make_shared_plan(g, Tr::kVec, shared_blocks_per_cu<Tr, true>(), &fp) ||
        (g.c % Tr::kVec != 0 &&
         make_folded_plan(g, Tr::kVec, folded_blocks_per_cu<Tr, true>(), &fp)))) {
