@@ -2658,13 +2658,13 @@ struct NchwArgs {
 // more than the overlap gives with many rows, unless the rounds are far from
 // full (f16 [128,512,56,56], 98 rows, 170 -> 186, [80,768,56,56], 62 rows, 171
 // -> 180; [128,384,56,56] 148 -> 159, [96,384,56,56], 74 rows, 112 -> 108;
-// [128,300,56,56], 98 rows, 133 -> 126); in f32, whose rows are computed faster, from 49 rows (f32 [64,256,56,56] 80.4
-// -> 85.5, [256,384,28,28] 149 -> 169, [128,320,28,28], 49 rows, 60.8 -> 64.9;
-// [90,260,28,28], 35, 40.6 -> 33.6); and where planes are shorter than a cache
-// line, which workgroups of other channels read too (f32 [4096,512,4,4], 32
-// rows, 90.8 -> 104, f16 [16384,512,2,4] 411 -> 524; in planes of one vector
-// even with all rows resident, [4096,512,2,4] forward 91 -> 103, grad 121 -> 138).
-// The other grads lose by fewer rows (f16 [256,512,28,28] 146 -> 154 us with
+// [128,300,56,56], 98 rows, 133 -> 126); in f32, whose rows are computed
+// faster, from 49 rows (f32 [64,256,56,56] 80.4 -> 85.5, [256,384,28,28] 149 ->
+// 169, [128,320,28,28], 49 rows, 60.8 -> 64.9; [90,260,28,28], 35, 40.6 ->
+// 33.6); and where planes are shorter than a cache line, which workgroups of
+// other channels read too (f32 [4096,512,4,4], 32 rows, 90.8 -> 104, f16
+// [16384,512,2,4] 411 -> 524; in planes of one vector even with all rows
+// resident, [4096,512,2,4] forward 91 -> 103, grad 121 -> 138).  The other grads lose by fewer rows (f16 [256,512,28,28] 146 -> 154 us with
 // (8, 4)).
 template <class Tr> struct OwnedRows {
   static constexpr int kFwd = 30, kFwdLds = 18, kFwd2 = 12, kFwd2Lds = 8, kGrad = 16;
@@ -3727,12 +3727,14 @@ bool make_unit_plan(const BnGeometry& g, int vec, bool grad, int blocks_per_cu, 
   const int64_t tw = u * plane / vec;
   if (g.c % u != 0 || tw > kFusedThreads) return false;
   const int64_t units = g.c / u;
+  if (tw < kUnitVectors && (tw < kUnitVectorsMany || units < kUnitsMany)) return false;
   const int64_t ry = kFusedThreads / tw;
   const int64_t row_b = g.c * plane * esz;
   int64_t groups = std::max<int64_t>(1, static_cast<int64_t>(DeviceCUs()) / units);
   groups = std::min(groups, std::max<int64_t>(1, g.n / (2 * ry)));
   const int64_t rpg = (g.n + groups - 1) / groups;
   groups = (g.n + rpg - 1) / rpg;
+  if (grad && vec == 8 && groups > 1 && g.n * row_b < kUnitGradBytes) return false;
   if ((rpg + 64 * ry) * row_b >= (int64_t{1} << 31) || groups > kMaxEpochGroups ||
       groups * g.c > 512 * static_cast<int64_t>(DeviceCUs()) || g.c > max_fused_channels() ||
       units * groups >= (int64_t{1} << 30))
@@ -3752,14 +3754,12 @@ bool make_unit_plan(const BnGeometry& g, int vec, bool grad, int blocks_per_cu, 
   return true;
 }
 
-  if (tw < kUnitVectors && (tw < kUnitVectorsMany || units < kUnitsMany)) return false;
 // Register rows per thread of the shared NCHW kernels (the largest spill-free
 // counts); ops with few rows per thread run the FewRows counts.
 template <class Tr, bool kGrad, bool kOdd>
 constexpr int shared_kr() {
   constexpr bool half = std::is_same<Tr, TF16>::value, bf = std::is_same<Tr, TBF16>::value;
   return kGrad ? (kOdd ? 14 : (half ? 17 : 15)) : (kOdd ? 26 : (half ? 32 : (bf ? 28 : 29)));
-  if (grad && vec == 8 && groups > 1 && g.n * row_b < kUnitGradBytes) return false;
 }
 
 template <class Tr, bool kGrad, bool kOdd, bool kTwo>
@@ -4464,7 +4464,11 @@ OwnedPick pick_owned(int64_t nk, int64_t c, int64_t pv) {
     return {&bn_nchw_owned_kernel<Tr, true, kr, kl>, kr, kl};
   } else {
     constexpr FewRows f1 = kFew1Fwd, f2 = kFew2Fwd;
+    constexpr int kr2 = OwnedRows<Tr>::kFwd2, kl2 = OwnedRows<Tr>::kFwd2Lds;
     constexpr int kr = OwnedRows<Tr>::kFwd, kl = OwnedRows<Tr>::kFwdLds;
+    const bool alone = (Tr::kVec == 4 ? nk > 48 : nk > (c * 8 >= slots * 7 ? 56 : 76) && full) ||
+                       (pv < 8 && full && nk > (pv == 1 ? 4 : f1.most));
+    if (alone) return {&bn_nchw_owned_kernel<Tr, false, kr, kl>, kr, kl};
     if (nk <= f1.most) return {&bn_nchw_owned_kernel<Tr, false, f1.kr, f1.kl>, f1.kr, f1.kl};
     if (nk <= f2.most / 2) return {&bn_nchw_owned_kernel<Tr, false, f2.kr, f2.kl>, f2.kr, f2.kl};
     return {&bn_nchw_owned_kernel<Tr, false, kr2, kl2>, kr2, kl2};
@@ -4503,11 +4507,7 @@ hipError_t launch_nchw_owned(const BnGeometry& g, const void* x, const void* dy,
   na.plane = g.h * g.w;
   na.pv = na.plane / Tr::kVec;
   na.div_plane = FastDiv(static_cast<uint32_t>(na.plane));
-    constexpr int kr2 = OwnedRows<Tr>::kFwd2, kl2 = OwnedRows<Tr>::kFwd2Lds;
   na.div_pv = FastDiv(static_cast<uint32_t>(na.pv));
-    const bool alone = (Tr::kVec == 4 ? nk > 48 : nk > (c * 8 >= slots * 7 ? 56 : 76) && full) ||
-                       (pv < 8 && full && nk > (pv == 1 ? 4 : f1.most));
-    if (alone) return {&bn_nchw_owned_kernel<Tr, false, kr, kl>, kr, kl};
   na.fin = fin;
   t_last_plan = TFMA_FusedBatchNormPlan{};
   t_last_plan.fused = 2;
