@@ -3635,21 +3635,27 @@ int folded_blocks_per_cu() {
 // Whole-vector channel counts (F = 1) that the folded kernel runs faster
 // than bn_fused_nhwc_kernel, whose tiles are a power of two of at most 32
 // vectors:
-//  - rows of one tile that leave at least 5 of 16 lanes idle (forward + grad
-//    back to back: f16 [64,56,56,136] 82.2 -> 72.4 us, [64,56,56,72] 49.5 ->
-//    43.0, f32 [32,14,14,72] 22.1 -> 19.6; 13 of 16 lanes in use, f16
-//    [64,56,56,104], 59.0 -> 62.1);
+//  - rows of one tile that leave lanes idle.  Grads, from 5 of 16 idle lanes
+//    (f16 [64,56,56,72] 28.0 -> 21.7 us, [64,56,56,176] 56.9 -> 54.3,
+//    [256,56,56,160] 266 -> 208; 13 of 16 lanes in use, [64,56,56,104], lose).
+//    Forwards, from 6.5 idle (f16 [64,56,56,152] 37.0 -> 33.0, f32 [64,56,56,
+//    76] 32.7 -> 30.5); with fewer, small ones (f16 [32,14,14,160] 11.5 ->
+//    10.4; but [128,56,56,88] 37.0 -> 40.4, f32 [64,56,56,88] 32.3 -> 35.8) and
+//    rows of an odd number of vectors (f16 [64,56,56,168] 38.7 -> 35.9);
 //  - rows in several tiles whose ends fall inside cache lines, from 16 MiB,
 //    where the folded kernel streams whole rows (f16 [64,28,28,400] 68.6 ->
 //    58.3, f32 [64,56,56,264] 312 -> 262; f16 [32,14,14,400] 26.5 -> 29.6:
 //    its partials are too many for few rows; whole lines, f16 [64,28,28,384],
 //    54.7 -> 55.4).
 // A forced slice width ("bn_slice_tw") keeps the fused kernel.
-bool prefer_folded(const BnGeometry& g, int vec) {
+bool prefer_folded(const BnGeometry& g, int vec, bool grad) {
   if (!g.nhwc || g.c % vec != 0 || TuneValue(kTuneBnSliceTw) >= 0) return false;
-  const int64_t cv = g.c / vec;
-  if (cv <= 32) return cv > 8 && cv * 16 <= (int64_t(11) << pow2_ceil_log2(cv));
-  return g.c <= kFoldChannels && cv * 16 % 128 != 0 && g.rows * cv * 16 >= (int64_t(16) << 20);
+  const int64_t cv = g.c / vec, bytes = g.rows * cv * 16;
+  if (cv > 32)
+    return g.c <= kFoldChannels && cv * 16 % 128 != 0 && bytes >= (int64_t(16) << 20);
+  const int64_t lanes = int64_t(1) << pow2_ceil_log2(cv);
+  if (cv <= 8 || cv * 16 > 11 * lanes) return false;
+  return grad || cv * 32 <= 19 * lanes || bytes < (int64_t(16) << 20) || (cv > 16 && cv % 2 != 0);
 }
 
 // The folded plan of an NHWC op (aligned pointers).  Fewer than 4 super-rows
@@ -4598,7 +4604,7 @@ hipError_t forward_t(const BnGeometry& g, const BnFwdArgs& a, void* ws,
     return launch_nchw_owned<Tr, false>(g, a.x, nullptr, a.y, fa, stream);
   const bool apart = !outputs_over_inputs(
       fa, a.x, nullptr, a.y, static_cast<size_t>(g.rows) * g.c * sizeof(typename Tr::S));
-  if (a.is_training && p.vec > 1 && fused_enabled() && apart && prefer_folded(g, p.vec) &&
+  if (a.is_training && p.vec > 1 && fused_enabled() && apart && prefer_folded(g, p.vec, false) &&
       make_folded_plan(g, p.vec, folded_blocks_per_cu<Tr, false>(), &fp))
     return launch_fused<Tr, false>(fp, g, a.x, nullptr, a.y, fa, stream);
   if (a.is_training && p.vec > 1 && fused_enabled() &&
@@ -4661,7 +4667,7 @@ hipError_t grad_t(const BnGeometry& g, const BnGradArgs& a, void* ws,
     return launch_nchw_owned<Tr, true>(g, a.x, a.dy, a.dx, fa, stream);
   const bool apart = !outputs_over_inputs(
       fa, a.x, a.dy, a.dx, static_cast<size_t>(g.rows) * g.c * sizeof(typename Tr::S));
-  if (p.vec > 1 && fused_enabled() && apart && prefer_folded(g, p.vec) &&
+  if (p.vec > 1 && fused_enabled() && apart && prefer_folded(g, p.vec, true) &&
       make_folded_plan(g, p.vec, folded_blocks_per_cu<Tr, true>(), &fp))
     return launch_fused<Tr, true>(fp, g, a.x, a.dy, a.dx, fa, stream);
   if (p.vec > 1 && fused_enabled() &&
