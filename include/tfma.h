@@ -460,6 +460,9 @@ const char* TFMA_LastKernelName(void);
  *   "bn_nchw_owned"     0: NCHW training keeps the split kernels instead of
  *                       one workgroup per channel, shared channels or units
  *                       of channels.
+ *   "bn_folded"         NHWC channel counts that are no multiple of 16 bytes:
+ *                       1 one launch at any size, 0 the split kernels
+ *                       (default: by size).
  *   "bag_fused"         0: BiasAddGrad runs as two kernels (partials, then
  *                       per-channel finals) instead of one launch.
  * Each starts from the environment variable TFMA_<NAME in upper case>,

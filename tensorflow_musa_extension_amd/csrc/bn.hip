@@ -3658,6 +3658,25 @@ bool prefer_folded(const BnGeometry& g, int vec, bool grad) {
   return grad || cv * 32 <= 19 * lanes || bytes < (int64_t(16) << 20) || (cv > 16 && cv % 2 != 0);
 }
 
+// Channel counts that are no multiple of a vector: from what size one launch
+// over folded super-rows is faster than the three of the split kernels, whose
+// loads are narrow but which have no hand-off and no fold (forward / grad):
+//   f16 [32,7,7,99] 9.9 / 9.9 -> 10.1 / 10.4 us, [32,14,14,99], 1.2 MB, 11.4 /
+//   13.0 -> 10.3 / 10.8; several tiles: [8,8,8,1001] 9.7 / 9.7 -> 10.9 / 12.0,
+//   [32,8,8,1001], 4 MB, 12.8 / 15.0 -> 11.4 / 12.7; one or two channels:
+//   [64,112,112,1], 1.6 MB, 17.6 / 17.4 -> 20.8 / 21.7, [64,224,224,1] 28.6 /
+//   29.9 -> 21.7 / 22.8.  In f32 the loads are half as many: [8,7,7,99] 9.8 /
+//   9.6 -> 8.8 / 8.6, but [32,28,28,3] 9.6 / 9.5 -> 10.3 / 10.2.
+// The "bn_folded" override 1 folds at any size, 0 never.
+bool folded_pays(const BnGeometry& g, int vec) {
+  if (!g.nhwc || g.c % vec == 0) return false;
+  const int tune = TuneValue(kTuneBnFolded);
+  if (tune >= 0) return tune != 0;
+  const int64_t bytes = g.rows * g.c * (16 / vec);
+  if (vec == 4) return g.c >= 4 || bytes >= (int64_t(1) << 20);
+  return bytes >= (g.c < 3 || g.c > kFoldChannels ? int64_t(9) << 18 : int64_t(9) << 17);
+}
+
 // The folded plan of an NHWC op (aligned pointers).  Fewer than 4 super-rows
 // stay with the split kernels.
 bool make_folded_plan(const BnGeometry& g, int vec, int blocks_per_cu, FusedPlan* fp) {
@@ -4615,7 +4634,7 @@ hipError_t forward_t(const BnGeometry& g, const BnFwdArgs& a, void* ws,
   if (a.is_training && aligned && fused_enabled() &&
       (make_unit_plan(g, Tr::kVec, false, folded_blocks_per_cu<Tr, false>(), &fp) ||
        make_shared_plan(g, Tr::kVec, shared_blocks_per_cu<Tr, false>(), &fp) ||
-       (g.c % Tr::kVec != 0 &&
+       (folded_pays(g, Tr::kVec) &&
         make_folded_plan(g, Tr::kVec, folded_blocks_per_cu<Tr, false>(), &fp)))) {
     if (waits_for_none(fp))
       return launch_waiting_for_none<Tr, false>(fp, g, a.x, nullptr, a.y, fa, stream);
@@ -4678,7 +4697,7 @@ hipError_t grad_t(const BnGeometry& g, const BnGradArgs& a, void* ws,
   if (aligned && fused_enabled() &&
       (make_unit_plan(g, Tr::kVec, true, folded_blocks_per_cu<Tr, true>(), &fp) ||
        make_shared_plan(g, Tr::kVec, shared_blocks_per_cu<Tr, true>(), &fp) ||
-       (g.c % Tr::kVec != 0 &&
+       (folded_pays(g, Tr::kVec) &&
         make_folded_plan(g, Tr::kVec, folded_blocks_per_cu<Tr, true>(), &fp)))) {
     if (waits_for_none(fp))
       return launch_waiting_for_none<Tr, true>(fp, g, a.x, a.dy, a.dx, fa, stream);

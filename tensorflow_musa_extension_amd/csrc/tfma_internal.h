@@ -64,6 +64,8 @@ void TraceCommit(const TraceEvents& ev);
 //     tiles of that many channel vectors.
 //   kTuneBnSlicedOverlap: 0 = sliced grads run the plain sliced pass.
 //   kTuneBnNchwOwned: 0 = NCHW training keeps the split kernels.
+//   kTuneBnFolded: NHWC channel counts that are no multiple of a vector: 1 =
+//     folded super-rows at any size, 0 = never.
 //   kTuneBagFused: 0 = BiasAddGrad runs as two kernels (partials, then finals)
 //     instead of one launch.
 enum Tune {
@@ -71,6 +73,7 @@ enum Tune {
   kTuneBnSliceTw,
   kTuneBnSlicedOverlap,
   kTuneBnNchwOwned,
+  kTuneBnFolded,
   kTuneBagFused,
   kTuneCount
 };

@@ -782,7 +782,8 @@ def _folded_rows(shape, dtype):
 
 @pytest.mark.parametrize("is_training", [True, False])
 @pytest.mark.parametrize("shape,dtype", FOLDED_CASES)
-def test_folded_matches_oracle(dev, shape, dtype, is_training):
+def test_folded_matches_oracle(dev, tune, shape, dtype, is_training):
+    tune("bn_folded", 1)  # small ones would keep the split kernels
     rng = np.random.default_rng(zlib.crc32(repr((shape, dtype, "folded")).encode()))
     eps = 1e-3
     c = shape[-1]
@@ -989,6 +990,7 @@ from tests.helpers import assert_close, gen, to_np
 from oracle import oracle
 
 dev = torch.device("cuda:0")
+ops.set_tuning_override("bn_folded", 1)
 for shape, dtype, fmt in _MADE_UP_FOR:
     print(shape, dtype, flush=True)
     rng = np.random.default_rng(zlib.crc32(repr((shape, dtype)).encode()))

@@ -108,7 +108,7 @@ def test_recorded_training_step_replays(dev, tune, shape, slice_tw, slices):
                                             ((64, 512, 7, 7), "NCHW", False),
                                             ((33, 512, 7, 7), "NCHW", True),
                                             ((9, 230, 28, 28), "NCHW", True)])
-def test_recorded_batch_norm_replays(dev, shape, fmt, same):
+def test_recorded_batch_norm_replays(dev, tune, shape, fmt, same):
     """Three replays between eager launches: bit for bit the eager results, or
     one another and within rounding of the eager results."""
     gen_ = torch.Generator(device=dev)
@@ -120,6 +120,7 @@ def test_recorded_batch_norm_replays(dev, shape, fmt, same):
     e = torch.empty(0, device=dev)
     kw = dict(epsilon=EPS, data_format=fmt)
     plans = []
+    tune("bn_folded", 1)
 
     def step():
         f = ops.FusedBatchNormV3(x, scale, offset, e, e, **kw)
@@ -193,11 +194,12 @@ def test_grouped_adam_recorded_replays(dev, gdtype):
 
 @pytest.mark.parametrize("shape,fmt", [((8, 13, 13, 99), "NHWC"), ((17, 96, 28, 28), "NCHW"),
                                        ((64, 512, 7, 7), "NCHW")])
-def test_replays_overlap_eager_odd_shapes(dev, shape, fmt):
+def test_replays_overlap_eager_odd_shapes(dev, tune, shape, fmt):
     """A replay of a fused batch norm on one stream and eager calls of shapes
     that are not recorded as such (odd channels, shared channels, units) on
     another, in no order: neither touches the other's words, and a workgroup
     that misses what another has no room to run makes up for it."""
+    tune("bn_folded", 1)
     g = torch.Generator(device=dev)
     g.manual_seed(35)
     kw = dict(epsilon=EPS)
