@@ -33,7 +33,7 @@ def _inputs(rng, shape, dtype, data_format, loc=0.0):
 
 
 def _run_fwd_grad(dev, x, scale, offset, dy, dtype, data_format, eps, poison=True,
-                  mean=None, var=None, factor=1.0, is_training=True):
+                  mean=None, var=None, factor=1.0, is_training=True, plans=None):
     f = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)
     tx = to_dev(x, dtype, dev)
     c = scale.shape[0]
@@ -49,6 +49,8 @@ def _run_fwd_grad(dev, x, scale, offset, dy, dtype, data_format, eps, poison=Tru
     fwd = ops.FusedBatchNormV3(tx, f(scale), f(offset), tm, tv, epsilon=eps,
                                exponential_avg_factor=factor, data_format=data_format,
                                is_training=is_training, out=out)
+    if plans is not None:
+        plans.append(ops.fused_batch_norm_last_plan())
     tdy = to_dev(dy, dtype, dev)
     gout = ops.FusedBatchNormGradV3Result(
         torch.empty_like(tx), torch.empty(c, **f32), torch.empty(c, **f32),
@@ -59,6 +61,8 @@ def _run_fwd_grad(dev, x, scale, offset, dy, dtype, data_format, eps, poison=Tru
     grad = ops.FusedBatchNormGradV3(tdy, tx, f(scale), fwd.reserve_space_1,
                                     fwd.reserve_space_2, fwd.reserve_space_3, epsilon=eps,
                                     data_format=data_format, is_training=is_training, out=gout)
+    if plans is not None:
+        plans.append(ops.fused_batch_norm_last_plan())
     torch.cuda.synchronize()
     return fwd, grad
 
@@ -816,10 +820,17 @@ def test_folded_matches_oracle(dev, tune, shape, dtype, is_training):
 def test_few_rows_kernels_match_oracle(dev, rows):
     """Rows per thread (256 row groups of 64 row lanes) on both sides of every
     change of kernel: 4, 8, 14 (grad) and 32 (forward)."""
+    if torch.cuda.get_device_properties(dev).multi_processor_count != 256:
+        pytest.skip("the rows are those of 256 CUs")
+    nk = -(-rows // (256 * 64))
+    want_fwd = (3, 1) if nk <= 4 else (6, 2) if nk <= 8 else (13, 1) if nk <= 32 else (8, 18)
+    want_grad = (3, 1) if nk <= 4 else (6, 2) if nk <= 14 else (13, 9)
     rng = np.random.default_rng(rows)
     shape, dtype = (1, 1, rows, 64), "float16"
     x, scale, offset, dy = _inputs(rng, shape, dtype, "NHWC", loc=0.5)
-    fwd, grad = _run_fwd_grad(dev, x, scale, offset, dy, dtype, "NHWC", 1e-3)
+    plans = []
+    fwd, grad = _run_fwd_grad(dev, x, scale, offset, dy, dtype, "NHWC", 1e-3, plans=plans)
+    assert [(p["register_rows"], p["lds_rows"]) for p in plans] == [want_fwd, want_grad], plans
     ry, _, rbv, rsm, rsv = oracle.bn_fwd(x, scale, offset, epsilon=1e-3, dtype=dtype)
     assert_close(to_np(fwd.y, dtype), ry, dtype, ACT_TOL[dtype], "y")
     assert_close(fwd.batch_variance.cpu().numpy(), rbv, "float32", STAT_TOL, "batch_variance")
@@ -840,24 +851,28 @@ def test_few_rows_kernels_match_oracle(dev, rows):
 # channels in a workgroup), whole and partial last vectors of a plane, planes
 # of one vector, more channels than CUs; units of channels (planes that are no
 # multiple of a vector), with one row group and several; channels that are no
-# whole unit; all rows on chip and streamed ones.
+# whole unit; few rows per thread (test_many_rows_kernels has many).
 NCHW_CASES = [
     ((5, 3, 4, 8), "float16"),
     ((3, 1, 8, 8), "float32"),
     ((64, 64, 28, 28), "float16"),
     ((17, 96, 28, 28), "bfloat16"),    # 2.67 workgroups per channel
-    ((9, 200, 8, 9), "float32"),
+    ((9, 200, 8, 9), "float32"),        # one part per channel
+    ((60, 200, 8, 9), "float32"),       # two channels in a workgroup
     ((16, 100, 5, 5), "float16"),      # 25 elements, no whole unit of 8
     ((4, 99, 35, 35), "float32"),
-    ((3, 301, 13, 15), "bfloat16"),    # more channels than CUs, odd planes
-    ((16, 64, 112, 112), "float16"),   # streamed rows
-    ((8, 48, 99, 99), "bfloat16"),     # the same, odd planes
+    ((3, 301, 13, 15), "bfloat16"),    # more channels than CUs, odd planes, one part
+    ((60, 301, 13, 15), "bfloat16"),   # the same, two channels in a workgroup
+    ((40, 301, 35, 35), "float32"),
+    ((16, 64, 112, 112), "float16"),   # 13 rows: the grad streams
+    ((8, 48, 99, 99), "bfloat16"),     # odd planes, all rows on chip
     ((2, 8, 7, 7), "float16"),         # one unit
-    ((33, 512, 7, 7), "float16"),
-    ((40, 2048, 7, 7), "bfloat16"),    # one row group
+    ((33, 512, 7, 7), "float16"),      # one row group
+    ((64, 512, 7, 7), "float16"),      # three
+    ((40, 2048, 7, 7), "bfloat16"),
     ((64, 256, 14, 14), "float16"),
     ((7, 36, 21, 21), "float32"),
-    ((256, 64, 21, 21), "float16"),    # 441 vectors of 512: streamed rows
+    ((256, 64, 21, 21), "float16"),    # 441 vectors of 512, 8 rows
     ((6, 512, 14, 14), "float32"),     # a workgroup per channel, few rows
     ((40, 256, 28, 28), "float16"),
     ((90, 260, 28, 28), "bfloat16"),
@@ -1036,3 +1051,74 @@ def test_waits_that_run_out_are_made_up_for(tmp_path):
                        text=True, timeout=100)
     assert r.returncode == 0, r.stdout + r.stderr
     assert "made up for" in r.stdout
+
+
+# Many rows per thread: every large kernel, with rows in registers, in LDS and
+# streamed.  Units with one row group and two; shared channels, whole and odd
+# planes, a whole number of workgroups per channel and any (a workgroup's second
+# channel then starts anywhere in its rows); folded super-rows in one tile and
+# in several.  (shape, type, layout, kernel, (register, LDS) rows of the forward
+# and of the grad.)
+MANY_ROWS = [
+    ((20, 1032, 21, 21), "float16", "NCHW", "fused", (13, 1), (11, 8)),
+    ((48, 1032, 21, 21), "float16", "NCHW", "fused", (24, 16), (11, 8)),
+    ((48, 1032, 21, 21), "bfloat16", "NCHW", "fused", (24, 16), (9, 8)),
+    ((50, 516, 21, 21), "float32", "NCHW", "fused", (28, 16), (12, 8)),
+    ((96, 1024, 21, 21), "float16", "NCHW", "fused", (24, 16), (11, 8)),
+    ((300, 64, 56, 56), "float16", "NCHW", "nchw_shared", (32, 18), (17, 9)),
+    ((300, 64, 56, 56), "bfloat16", "NCHW", "nchw_shared", (28, 18), (15, 9)),
+    ((140, 64, 56, 56), "float32", "NCHW", "nchw_shared", (29, 18), (15, 9)),
+    ((200, 96, 56, 56), "float16", "NCHW", "nchw_shared", (32, 18), (17, 9)),
+    ((100, 96, 56, 56), "float32", "NCHW", "nchw_shared", (29, 18), (15, 9)),
+    ((60, 64, 111, 111), "float16", "NCHW", "nchw_shared", (26, 18), (14, 9)),
+    ((60, 96, 99, 99), "bfloat16", "NCHW", "nchw_shared", (26, 18), (14, 9)),
+    ((30, 96, 99, 99), "float32", "NCHW", "nchw_shared", (26, 18), (14, 9)),
+    ((150, 56, 56, 99), "float16", "NHWC", "fused", (24, 16), (11, 8)),
+    ((150, 56, 56, 99), "bfloat16", "NHWC", "fused", (24, 16), (9, 8)),
+    ((80, 56, 56, 99), "float32", "NHWC", "fused", (28, 16), (12, 8)),
+    ((60, 28, 28, 1021), "float16", "NHWC", "fused", (24, 16), (11, 8)),
+    ((33, 28, 28, 1021), "float32", "NHWC", "fused", (28, 16), (12, 8)),
+]
+
+
+@pytest.mark.parametrize("shape,dtype,fmt,kernel,fwd_rows,grad_rows", MANY_ROWS)
+def test_many_rows_kernels(dev, shape, dtype, fmt, kernel, fwd_rows, grad_rows):
+    if torch.cuda.get_device_properties(dev).multi_processor_count != 256:
+        pytest.skip("the rows are those of 256 CUs")
+    dt, eps = getattr(torch, dtype), 1e-3
+    dims = [0, 2, 3] if fmt == "NCHW" else [0, 1, 2]
+    c = shape[1] if fmt == "NCHW" else shape[3]
+    per = (lambda v: v.view(1, c, 1, 1)) if fmt == "NCHW" else (lambda v: v)
+    g = torch.Generator(device=dev)
+    g.manual_seed(c)
+    scale = torch.rand(c, generator=g, device=dev) + 0.5
+    offset = torch.randn(c, generator=g, device=dev)
+    x = (torch.randn(shape, generator=g, device=dev) + per(offset)).to(dt)
+    dy = (torch.randn(shape, generator=g, device=dev) + 0.25).to(dt)
+    e = torch.empty(0, device=dev)
+
+    def plan(name, rows):
+        p = ops.fused_batch_norm_last_plan()
+        assert ops.last_kernel_name() == f"tfma_bn_{name}_{kernel}"
+        assert (p["register_rows"], p["lds_rows"]) == rows, p
+
+    f = ops.FusedBatchNormV3(x, scale, offset, e, e, epsilon=eps, data_format=fmt)
+    plan("fwd", fwd_rows)
+    b = ops.FusedBatchNormGradV3(dy, x, scale, f.reserve_space_1, f.reserve_space_2,
+                                 f.reserve_space_3, epsilon=eps, data_format=fmt)
+    plan("grad", grad_rows)
+    xd, dyd, n = x.double(), dy.double(), x.numel() // c
+    mean = xd.mean(dims)
+    var = (xd - per(mean)).square_().mean(dims)
+    close = lambda got, want, tol: ((got.double() - want).abs().max()
+                                    <= tol * want.abs().max()).item()
+    assert close(f.reserve_space_1, mean, STAT_TOL) and close(f.reserve_space_2, var, STAT_TOL)
+    mu, k = f.reserve_space_1.double(), (f.reserve_space_2.double() + eps).rsqrt()
+    xc = xd.sub_(per(mu))
+    assert close(f.y, xc * per(k * scale) + per(offset.double()), ACT_TOL[dtype])
+    s1, s2 = dyd.sum(dims), (dyd * xc).sum(dims)
+    # Both sums: relative to the spread of n terms where they cancel.
+    for got, want in ((b.offset_backprop, s1), (b.scale_backprop, s2 * k)):
+        assert (got.double() - want).abs().max() <= STAT_TOL * max(want.abs().max(), n ** 0.5)
+    want = (dyd.sub_(per(s1 / n)) - xc * per(k * k * s2 / n)) * per(k * scale)
+    assert close(b.x_backprop, want, ACT_TOL[dtype])
