@@ -24,8 +24,8 @@ cpu_baseline: the TF-CPU restatement (oracle/, C + OpenMP; TensorFlow is
         repeated for >= 10 s on the box's CPU share (at most 16 threads;
         lscpu model and os.cpu_count() reported), and under "components" the
         same for Adam cfg3, a stated sample of cfg5 and the cfg4 chains.
-components: cfg1 (FusedBatchNormV3 forward, f32 [32,56,56,64]), BN on the
-        split path (NCHW training fwd and grad, NHWC inference), and the
+components: cfg1 (FusedBatchNormV3 forward, f32 [32,56,56,64]), BN in
+        NCHW (training fwd and grad) and inference, and the
         other kernels (Adam, mixed-precision Adam, grouped Adam at
         the ResNet-50 and 1.31e9-parameter configs, the elementwise chains,
         ReluGrad, BiasAddGrad) at their config shapes, each of 20 reps timed

@@ -474,7 +474,8 @@ const char* TFMA_LastKernelName(void);
  * in normal use): TFMA_BN_FORCE_GIVE_UP=1 makes every eager fused BatchNorm
  * launch give up its grid-wide waits after a short spin (exercises the
  * co-residency error path: NaN outputs, then INTERNAL, see
- * TFMA_FusedBatchNormBarrierTimedOut); TFMA_BN_EPOCH_START=<n> starts the
+ * TFMA_FusedBatchNormBarrierTimedOut; odd shapes work out what they miss);
+ * TFMA_BN_EPOCH_START=<n> starts the
  * fused launches' epoch counter at n (runs launches across its wrap);
  * TFMA_BN_FUSED=0 disables the fused BatchNorm kernels; TFMA_BN_DYN_PCT,
  * TFMA_BN_DYN_CHUNK, TFMA_BN_TARGET_WGS and TFMA_EW_BLOCKS_PER_CU change

@@ -844,7 +844,9 @@ constexpr int fused_kl() { return kGrad ? Resident<Tr>::kLdsGrad : Resident<Tr>:
 //   f32 [32,56,56,64] (13)        15.1 / 19.0 -> 14.0 / 18.2 us
 //   f16 [64,28,28,384] (19)       23.8 -> 21.7 us (forward, (13, 1))
 //   f16 [64,56,56,128] (25)       27.6 -> 24.6 us (forward, (13, 1))
-// The rows such a forward streams come back from the caches; at 49 rows
+// The rows such a forward streams come back from the caches (also over buffers
+// larger than those: [256,7,7,2048], 25 rows, 26.9 -> 25.5 us; but 26.5 -> 28.2
+// behind another op, whose write-backs compete); at 49 rows
 // (f16 [256,14,14,1024]) (13, 1) takes 45.0 us and the (8, 18) kernel 43.9,
 // and the grads past 14 rows gain nothing ([256,7,7,2048] bf16 32.6 us with
 // all resident rows, 33.2 with (12, 2)).
@@ -4459,8 +4461,8 @@ size_t partial_region_bytes(DType t, const BnGeometry& g) {
 }
 
 // The channel-per-workgroup NCHW kernel: training, 16-byte plane vectors, at
-// least one channel per CU (fewer channels leave CUs idle: the split path's
-// reduce spreads every channel over many workgroups), and offsets that fit
+// least one channel per CU (fewer channels would leave CUs idle: they are
+// shared between workgroups, make_shared_plan), and offsets that fit
 // the kernel's 32-bit buffer offsets (rows up to 16 images past the tensor's
 // end).  The "bn_nchw_owned" override 0 keeps the split path.
 bool nchw_owned_ok(const BnGeometry& g, int vec, int elem) {
@@ -4621,9 +4623,11 @@ hipError_t forward_t(const BnGeometry& g, const BnFwdArgs& a, void* ws,
   FusedPlan fp;
   if (a.is_training && nchw_owned_ok(g, p.vec, sizeof(typename Tr::S)))
     return launch_nchw_owned<Tr, false>(g, a.x, nullptr, a.y, fa, stream);
-  const bool apart = !outputs_over_inputs(
-      fa, a.x, nullptr, a.y, static_cast<size_t>(g.rows) * g.c * sizeof(typename Tr::S));
-  if (a.is_training && p.vec > 1 && fused_enabled() && apart && prefer_folded(g, p.vec, false) &&
+  const auto apart = [&] {
+    return !outputs_over_inputs(fa, a.x, nullptr, a.y,
+                                static_cast<size_t>(g.rows) * g.c * sizeof(typename Tr::S));
+  };
+  if (a.is_training && p.vec > 1 && fused_enabled() && prefer_folded(g, p.vec, false) && apart() &&
       make_folded_plan(g, p.vec, folded_blocks_per_cu<Tr, false>(), &fp))
     return launch_fused<Tr, false>(fp, g, a.x, nullptr, a.y, fa, stream);
   if (a.is_training && p.vec > 1 && fused_enabled() &&
@@ -4638,7 +4642,7 @@ hipError_t forward_t(const BnGeometry& g, const BnFwdArgs& a, void* ws,
         make_folded_plan(g, Tr::kVec, folded_blocks_per_cu<Tr, false>(), &fp)))) {
     if (waits_for_none(fp))
       return launch_waiting_for_none<Tr, false>(fp, g, a.x, nullptr, a.y, fa, stream);
-    if (apart && !recording(stream))
+    if (apart() && !recording(stream))
       return launch_fused<Tr, false>(fp, g, a.x, nullptr, a.y, fa, stream);
   }
   note_split_plan(p);
@@ -4684,9 +4688,11 @@ hipError_t grad_t(const BnGeometry& g, const BnGradArgs& a, void* ws,
   FusedPlan fp;
   if (nchw_owned_ok(g, p.vec, sizeof(typename Tr::S)))
     return launch_nchw_owned<Tr, true>(g, a.x, a.dy, a.dx, fa, stream);
-  const bool apart = !outputs_over_inputs(
-      fa, a.x, a.dy, a.dx, static_cast<size_t>(g.rows) * g.c * sizeof(typename Tr::S));
-  if (p.vec > 1 && fused_enabled() && apart && prefer_folded(g, p.vec, true) &&
+  const auto apart = [&] {
+    return !outputs_over_inputs(fa, a.x, a.dy, a.dx,
+                                static_cast<size_t>(g.rows) * g.c * sizeof(typename Tr::S));
+  };
+  if (p.vec > 1 && fused_enabled() && prefer_folded(g, p.vec, true) && apart() &&
       make_folded_plan(g, p.vec, folded_blocks_per_cu<Tr, true>(), &fp))
     return launch_fused<Tr, true>(fp, g, a.x, a.dy, a.dx, fa, stream);
   if (p.vec > 1 && fused_enabled() &&
@@ -4701,7 +4707,7 @@ hipError_t grad_t(const BnGeometry& g, const BnGradArgs& a, void* ws,
         make_folded_plan(g, Tr::kVec, folded_blocks_per_cu<Tr, true>(), &fp)))) {
     if (waits_for_none(fp))
       return launch_waiting_for_none<Tr, true>(fp, g, a.x, a.dy, a.dx, fa, stream);
-    if (apart && !recording(stream))
+    if (apart() && !recording(stream))
       return launch_fused<Tr, true>(fp, g, a.x, a.dy, a.dx, fa, stream);
   }
   note_split_plan(p);
