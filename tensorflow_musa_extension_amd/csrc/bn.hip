@@ -844,9 +844,9 @@ constexpr int fused_kl() { return kGrad ? Resident<Tr>::kLdsGrad : Resident<Tr>:
 //   f32 [32,56,56,64] (13)        15.1 / 19.0 -> 14.0 / 18.2 us
 //   f16 [64,28,28,384] (19)       23.8 -> 21.7 us (forward, (13, 1))
 //   f16 [64,56,56,128] (25)       27.6 -> 24.6 us (forward, (13, 1))
-// The rows such a forward streams come back from the caches (also over buffers
-// larger than those: [256,7,7,2048], 25 rows, 26.9 -> 25.5 us; but 26.5 -> 28.2
-// behind another op, whose write-backs compete); at 49 rows
+// The rows such a forward streams come back from the L2 (also over buffers
+// that no cache holds: [256,7,7,2048], 25 rows, 26.9 -> 25.5 us; between other
+// batch norms, though, 26.5 -> 28.2 with the same traffic); at 49 rows
 // (f16 [256,14,14,1024]) (13, 1) takes 45.0 us and the (8, 18) kernel 43.9,
 // and the grads past 14 rows gain nothing ([256,7,7,2048] bf16 32.6 us with
 // all resident rows, 33.2 with (12, 2)).
