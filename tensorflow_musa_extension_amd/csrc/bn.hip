@@ -2579,7 +2579,8 @@ __global__ __launch_bounds__(kFusedThreads) void bn_folded_nhwc_kernel(FoldedArg
     own_cf = make_float4(bits_f32(v0[0]), bits_f32(v0[2]), bits_f32(v1[0]), bits_f32(v1[2]));
     if (__builtin_expect(lost, 0))
       own_cf = folded_rescue<Tr, kGrad, kUnit>(
-          arguments_again<FoldedArgs>(), g + 1 < fa.row_groups ? (g + 1) * (a.groups / fa.row_groups) : 0, ch_t, k_own, wtag,
+          arguments_again<FoldedArgs>(),
+          g + 1 < fa.row_groups ? (g + 1) * (a.groups / fa.row_groups) : 0, ch_t, k_own, wtag,
           static_cast<uint32_t>(etag >> 32));
   }
   __syncthreads();
@@ -2666,8 +2667,8 @@ struct NchwArgs {
 // 33.6); and where planes are shorter than a cache line, which workgroups of
 // other channels read too (f32 [4096,512,4,4], 32 rows, 90.8 -> 104, f16
 // [16384,512,2,4] 411 -> 524; in planes of one vector even with all rows
-// resident, [4096,512,2,4] forward 91 -> 103, grad 121 -> 138).  The other grads lose by fewer rows (f16 [256,512,28,28] 146 -> 154 us with
-// (8, 4)).
+// resident, [4096,512,2,4] forward 91 -> 103, grad 121 -> 138).  The other
+// grads lose by fewer rows (f16 [256,512,28,28] 146 -> 154 us with (8, 4)).
 template <class Tr> struct OwnedRows {
   static constexpr int kFwd = 30, kFwdLds = 18, kFwd2 = 12, kFwd2Lds = 8, kGrad = 16;
 };
@@ -4118,8 +4119,10 @@ SharedNchwArgs shared_args(const FusedPlan& fp, const BnGeometry& g, const Fused
 template <class Tr, bool kGrad>
 FusedPick pick_shared(const FusedPlan& fp, const BnGeometry& g, int64_t nk) {
   if (g.h * g.w % Tr::kVec != 0)
-    return fp.two ? pick_shared<Tr, kGrad, true, true>(nk) : pick_shared<Tr, kGrad, true, false>(nk);
-  return fp.two ? pick_shared<Tr, kGrad, false, true>(nk) : pick_shared<Tr, kGrad, false, false>(nk);
+    return fp.two ? pick_shared<Tr, kGrad, true, true>(nk)
+                  : pick_shared<Tr, kGrad, true, false>(nk);
+  return fp.two ? pick_shared<Tr, kGrad, false, true>(nk)
+                : pick_shared<Tr, kGrad, false, false>(nk);
 }
 
 template <bool kGrad>
@@ -4568,12 +4571,13 @@ bool recording(hipStream_t stream) {
 bool outputs_over_inputs(const FinArgs& f, const void* x, const void* dy, const void* out,
                          size_t tensor_bytes) {
   const size_t bytes = static_cast<size_t>(f.c) * sizeof(float);
+  const size_t stats = f.f != 1.0f ? bytes : 0;  // else not read (f is 0 for the grad)
   struct Range {
     const void* p;
     size_t n;
   };
   const Range in[] = {{x, tensor_bytes}, {dy, tensor_bytes}, {f.scale, bytes},
-                      {f.offset, bytes}, {f.mean_in, bytes}, {f.var_in, bytes}};
+                      {f.offset, bytes}, {f.mean_in, stats}, {f.var_in, stats}};
   const Range to[] = {{out, tensor_bytes}, {f.batch_mean, bytes}, {f.batch_var, bytes},
                       {f.saved_mean, bytes}, {f.saved_var, bytes}, {f.reserve3, sizeof(float)},
                       {f.scale_bp, bytes}, {f.offset_bp, bytes},
@@ -4582,7 +4586,7 @@ bool outputs_over_inputs(const FinArgs& f, const void* x, const void* dy, const 
   for (const Range& i : in)
     for (const Range& o : to) {
       const uintptr_t a = reinterpret_cast<uintptr_t>(i.p), b = reinterpret_cast<uintptr_t>(o.p);
-      if (i.p && o.p && a < b + o.n && b < a + i.n) return true;
+      if (i.p && o.p && i.n > 0 && a < b + o.n && b < a + i.n) return true;
     }
   return false;
 }
